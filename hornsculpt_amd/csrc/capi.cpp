@@ -1505,15 +1505,15 @@ int hsbem_dense_lu_solve(hsbem_context *c, uint32_t n, const double *A, uint32_t
         hsbem::DeviceBuffer<double> dA(2 * nn), dB(2 * static_cast<std::size_t>(n) * nrhs);
         hsbem::DeviceBuffer<std::int32_t> piv(n);
         hsbem::DeviceBuffer<int> info(1);
+        hsbem::DeviceBuffer<double> work(hsbem::dev::kLuWorkDoubles);
         hsbem::hip_check(hipMemcpyAsync(dA.data(), A, dA.bytes(), hipMemcpyHostToDevice, s), "A upload");
         hsbem::hip_check(hipMemcpyAsync(dB.data(), B, dB.bytes(), hipMemcpyHostToDevice, s), "B upload");
         hsbem::hip_check(hipMemsetAsync(info.data(), 0, sizeof(int), s), "info clear");
-        hsbem::dev::lu_factor(dA.data(), n, piv.data(), info.data(), nullptr, s);
+        hsbem::dev::lu_factor(dA.data(), n, piv.data(), info.data(), work.data(), s);
         int code = 0;
         hsbem::hip_check(hipMemcpyAsync(&code, info.data(), sizeof(int), hipMemcpyDeviceToHost, s), "info download");
         hsbem::hip_check(hipStreamSynchronize(s), "LU sync");
-        if (code)
-            throw std::runtime_error("LU factorization failed at pivot " + std::to_string(code));
+        hsbem::dev::check_lu_status(code, "LU factorization failed at pivot ");
         hsbem::dev::lu_solve(dA.data(), n, piv.data(), dB.data(), nrhs, s);
         hsbem::hip_check(hipMemcpyAsync(B, dB.data(), dB.bytes(), hipMemcpyDeviceToHost, s), "B download");
         hsbem::hip_check(hipStreamSynchronize(s), "LU solve sync");

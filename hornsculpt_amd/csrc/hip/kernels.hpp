@@ -180,9 +180,13 @@ void launch_norm2(const double *x, std::uint32_t n, const double *weight, double
                   hipStream_t stream);
 std::size_t reduction_scratch_doubles(std::uint32_t n, std::uint32_t m);
 
-// Complex LU with partial pivoting in place (A n x n), pivots n.
+// Complex LU with partial pivoting in place (A n x n), pivots n. info (cleared by the caller):
+// the first zero pivot's column + 1, or negative when the panel's workgroups gave up waiting
+// for each other (see check_lu_status). work: kLuWorkDoubles doubles of this call's own.
+inline constexpr std::size_t kLuWorkDoubles = 4 * 120 * 132 + 64;
 void lu_factor(double *A, std::uint32_t n, std::int32_t *pivots, int *info, double *work, hipStream_t stream);
-std::size_t lu_work_doubles(std::uint32_t n);
+// Throws std::runtime_error for a nonzero info: `singular` and the column, or the failed wait.
+void check_lu_status(int info, const char *singular);
 // Solve with the factors for nrhs right-hand sides in place (B n x nrhs).
 void lu_solve(const double *LU, std::uint32_t n, const std::int32_t *pivots, double *B, std::uint32_t nrhs,
               hipStream_t stream);

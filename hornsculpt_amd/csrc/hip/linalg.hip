@@ -1,18 +1,13 @@
 // Dense complex FP64 linear algebra for the Burton-Miller system, gfx950.
 //
 // Replaces the vendor calls of the reference dense path
-// (cusolverDnCgetrf/Cgetrs, cuda_solver.cu:1485-1513; cublasZgemv/Zaxpy/Dznrm2
-// in device_gmres.cu:115-157) with own kernels:
+// (cublasZgemv/Zaxpy/Dznrm2 in device_gmres.cu:115-157; the LU is in lu.hip) with own kernels:
 //   gemv            y = A X for up to 8 vectors (A FP64 or FP32, vectors FP64):
 //                   64 rows x 512 columns per workgroup, A streamed once (HBM
 //                   bound), deterministic split-K partials reduced in a second pass;
 //                   for one vector the column chunk (512, 1024 or 2048) is chosen by
 //                   timing the candidates once per (n, precision) on the live stream.
 //   project         CGS2 projections V^H w, one wavefront per (basis column, row block).
-//   lu_factor       right-looking blocked LU (panel 32, 4-column leaves): pivot
-//                   search, row interchanges, unit-lower TRSM, and trailing
-//                   updates on the FP64 matrix cores.
-//   lu_solve        blocked forward/backward substitution.
 #include "../autotune.hpp"
 #include "device.hpp"
 
@@ -326,338 +321,6 @@ __global__ void subtract_vectors(const double *b, const double *ax, std::size_t 
     const std::size_t i = static_cast<std::size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i < count)
         r[i] = b[i] - ax[i];
-}
-
-// ---------------- LU ----------------
-constexpr int kPanel = 32;
-constexpr int kPanelThreads = 1024;
-
-// Factor the leaf columns [j0, j0 + w) of the panel [k0, pe) over rows [j0, n).
-// Per column j, three barriers: (1) pivot search (largest squared modulus, ties to
-// the lowest row) reduced per wavefront into LDS; (2) every thread finishes the
-// reduction itself, a few threads stage the pivot row p's leaf entries in LDS and
-// one records the pivot; (3) one pass over the rows r > j writes
-// l = a[r][j] / a[p][j] and a[r][c] - l u[c] for the leaf columns c > j, reading
-// row j in place of row p (the interchange folded in), while the thread of row p
-// also writes the pivot row into row j, and the other panel columns (the leaf's
-// factored columns before j included) swap rows j and p. One workgroup; pivot rows
-// are recorded as absolute indices.
-constexpr int kLeaf = 4;
-__global__ __launch_bounds__(kPanelThreads) void lu_leaf(double *A, std::uint32_t n, std::uint32_t k0, std::uint32_t j0,
-                                                        std::uint32_t w, std::uint32_t pe, std::int32_t *piv, int *info) {
-    __shared__ double best[kPanelThreads / 64];
-    __shared__ std::uint32_t where[kPanelThreads / 64];
-    __shared__ double2 u[kLeaf];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid / 64;
-    double2 *A2 = reinterpret_cast<double2 *>(A);
-    auto at = [&](std::uint32_t c, std::uint32_t r) -> double2 & { return A2[static_cast<std::size_t>(c) * n + r]; };
-    const std::uint32_t je = j0 + w;
-    for (std::uint32_t j = j0; j < je; ++j) {
-        double bv = -1;
-        std::uint32_t bi = j;
-        for (std::uint32_t r = j + tid; r < n; r += kPanelThreads) {
-            const double2 v = at(j, r);
-            const double m = v.x * v.x + v.y * v.y;
-            if (m > bv) {
-                bv = m;
-                bi = r;
-            }
-        }
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            const double ov = __shfl_xor(bv, off, 64);
-            const std::uint32_t oi = __shfl_xor(bi, off, 64);
-            if (ov > bv || (ov == bv && oi < bi)) {
-                bv = ov;
-                bi = oi;
-            }
-        }
-        if (lane == 0) {
-            best[wave] = bv;
-            where[wave] = bi;
-        }
-        __syncthreads(); // (1)
-        double v = best[0];
-        std::uint32_t p = where[0];
-        for (int q = 1; q < kPanelThreads / 64; ++q)
-            if (best[q] > v || (best[q] == v && where[q] < p)) {
-                v = best[q];
-                p = where[q];
-            }
-        if (tid < static_cast<int>(je - j))
-            u[tid] = at(j + tid, p);
-        if (tid == 0) {
-            piv[j] = static_cast<std::int32_t>(p);
-            if (!(v > 0) && *info == 0)
-                *info = static_cast<int>(j) + 1;
-        }
-        __syncthreads(); // (2): every thread has p and the pivot row's leaf entries
-        const double2 d = u[0];
-        const double dd = d.x * d.x + d.y * d.y;
-        const double ir = dd > 0 ? d.x / dd : 0.0, ii = dd > 0 ? -d.y / dd : 0.0; // 1/a = conj(a)/|a|^2
-        for (std::uint32_t r = j + 1 + tid; r < n; r += kPanelThreads) {
-            const std::uint32_t src = r == p ? j : r; // row p receives the old row j
-            const double2 a = at(j, src);
-            const double lr = a.x * ir - a.y * ii, li = a.x * ii + a.y * ir;
-            for (std::uint32_t c = j + 1; c < je; ++c) {
-                const double2 b = at(c, src), uc = u[c - j];
-                at(c, r) = double2{b.x - (lr * uc.x - li * uc.y), b.y - (lr * uc.y + li * uc.x)};
-            }
-            at(j, r) = double2{lr, li};
-            if (r == p) // this thread read the old row j; the pivot row takes its place
-                for (std::uint32_t c = j; c < je; ++c)
-                    at(c, j) = u[c - j];
-        }
-        if (p != j) // the other panel columns (incl. this leaf's L columns before j): interchange rows j and p
-            for (std::uint32_t c = k0 + tid; c < pe; c += kPanelThreads)
-                if (c < j || c >= je) {
-                    const double2 t = at(c, j);
-                    at(c, j) = at(c, p);
-                    at(c, p) = t;
-                }
-        __syncthreads(); // (3)
-    }
-}
-
-// Apply the panel's row interchanges to the columns outside it.
-__global__ void lu_swap(double *A, std::uint32_t n, std::uint32_t k0, std::uint32_t nb, const std::int32_t *piv) {
-    const std::uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= n || (c >= k0 && c < k0 + nb))
-        return;
-    double *col = A + 2 * static_cast<std::size_t>(c) * n;
-    for (std::uint32_t j = k0; j < k0 + nb; ++j) {
-        const std::uint32_t p = static_cast<std::uint32_t>(piv[j]);
-        if (p != j) {
-            const double t0 = col[2 * j], t1 = col[2 * j + 1];
-            col[2 * j] = col[2 * p];
-            col[2 * j + 1] = col[2 * p + 1];
-            col[2 * p] = t0;
-            col[2 * p + 1] = t1;
-        }
-    }
-}
-
-// U12 = L11^{-1} A12 (unit lower nb x nb L11 at [k0, k0 + nb)) for the columns
-// [k0 + nb, c_end): 64 threads per 64 columns. The block's nb x 64 slice of A12 is
-// staged through LDS with consecutive threads on consecutive rows of a column
-// (coalesced), each thread solves one column from LDS, and the slice is written back
-// the same way. Rows of the staged slice are padded against LDS bank conflicts.
-__global__ __launch_bounds__(64) void lu_trsm(double *A, std::uint32_t n, std::uint32_t k0, std::uint32_t nb,
-                                              std::uint32_t c_end) {
-    __shared__ double L[kPanel][kPanel][2];
-    __shared__ double2 X[64][kPanel + 1];
-    for (std::uint32_t e = threadIdx.x; e < nb * nb; e += 64) {
-        const std::uint32_t r = e % nb, c = e / nb;
-        L[r][c][0] = A[2 * ((static_cast<std::size_t>(k0) + c) * n + k0 + r)];
-        L[r][c][1] = A[2 * ((static_cast<std::size_t>(k0) + c) * n + k0 + r) + 1];
-    }
-    const std::uint32_t c_first = k0 + nb + blockIdx.x * 64;
-    const std::uint32_t cols = min(64u, c_end - c_first);
-    double2 *A2 = reinterpret_cast<double2 *>(A);
-    for (std::uint32_t e = threadIdx.x; e < cols * nb; e += 64) {
-        const std::uint32_t q = e / nb, r = e % nb;
-        X[q][r] = A2[static_cast<std::size_t>(c_first + q) * n + k0 + r];
-    }
-    __syncthreads();
-    const std::uint32_t t = threadIdx.x;
-    if (t < cols) {
-        double xr[kPanel], xi[kPanel];
-        for (std::uint32_t i = 0; i < nb; ++i) {
-            double vr = X[t][i].x, vi = X[t][i].y;
-            for (std::uint32_t j = 0; j < i; ++j) {
-                vr -= L[i][j][0] * xr[j] - L[i][j][1] * xi[j];
-                vi -= L[i][j][0] * xi[j] + L[i][j][1] * xr[j];
-            }
-            xr[i] = vr;
-            xi[i] = vi;
-            X[t][i] = double2{vr, vi};
-        }
-    }
-    __syncthreads();
-    for (std::uint32_t e = threadIdx.x; e < cols * nb; e += 64) {
-        const std::uint32_t q = e / nb, r = e % nb;
-        A2[static_cast<std::size_t>(c_first + q) * n + k0 + r] = X[q][r];
-    }
-}
-
-// C -= L U over rows [r_begin, r_end) and columns [c_begin, c_end) with L = A[rows][k0 ..
-// k0 + nb) and U = A[k0 .. k0 + nb)[columns], K = nb <= 2 kPanel (staged through LDS in chunks
-// of kPanel, the accumulators carried across the chunks), on the FP64 matrix cores: 256
-// threads per 64 x 64 complex output tile, each wavefront a 32 x 32 quarter as 2 x 2 blocks
-// of 16 x 16. The product is formed transposed, D = U^T L^T (v_mfma_f64_16x16x4f64: A[i][k]
-// from lane i + 16 k, B[k][j] from lane j + 16 k, D[i][j] in lane j + 16 (i mod 4), register
-// i / 4), so D's index j runs over rows and each 16-lane group writes 16 consecutive rows of
-// one column. A complex MAC is four real MFMAs: Re += Ur Lr - Ui Li, Im += Ui Lr + Ur Li.
-// Each chunk's K is padded with zeros to a multiple of 4.
-typedef double lu_v4d __attribute__((ext_vector_type(4)));
-__global__ __launch_bounds__(256) void lu_update_mfma(double *A, std::uint32_t n, std::uint32_t k0, std::uint32_t nb,
-                                                      std::uint32_t r_begin, std::uint32_t r_end,
-                                                      std::uint32_t c_begin, std::uint32_t c_end) {
-    __shared__ double2 Ls[kPanel][65]; // Ls[k][q] = A[r0 + q][k0 + kc + k] (padded row: no bank conflicts across k)
-    __shared__ double2 Us[kPanel][65]; // Us[k][q] = A[k0 + kc + k][c0 + q]
-    const std::uint32_t r0 = r_begin + blockIdx.x * 64, c0 = c_begin + blockIdx.y * 64;
-    const double2 *A2 = reinterpret_cast<const double2 *>(A);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = lane & 15, kq = lane >> 4;
-    const int rh = wave & 1, ch = wave >> 1;
-    // this lane's old C values, loaded first so their latency hides behind the staging and the MFMAs
-    double2 cold[2][2][4];
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const std::uint32_t r = r0 + rh * 32 + a * 16 + i, c = c0 + ch * 32 + b * 16 + 4 * v + kq;
-                cold[a][b][v] = r < r_end && c < c_end ? A2[static_cast<std::size_t>(c) * n + r] : double2{0.0, 0.0};
-            }
-    lu_v4d accr[2][2], acci[2][2];
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-            accr[a][b] = acci[a][b] = lu_v4d{0.0, 0.0, 0.0, 0.0};
-    for (std::uint32_t kc = 0; kc < nb; kc += kPanel) {
-        const std::uint32_t kn = min(static_cast<std::uint32_t>(kPanel), nb - kc), kpad = (kn + 3) & ~3u;
-        if (kc)
-            __syncthreads(); // the previous chunk's reads are done
-        for (std::uint32_t e = threadIdx.x; e < kpad * 64; e += 256) {
-            const std::uint32_t kk = e / 64, q = e % 64, r = r0 + q, c = c0 + q;
-            const std::size_t k = static_cast<std::size_t>(k0) + kc + kk;
-            Ls[kk][q] = kk < kn && r < r_end ? A2[k * n + r] : double2{0.0, 0.0};
-            Us[kk][q] = kk < kn && c < c_end ? A2[static_cast<std::size_t>(c) * n + k] : double2{0.0, 0.0};
-        }
-        __syncthreads();
-        for (std::uint32_t ks = 0; ks < kpad / 4; ++ks) {
-            const std::uint32_t kk = 4 * ks + kq;
-            double lr[2], li[2], ur[2], ui[2];
-#pragma unroll
-            for (int a = 0; a < 2; ++a) {
-                const double2 l = Ls[kk][rh * 32 + a * 16 + i];
-                lr[a] = l.x;
-                li[a] = l.y;
-            }
-#pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                const double2 u = Us[kk][ch * 32 + b * 16 + i];
-                ur[b] = u.x;
-                ui[b] = u.y;
-            }
-            // four passes over the eight independent accumulators: no MFMA waits on the one before it
-#pragma unroll
-            for (int a = 0; a < 2; ++a)
-#pragma unroll
-                for (int b = 0; b < 2; ++b) {
-                    accr[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ur[b], lr[a], accr[a][b], 0, 0, 0);
-                    acci[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ui[b], lr[a], acci[a][b], 0, 0, 0);
-                }
-#pragma unroll
-            for (int a = 0; a < 2; ++a)
-#pragma unroll
-                for (int b = 0; b < 2; ++b) {
-                    accr[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(-ui[b], li[a], accr[a][b], 0, 0, 0);
-                    acci[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ur[b], li[a], acci[a][b], 0, 0, 0);
-                }
-        }
-    }
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const std::uint32_t r = r0 + rh * 32 + a * 16 + i, c = c0 + ch * 32 + b * 16 + 4 * v + kq;
-                if (r < r_end && c < c_end)
-                    reinterpret_cast<double2 *>(A)[static_cast<std::size_t>(c) * n + r] =
-                        double2{cold[a][b][v].x - accr[a][b][v], cold[a][b][v].y - acci[a][b][v]};
-            }
-}
-
-// Row interchanges of every panel applied to the right-hand sides.
-__global__ void apply_pivots(double *B, std::uint32_t n, const std::int32_t *piv, std::uint32_t nrhs) {
-    const std::uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= nrhs)
-        return;
-    double *x = B + 2 * static_cast<std::size_t>(e) * n;
-    for (std::uint32_t j = 0; j < n; ++j) {
-        const std::uint32_t p = static_cast<std::uint32_t>(piv[j]);
-        if (p != j) {
-            const double t0 = x[2 * j], t1 = x[2 * j + 1];
-            x[2 * j] = x[2 * p];
-            x[2 * j + 1] = x[2 * p + 1];
-            x[2 * p] = t0;
-            x[2 * p + 1] = t1;
-        }
-    }
-}
-
-constexpr int kSolveBlock = 64;
-
-// Solve the diagonal block [j0, j0+nb) (lower unit or upper) for every rhs; one
-// workgroup per rhs. The block is staged in LDS first (column by column, rows over
-// the threads: coalesced, independent loads), so the nb sequential steps read LDS
-// only; the arithmetic and its order are those of a column-by-column substitution.
-__global__ __launch_bounds__(64) void block_substitute(const double *LU, std::uint32_t n, double *B, std::uint32_t j0,
-                                                      std::uint32_t nb, int upper) {
-    __shared__ double2 blk[kSolveBlock][kSolveBlock + 1]; // blk[c][r] = LU[j0 + r][j0 + c]
-    __shared__ double2 x[kSolveBlock];
-    const double2 *LU2 = reinterpret_cast<const double2 *>(LU);
-    double2 *b = reinterpret_cast<double2 *>(B) + static_cast<std::size_t>(blockIdx.x) * n + j0;
-    const int t = threadIdx.x, m = static_cast<int>(nb);
-    if (t < m) {
-        for (int c = 0; c < m; ++c)
-            blk[c][t] = LU2[(static_cast<std::size_t>(j0) + c) * n + j0 + t];
-        x[t] = b[t];
-    }
-    __syncthreads();
-    if (!upper) {
-        for (int j = 0; j < m; ++j) {
-            if (t > j && t < m) {
-                const double2 l = blk[j][t], xj = x[j];
-                x[t].x -= l.x * xj.x - l.y * xj.y;
-                x[t].y -= l.x * xj.y + l.y * xj.x;
-            }
-            __syncthreads();
-        }
-    } else {
-        for (int jj = m - 1; jj >= 0; --jj) {
-            if (t == jj) {
-                const double2 u = blk[jj][jj];
-                const double d = u.x * u.x + u.y * u.y;
-                const double vr = x[jj].x, vi = x[jj].y;
-                x[jj] = double2{(vr * u.x + vi * u.y) / d, (vi * u.x - vr * u.y) / d};
-            }
-            __syncthreads();
-            if (t < jj) {
-                const double2 u = blk[jj][t], xj = x[jj];
-                x[t].x -= u.x * xj.x - u.y * xj.y;
-                x[t].y -= u.x * xj.y + u.y * xj.x;
-            }
-            __syncthreads();
-        }
-    }
-    if (t < m)
-        b[t] = x[t];
-}
-
-// B[rows] -= LU[rows, j0:j0+nb] * B[j0:j0+nb] for rows outside the block
-// (below for the lower sweep, above for the upper sweep).
-__global__ __launch_bounds__(256) void block_eliminate(const double *LU, std::uint32_t n, double *B, std::uint32_t j0,
-                                                      std::uint32_t nb, std::uint32_t r_begin, std::uint32_t r_end) {
-    const std::uint32_t r = r_begin + blockIdx.x * 256 + threadIdx.x;
-    const double *b = B + 2 * static_cast<std::size_t>(blockIdx.y) * n;
-    if (r >= r_end)
-        return;
-    double re = 0, im = 0;
-    for (std::uint32_t j = 0; j < nb; ++j) {
-        const double lr = LU[2 * ((static_cast<std::size_t>(j0) + j) * n + r)],
-                     li = LU[2 * ((static_cast<std::size_t>(j0) + j) * n + r) + 1];
-        const double xr = b[2 * (j0 + j)], xi = b[2 * (j0 + j) + 1];
-        re += lr * xr - li * xi;
-        im += lr * xi + li * xr;
-    }
-    double *out = B + 2 * (static_cast<std::size_t>(blockIdx.y) * n + r);
-    out[0] -= re;
-    out[1] -= im;
 }
 
 // ---- block-Jacobi preconditioner: explicit inverses of the kJacobi x kJacobi
@@ -1260,91 +923,6 @@ void launch_residual(const void *A, bool fp32, std::uint32_t n, const double *b,
     launch_gemv(A, fp32, n, x, residual, nvec, scratch, stream);
     const std::size_t count = 2 * static_cast<std::size_t>(n) * nvec;
     hipLaunchKernelGGL(subtract_vectors, dim3((count + 255) / 256), dim3(256), 0, stream, b, residual, count, residual);
-}
-
-std::size_t lu_work_doubles(std::uint32_t) { return 0; }
-
-namespace {
-
-// The leaves of panel [k0, k0 + nb): pivoted 4-column leaves (row interchanges inside the
-// panel), each leaf's U rows of the panel and the rank-4 update of the panel below it.
-void factor_panel(double *A, std::uint32_t n, std::uint32_t k0, std::uint32_t nb, std::int32_t *piv, int *info,
-                  hipStream_t stream) {
-    const std::uint32_t pe = k0 + nb;
-    for (std::uint32_t j0 = k0; j0 < pe; j0 += kLeaf) {
-        const std::uint32_t w = std::min<std::uint32_t>(kLeaf, pe - j0);
-        hipLaunchKernelGGL(lu_leaf, dim3(1), dim3(kPanelThreads), 0, stream, A, n, k0, j0, w, pe, piv, info);
-        if (j0 + w >= pe)
-            continue;
-        hipLaunchKernelGGL(lu_trsm, dim3(1), dim3(64), 0, stream, A, n, j0, w, pe);
-        const std::uint32_t below = n - j0 - w;
-        hipLaunchKernelGGL(lu_update_mfma, dim3((below + 63) / 64, 1), dim3(256), 0, stream, A, n, j0, w, j0 + w, n,
-                           j0 + w, pe);
-    }
-}
-
-// C -= L U over rows [r0, r1) x columns [c0, c1) with K = A's columns / rows [k0, k0 + nb).
-void update(double *A, std::uint32_t n, std::uint32_t k0, std::uint32_t nb, std::uint32_t r0, std::uint32_t r1,
-            std::uint32_t c0, std::uint32_t c1, hipStream_t stream) {
-    if (r1 > r0 && c1 > c0)
-        hipLaunchKernelGGL(lu_update_mfma, dim3((r1 - r0 + 63) / 64, (c1 - c0 + 63) / 64), dim3(256), 0, stream, A, n,
-                           k0, nb, r0, r1, c0, c1);
-}
-
-} // namespace
-
-// Right-looking blocked LU with partial pivoting: panels of kPanel columns, each
-// factored in leaves of kLeaf columns (lu_leaf on one workgroup, then the leaf's
-// rows of U for the rest of the panel and a rank-kLeaf update of the panel below
-// it on every CU), then the panel's interchanges outside it, U12 and the trailing
-// update on the matrix cores, two panels to one rank-2 kPanel trailing update.
-void lu_factor(double *A, std::uint32_t n, std::int32_t *piv, int *info, double *, hipStream_t stream) {
-    // Pairs of kPanel-column panels P1 = [k0, e1), P2 = [e1, e2) share one rank-2 kPanel
-    // trailing update (half the trailing matrix's HBM traffic per flop of rank-kPanel
-    // updates): P1 is factored, its interchanges applied and its U rows solved over every
-    // later column; P1's update reaches P2's columns before P2 is factored; after P2's
-    // interchanges (applied to the still un-updated trailing rows and to P1's L rows alike)
-    // P1's update reaches P2's U rows, P2's U rows are solved, and the rows below P2 take
-    // both panels' updates at once.
-    for (std::uint32_t k0 = 0; k0 < n; k0 += 2 * kPanel) {
-        const std::uint32_t n1 = std::min<std::uint32_t>(kPanel, n - k0), e1 = k0 + n1;
-        factor_panel(A, n, k0, n1, piv, info, stream);
-        hipLaunchKernelGGL(lu_swap, dim3((n + 63) / 64), dim3(64), 0, stream, A, n, k0, n1, piv);
-        if (e1 == n)
-            break;
-        hipLaunchKernelGGL(lu_trsm, dim3((n - e1 + 63) / 64), dim3(64), 0, stream, A, n, k0, n1, n);
-        const std::uint32_t n2 = std::min<std::uint32_t>(kPanel, n - e1), e2 = e1 + n2;
-        update(A, n, k0, n1, e1, n, e1, e2, stream);
-        factor_panel(A, n, e1, n2, piv, info, stream);
-        hipLaunchKernelGGL(lu_swap, dim3((n + 63) / 64), dim3(64), 0, stream, A, n, e1, n2, piv);
-        if (e2 == n)
-            break;
-        update(A, n, k0, n1, e1, e2, e2, n, stream);
-        hipLaunchKernelGGL(lu_trsm, dim3((n - e2 + 63) / 64), dim3(64), 0, stream, A, n, e1, n2, n);
-        update(A, n, k0, n1 + n2, e2, n, e2, n, stream);
-    }
-}
-
-void lu_solve(const double *LU, std::uint32_t n, const std::int32_t *piv, double *B, std::uint32_t nrhs,
-              hipStream_t stream) {
-    hipLaunchKernelGGL(apply_pivots, dim3((nrhs + 63) / 64), dim3(64), 0, stream, B, n, piv, nrhs);
-    for (std::uint32_t j0 = 0; j0 < n; j0 += kSolveBlock) {
-        const std::uint32_t nb = std::min<std::uint32_t>(kSolveBlock, n - j0);
-        hipLaunchKernelGGL(block_substitute, dim3(nrhs), dim3(64), 0, stream, LU, n, B, j0, nb, 0);
-        const std::uint32_t rows = n - j0 - nb;
-        if (rows)
-            hipLaunchKernelGGL(block_eliminate, dim3((rows + 255) / 256, nrhs), dim3(256), 0, stream, LU, n, B, j0, nb,
-                               j0 + nb, n);
-    }
-    const std::uint32_t last = ((n - 1) / kSolveBlock) * kSolveBlock;
-    for (std::int64_t j0 = last; j0 >= 0; j0 -= kSolveBlock) {
-        const std::uint32_t nb = std::min<std::uint32_t>(kSolveBlock, n - static_cast<std::uint32_t>(j0));
-        hipLaunchKernelGGL(block_substitute, dim3(nrhs), dim3(64), 0, stream, LU, n, B, static_cast<std::uint32_t>(j0),
-                           nb, 1);
-        if (j0 > 0)
-            hipLaunchKernelGGL(block_eliminate, dim3((static_cast<std::uint32_t>(j0) + 255) / 256, nrhs), dim3(256), 0,
-                               stream, LU, n, B, static_cast<std::uint32_t>(j0), nb, 0u, static_cast<std::uint32_t>(j0));
-    }
 }
 
 std::size_t jacobi_factor_doubles(std::uint32_t n) {

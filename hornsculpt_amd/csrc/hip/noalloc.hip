@@ -1,8 +1,8 @@
 // Dense complex LU solve that allocates no device memory.
 //
 // The factorization needs device memory beyond the caller's matrix and
-// right-hand sides: the pivot rows (n int32) and the singular-pivot status
-// word. Here they live in one file-scope device array (`scratch`) instead of
+// right-hand sides: the pivot rows (n int32), the singular-pivot status
+// word and the exchange words of the panel's workgroups. Here they live in one file-scope device array (`scratch`) instead of
 // hipMalloc'd buffers, so the entry point can serve callers that may not
 // allocate (code under stream capture, tight serving loops, harnesses that
 // forbid hipMalloc). Every GPU the library runs on holds its own copy of the
@@ -24,12 +24,13 @@
 namespace {
 // Largest n the scratch array holds pivots for.
 constexpr std::uint32_t kNoAllocMaxOrder = 65536;
-// Layout: status word at offset 0 (256-byte slot), pivots from offset 256.
+// Layout: status word at offset 0 (256-byte slot), pivots from offset 256, then the exchange words.
 constexpr std::size_t kStatusBytes = 256;
-constexpr std::size_t kScratchBytes = kStatusBytes + sizeof(std::int32_t) * kNoAllocMaxOrder;
+constexpr std::size_t kExchangeOffset = kStatusBytes + sizeof(std::int32_t) * kNoAllocMaxOrder;
+constexpr std::size_t kScratchBytes = kExchangeOffset + sizeof(double) * hsbem::dev::kLuWorkDoubles;
 } // namespace
 
-// 256 KiB + 256 B per GPU, held until the process ends.
+// 752 KiB per GPU, held until the process ends.
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 namespace hsbem::dev {
@@ -76,12 +77,11 @@ void dense_lu_solve_noalloc(int device, hipStream_t stream, std::uint32_t n, dou
     auto *pivots = reinterpret_cast<std::int32_t *>(base + kStatusBytes);
     hipLaunchKernelGGL(clear_status, dim3(1), dim3(1), 0, stream, status);
     hip_check(hipGetLastError(), "status clear");
-    lu_factor(A, n, pivots, status, nullptr, stream);
+    lu_factor(A, n, pivots, status, reinterpret_cast<double *>(base + kExchangeOffset), stream);
     int code = 0;
     hip_check(hipMemcpyAsync(&code, status, sizeof(int), hipMemcpyDeviceToHost, stream), "status download");
     hip_check(hipStreamSynchronize(stream), "LU sync");
-    if (code)
-        throw std::runtime_error("LU factorization failed at pivot " + std::to_string(code));
+    check_lu_status(code, "LU factorization failed at pivot ");
     lu_solve(A, n, pivots, B, nrhs, stream);
     hip_check(hipStreamSynchronize(stream), "LU solve sync");
 }

@@ -1447,9 +1447,10 @@ std::shared_ptr<PreparedRequest> MeshSolver::prepare(const Request &req) const {
     const bool lu = !mixed && num.solver == 0;
     const std::uint64_t nv2 = static_cast<std::uint64_t>(nv) * nv, nd1 = std::max<std::uint32_t>(P->nd, 1);
     const std::uint64_t nobs = P->observers.size();
-    const std::uint64_t scratch = std::max({dev::gemv_scratch_doubles(nv, std::min<std::uint32_t>(ne, 8)),
-                                            dev::reduction_scratch_doubles(nv, num.gmres_restart + 1), std::size_t{4096}});
     const bool fmm = num.acceleration == 1;
+    const std::uint64_t scratch = std::max({dev::gemv_scratch_doubles(nv, std::min<std::uint32_t>(ne, 8)),
+                                            dev::reduction_scratch_doubles(nv, num.gmres_restart + 1), std::size_t{4096},
+                                            lu && !fmm ? dev::kLuWorkDoubles : 0});
     std::uint64_t bytes = (fmm ? 0 : (mixed ? 8 : 16) * nv2) + 16 * nv * nd1 + 16 * nd1 * ne + 3 * 16ull * nv * ne +
                           16ull * nt * ne + 8 * scratch + 4ull * nt;
     if (fmm) {
@@ -1503,10 +1504,12 @@ void MeshSolver::bind(const PreparedRequest &P, Workspace &ws) {
     ws.r.resize(2 * static_cast<std::size_t>(nv) * ne);
     ws.flux.resize(2 * static_cast<std::size_t>(nt) * ne);
     ws.flux_column.upload(P.flux_column, ws.stream);
+    const bool lu = !fmm && !mixed && num.solver == 0;
     const std::size_t scratch = std::max({dev::gemv_scratch_doubles(nv, std::min<std::uint32_t>(ne, 8)),
-                                          dev::reduction_scratch_doubles(nv, num.gmres_restart + 1), std::size_t{4096}});
+                                          dev::reduction_scratch_doubles(nv, num.gmres_restart + 1), std::size_t{4096},
+                                          lu ? dev::kLuWorkDoubles : 0});
     ws.scratch.resize(scratch);
-    if (!fmm && !mixed && num.solver == 0) {
+    if (lu) {
         ws.LU.resize(2 * nv2);
         ws.pivots.resize(nv);
     }
@@ -1676,13 +1679,12 @@ FrequencyResult MeshSolver::solve_frequency(const PreparedRequest &P, std::size_
         hip_check(hipMemcpyAsync(ws.LU.data(), ws.A.data(), ws.A.bytes(), hipMemcpyDeviceToDevice, s), "LU copy");
         hip_check(hipMemsetAsync(ws.error.data(), 0, sizeof(int), s), "clear info");
         const auto t_f = Clock::now();
-        dev::lu_factor(ws.LU.data(), nv, ws.pivots.data(), ws.error.data(), nullptr, s);
+        dev::lu_factor(ws.LU.data(), nv, ws.pivots.data(), ws.error.data(), ws.scratch.data(), s);
         int info = 0;
         hip_check(hipMemcpyAsync(&info, ws.error.data(), sizeof(int), hipMemcpyDeviceToHost, s), "info");
         hip_check(hipStreamSynchronize(s), "LU sync");
         fr.ms[2] = ms_since(t_f);
-        if (info)
-            throw std::runtime_error("LU factorization hit a zero pivot at column " + std::to_string(info));
+        dev::check_lu_status(info, "LU factorization hit a zero pivot at column ");
         const auto t_t = Clock::now();
         hip_check(hipMemcpyAsync(ws.x.data(), ws.rhs.data(), ws.rhs.bytes(), hipMemcpyDeviceToDevice, s), "rhs copy");
         dev::lu_solve(ws.LU.data(), nv, ws.pivots.data(), ws.x.data(), ne, s);
