@@ -8,13 +8,15 @@
 //                   orientations, every 3x3 pair block accumulated in two LDS node
 //                   tiles (ds_add) flushed once per tile to HBM, so global atomics
 //                   drop from 18 per ordered pair to about one per tile entry.
-//   touching_jobs   one wavefront per touching pair: Sauter-Schwab (u,v,w) tuples
-//                   over lanes with the radial coordinate innermost (every sector map
-//                   is linear in r), shuffle reduction, one lane scatters. Always FP64.
-//   near_patches    one thread per tensor near patch (16x16 or 64x64 points of the
-//                   patch's test and trial sub-triangles), two-stage contraction as
-//                   for regular pairs with the affine sub-triangle maps applied on
-//                   the fly; one scatter per patch.
+//   touching_jobs   16 lanes per touching pair: Sauter-Schwab (u,v,w) tuples over
+//                   lanes with the radial coordinate innermost (every sector map is
+//                   linear in r), DPP sums, a lane per entry scatters. Always FP64.
+//   near_tiles      one workgroup per chunk of the tensor near patches of a cluster pair,
+//                   one thread per patch (16x16 or 64x64 points of the patch's test and
+//                   trial sub-triangles), two-stage contraction as for regular pairs
+//                   with the affine sub-triangle maps applied on the fly; entries
+//                   gathered in LDS node tiles. near_patches: the same for a CSR, one
+//                   scatter per patch.
 //   near_jobs       one wavefront per near job holding a projection-fan patch,
 //                   patch points over lanes.
 //   mass            1/2 M_pp into A, -alpha 1/2 M_pq into the flux columns.
@@ -236,12 +238,13 @@ __device__ __forceinline__ double dot3(const double *a, const double *b) { retur
 // Pair constants are formed in FP64 and rounded to R; wscale = 4 A_x A_y / (4 pi)
 // (times the area fraction of a near patch). N = 0 takes n points from `rule` for
 // both panels; N > 0 takes the test points from `rule` and the trial points from
-// `yrule` (N of them, unrolled: a kernel-argument array). bad is raised when the
+// `yrule` (N of them, unrolled: a kernel-argument array). x_first and x_step take part of
+// the test points (the moments are sums over them). bad is raised when the
 // sum of G is not finite (a zero or invalid distance somewhere in the pair).
 template <class R, int N = 0>
 __device__ __forceinline__ void contract(MomentsT<R> &m, const Frame &t, const Frame &s, double wscale_d,
                                          const R *rule, int n_runtime, double k, bool &bad,
-                                         const R (*yrule)[4] = nullptr) {
+                                         const R (*yrule)[4] = nullptr, int x_first = 0, int x_step = 1) {
     const int n = N > 0 ? N : n_runtime;
     const double b[3] = {t.v0[0] - s.v0[0], t.v0[1] - s.v0[1], t.v0[2] - s.v0[2]};
     const double inv_k = 1.0 / k;
@@ -263,7 +266,7 @@ __device__ __forceinline__ void contract(MomentsT<R> &m, const Frame &t, const F
         se2[i] = static_cast<R>(s.e2[i]);
     }
 #pragma unroll 1
-    for (int xi = 0; xi < n; ++xi) {
+    for (int xi = x_first; xi < n; xi += x_step) {
         const R *xp = rule + 4 * xi;
         const R x1 = xp[1], x2 = xp[2], xw = xp[3] * wscale;
         R blt[3];
@@ -920,12 +923,40 @@ __device__ __forceinline__ void scatter_pair(const AssemblyArgs &args, M *A, con
     }
 }
 
+// Matrix moment (i, j) of a pair with its curl term, a - i g (curl_i . curl_j) / k.
+__device__ __forceinline__ CplxT<double> with_curls(const AssemblyArgs &args, CplxT<double> a, CplxT<double> g,
+                                                    std::uint32_t ti, std::uint32_t si, int i, int j) {
+    const PanelView &pv = args.panels;
+    double cc = 0;
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+        cc += g_at(pv.geo, G_C0 + 3 * i + c, pv.nt, ti) * g_at(pv.geo, G_C0 + 3 * j + c, pv.nt, si);
+    cc /= args.k;
+    return {a.re + g.im * cc, a.im - g.re * cc};
+}
+
 // Destination of a pair's moments in the dense path.
 template <class M> struct DenseSink {
     template <class R>
     __device__ __forceinline__ void operator()(const AssemblyArgs &args, const MomentsT<R> &m, std::uint32_t,
                                                std::uint32_t ti, std::uint32_t si) const {
         scatter_pair(args, matrix_of<M>(args), m, ti, si);
+    }
+    // One entry of a pair: matrix entry (e / 3, e % 3) for e < 9 from its moment v and the sum g
+    // of G, flux moment e - 9 otherwise.
+    __device__ __forceinline__ void entry(const AssemblyArgs &args, CplxT<double> v, CplxT<double> g, std::uint32_t,
+                                          std::uint32_t ti, std::uint32_t si, int e) const {
+        const PanelView &pv = args.panels;
+        const int i = e < 9 ? e / 3 : e - 9;
+        const std::uint32_t row = pv.nodes[static_cast<std::size_t>(i) * pv.nt + ti];
+        const double rs = args.row_scale[row];
+        if (e < 9) {
+            const CplxT<double> a = with_curls(args, v, g, ti, si, i, e % 3);
+            const std::uint32_t col = pv.nodes[static_cast<std::size_t>(e % 3) * pv.nt + si];
+            atomic_add_entry(matrix_of<M>(args) + 2 * (static_cast<std::size_t>(col) * pv.nv + row), a.re * rs, a.im * rs);
+        } else if (const std::int32_t fc = args.flux_column[si]; fc >= 0) {
+            atomic_add_entry(args.BD + 2 * (static_cast<std::size_t>(fc) * pv.nv + row), v.re * rs, v.im * rs);
+        }
     }
 };
 
@@ -972,6 +1003,22 @@ struct CsrSink {
                                  static_cast<double>(m.b[i].re) * rs, static_cast<double>(m.b[i].im) * rs);
         }
     }
+    __device__ __forceinline__ void entry(const AssemblyArgs &args, CplxT<double> w, CplxT<double> g, std::uint32_t job,
+                                          std::uint32_t ti, std::uint32_t si, int e) const {
+        if (!(v.masks[job] >> e & 1u))
+            return;
+        const PanelView &pv = args.panels;
+        const int i = e < 9 ? e / 3 : e - 9;
+        const std::uint32_t row = pv.nodes[static_cast<std::size_t>(i) * pv.nt + ti];
+        const double rs = args.row_scale[row];
+        if (e < 9) {
+            const CplxT<double> a = with_curls(args, w, g, ti, si, i, e % 3);
+            const std::uint32_t col = pv.nodes[static_cast<std::size_t>(e % 3) * pv.nt + si];
+            atomic_add_entry(v.values + 2 * csr_slot(v.row_offsets, v.columns, row, col), a.re * rs, a.im * rs);
+        } else if (const std::uint32_t fc = v.face_column[si]; fc != UINT32_MAX) {
+            atomic_add_entry(v.flux_values + 2 * csr_slot(v.flux_offsets, v.flux_columns, row, fc), w.re * rs, w.im * rs);
+        }
+    }
 };
 
 __device__ __forceinline__ void load_geo(const PanelView &pv, std::uint32_t t, double *g) {
@@ -980,15 +1027,37 @@ __device__ __forceinline__ void load_geo(const PanelView &pv, std::uint32_t t, d
         g[f] = g_at(pv.geo, f, pv.nt, t);
 }
 
+// Sum over the 16 lanes of a DPP row, in each of them.
+template <int kControl> __device__ __forceinline__ double dpp_add(double v) {
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+    const int lo = static_cast<int>(b), hi = static_cast<int>(b >> 32);
+    const std::uint32_t olo = __builtin_amdgcn_update_dpp(0, lo, kControl, 0xf, 0xf, false);
+    const std::uint32_t ohi = __builtin_amdgcn_update_dpp(0, hi, kControl, 0xf, 0xf, false);
+    return v + __builtin_bit_cast(double, static_cast<unsigned long long>(ohi) << 32 | olo);
+}
+
+__device__ __forceinline__ double row_sum(double v) {
+    v = dpp_add<0xB1>(v);  // lanes 1 apart
+    v = dpp_add<0x4E>(v);  // 2 apart
+    v = dpp_add<0x141>(v); // mirrored halves of the row
+    return dpp_add<0x140>(v); // mirrored row
+}
+
 // Touching pairs are integrated in FP64 in both forms (the hypersingular weak
-// form); M is the matrix element type.
+// form); M is the matrix element type. 16 lanes per job: the 26 sums then cost four
+// DPP additions each (a wavefront per job spent as much on its shuffles as on the
+// samples), and 12 lanes add one entry each. 20.7k-triangle horn (270 thousand jobs): 2.54
+// -> 1.09 ms.
+constexpr int kTouchingLanes = 16;
+constexpr std::uint32_t touching_groups(std::uint32_t jobs) {
+    return (jobs + 256 / kTouchingLanes - 1) / (256 / kTouchingLanes);
+}
 template <class Sink>
 __global__ __launch_bounds__(256) void touching_jobs(AssemblyArgs args, const TouchingJob *jobs, std::uint32_t njobs,
                                                      const double *gauss, unsigned order, Sink sink) {
-    const std::uint32_t job = blockIdx.x * 4 + threadIdx.x / 64;
-    const int lane = threadIdx.x & 63;
-    if (job >= njobs)
-        return;
+    const std::uint32_t mine = (blockIdx.x * 256 + threadIdx.x) / kTouchingLanes;
+    const std::uint32_t job = min(mine, njobs - 1); // a lane without a job takes part in the sums' row only
+    const int lane = threadIdx.x & (kTouchingLanes - 1);
     const TouchingJob tj = jobs[job];
     const PanelView &pv = args.panels;
     double gt[G_COUNT], gs[G_COUNT];
@@ -998,49 +1067,69 @@ __global__ __launch_bounds__(256) void touching_jobs(AssemblyArgs args, const To
     const bool coincident = topo == Topology::coincident;
     const PairConst<double> pc = pair_const<double>(gt, gs, args.k);
     const double wscale = 4.0 * gt[G_AREA] * gs[G_AREA] * 0.07957747154594766788;
-    const double bx = gt[G_V0] - gs[G_V0], by = gt[G_V0 + 1] - gs[G_V0 + 1], bz = gt[G_V0 + 2] - gs[G_V0 + 2];
+    // Edges from the common vertex (first in both permutations): the points, sums and
+    // entries below are in the permuted vertex order, where every sector map is linear in r
+    // about vertex 0 and no array is indexed at run time.
+    double et1[3], et2[3], es1[3], es2[3];
+    auto edges = [](const double *g, const std::uint8_t *order, double *e1, double *e2) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const double u = g[G_E1 + c], w = g[G_E2 + c];
+            auto corner = [u, w](std::uint8_t l) { return (l == 1 ? 1.0 : 0.0) * u + (l == 2 ? 1.0 : 0.0) * w; };
+            const double from = corner(order[0]);
+            e1[c] = corner(order[1]) - from;
+            e2[c] = corner(order[2]) - from;
+        }
+    };
+    edges(gt, tj.permutation.test, et1, et2);
+    edges(gs, tj.permutation.trial, es1, es2);
     const unsigned per = order * order * order;
     const unsigned total = sector_count(topo) * per;
-    const int at = tj.permutation.test[0], as = tj.permutation.trial[0];
     MomentsT<double> m;
     zero_t(m);
     bool bad = false;
-    for (unsigned idx = lane; idx < total; idx += 64) {
+    for (unsigned idx = lane; idx < total; idx += kTouchingLanes) {
         unsigned tuple = idx % per;
         const unsigned wi = tuple % order;
         tuple /= order;
         const unsigned vi = tuple % order;
         const unsigned ui = tuple / order;
-        PairPoint c = sauter_schwab_point(topo, idx / per, 1.0, gauss[2 * ui], gauss[2 * vi], gauss[2 * wi]);
-        c.weight *= gauss[2 * ui + 1] * gauss[2 * vi + 1] * gauss[2 * wi + 1];
-        const PairPoint p = unpermute(c, tj.permutation);
-        const double ltx = gt[G_E1] * p.test[1] + gt[G_E2] * p.test[2],
-                     lty = gt[G_E1 + 1] * p.test[1] + gt[G_E2 + 1] * p.test[2],
-                     ltz = gt[G_E1 + 2] * p.test[1] + gt[G_E2 + 2] * p.test[2];
-        const double lsx = gs[G_E1] * p.trial[1] + gs[G_E2] * p.trial[2],
-                     lsy = gs[G_E1 + 1] * p.trial[1] + gs[G_E2 + 1] * p.trial[2],
-                     lsz = gs[G_E1 + 2] * p.trial[1] + gs[G_E2 + 2] * p.trial[2];
-        const double dx = bx + (ltx - lsx), dy = by + (lty - lsy), dz = bz + (ltz - lsz);
+        PairPoint p = sauter_schwab_point(topo, idx / per, 1.0, gauss[2 * ui], gauss[2 * vi], gauss[2 * wi]);
+        p.weight *= gauss[2 * ui + 1] * gauss[2 * vi + 1] * gauss[2 * wi + 1] * wscale;
+        double d[3];
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+            d[c] = (et1[c] * p.test[1] + et2[c] * p.test[2]) - (es1[c] * p.trial[1] + es2[c] * p.trial[2]);
         for (unsigned ri = 0; ri < order; ++ri) {
             const double r = gauss[2 * ri];
-            double xt[3], xs[3];
-#pragma unroll
-            for (int i = 0; i < 3; ++i) {
-                xt[i] = r * p.test[i];
-                xs[i] = r * p.trial[i];
-            }
-            xt[at] += 1 - r;
-            xs[as] += 1 - r;
+            const double xt[3] = {1 - r * (1 - p.test[0]), r * p.test[1], r * p.test[2]};
+            const double xs[3] = {1 - r * (1 - p.trial[0]), r * p.trial[1], r * p.trial[2]};
             const SampleT<double> s =
-                sample(r * dx, r * dy, r * dz, c.weight * r * r * r * gauss[2 * ri + 1] * wscale, pc, coincident, bad);
+                sample(r * d[0], r * d[1], r * d[2], p.weight * r * r * r * gauss[2 * ri + 1], pc, coincident, bad);
             add_sample_t(m, s, xt, xs);
         }
     }
     if (bad)
         atomicExch(args.error, ERR_DISTANCE);
-    wave_reduce_t(m);
-    if (lane == 0)
-        sink(args, m, job, tj.test, tj.trial);
+    CplxT<double> mine_of = {0, 0};
+    auto total_of = [&](CplxT<double> v, int e) {
+        const CplxT<double> s = {row_sum(v.re), row_sum(v.im)};
+        if (lane == e)
+            mine_of = s;
+        return s;
+    };
+#pragma unroll
+    for (int i = 0; i < 9; ++i)
+        total_of(m.a[i], i);
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+        total_of(m.b[i], 9 + i);
+    const CplxT<double> g = total_of(m.g, -1);
+    if (mine < njobs && lane < 12) { // from the permuted vertex order to the panels' own
+        const int i = jobs[job].permutation.test[lane < 9 ? lane / 3 : lane - 9],
+                  j = jobs[job].permutation.trial[lane < 9 ? lane % 3 : 0];
+        sink.entry(args, mine_of, g, job, tj.test, tj.trial, lane < 9 ? 3 * i + j : 9 + i);
+    }
 }
 
 __device__ __forceinline__ FanPanel fan_of(const double *g) {
@@ -1142,6 +1231,108 @@ __global__ __launch_bounds__(256) void near_patches(AssemblyArgs args, const Nea
     if (bad)
         atomicExch(args.error, ERR_DISTANCE);
     sink(args, m, idx, it.test, it.trial);
+}
+
+// Tensor near patches of the dense matrix, one workgroup per chunk of a cluster pair's.
+// Bound by atomics when each patch adds its 18 entries to the matrix itself: the patches of
+// a pair, and pairs with common nodes, hit the same entries. Here they add to LDS node tiles
+// as the regular pairs do ([B node][A node] for a test panel in A, [A node][B node] for one
+// in B) and each touched entry goes to the matrix once per chunk. A chunk with few patches
+// gives a patch to several threads, each a part of its test points. 1.5k-triangle horn
+// (498 thousand patches): 2.20 -> 0.43 ms FP32, 2.16 -> 0.88 ms FP64; 20.7k triangles (1.31
+// million): 3.3 -> 1.09 and 3.2 -> 2.6 ms, now bound by the samples.
+template <class R>
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 2)))
+void near_tiles(AssemblyArgs args, ClusterView cl, const NearChunk *chunks,
+                                                           const NearPatchItem *items, const PairPatch *patches,
+                                                           const double *rules, TileRules<R> fixed) {
+    __shared__ R tab[kTileNodes * kStrideAB];
+    __shared__ R tba[kTileNodes * kStrideBA];
+    __shared__ R srule[4 * (16 + 64)];
+    const NearChunk chunk = chunks[blockIdx.x];
+    const std::uint32_t a0 = cl.node_offsets[chunk.a], nA = cl.node_offsets[chunk.a + 1] - a0;
+    const std::uint32_t b0 = cl.node_offsets[chunk.b], nB = cl.node_offsets[chunk.b + 1] - b0;
+    const bool diag = chunk.a == chunk.b;
+    const PanelView &pv = args.panels;
+    const int tid = threadIdx.x;
+    for (int e = tid; e < kTileNodes * kStrideAB; e += kTileThreads)
+        tab[e] = tba[e] = R(0);
+    for (int e = tid; e < 4 * 16; e += kTileThreads)
+        srule[e] = static_cast<R>(rules[4 * kRule8 + e]);
+    for (int e = tid; e < 4 * 64; e += kTileThreads)
+        srule[4 * 16 + e] = static_cast<R>(rules[4 * kRule14 + e]);
+    __syncthreads();
+    const bool high = patches[items[chunk.first].patch].degree == 14;
+    std::uint32_t parts = 1;
+    while (parts < 16 && (2 * parts * chunk.count <= kTileThreads || (high && parts < 16)))
+        parts *= 2;
+    bool bad = false;
+    for (std::uint32_t u = tid; u < chunk.count * parts; u += kTileThreads) {
+        const NearPatchItem it = items[chunk.first + u / parts];
+        const int part = static_cast<int>(u % parts);
+        const PairPatch &patch = patches[it.patch];
+        double gt[G_COUNT], gs[G_COUNT];
+        load_geo(pv, it.test, gt);
+        load_geo(pv, it.trial, gs);
+        MomentsT<R> m;
+        zero_t(m);
+        const bool swap = it.swap & kNearSwap;
+        const double *Tt = swap ? patch.trial : patch.test, *Ts = swap ? patch.test : patch.trial;
+        const Frame ft = sub_frame(frame_of(gt), Tt), fs = sub_frame(frame_of(gs), Ts);
+        const double wscale = 4.0 * gt[G_AREA] * gs[G_AREA] * 0.07957747154594766788 * patch.area_fraction;
+        if (high)
+            contract<R>(m, ft, fs, wscale, srule + 4 * 16, 64, args.k, bad, nullptr, part, parts);
+        else
+            contract<R, 16>(m, ft, fs, wscale, srule, 16, args.k, bad, fixed.d8, part, parts);
+        to_parent(m, Tt, Ts);
+        const bool in_b = it.swap & kNearTestInB;
+        const R inv_k = static_cast<R>(1.0 / args.k);
+        int row[3], col[3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            row[i] = cl.local[static_cast<std::size_t>(i) * pv.nt + it.test];
+            col[i] = cl.local[static_cast<std::size_t>(i) * pv.nt + it.trial];
+        }
+        R *tile = in_b ? tba : tab;
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+                const R cc = static_cast<R>(gt[G_C0 + 3 * i] * gs[G_C0 + 3 * j] + gt[G_C0 + 3 * i + 1] * gs[G_C0 + 3 * j + 1] +
+                                            gt[G_C0 + 3 * i + 2] * gs[G_C0 + 3 * j + 2]) * inv_k;
+                R *slot = tile + col[j] * kStrideAB + 2 * row[i];
+                unsafeAtomicAdd(slot, m.a[3 * i + j].re + m.g.im * cc);
+                unsafeAtomicAdd(slot + 1, m.a[3 * i + j].im - m.g.re * cc);
+            }
+        const std::int32_t fc = args.flux_column[it.trial];
+        if (fc >= 0)
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                const std::uint32_t node = pv.nodes[static_cast<std::size_t>(i) * pv.nt + it.test];
+                const double rs = args.row_scale[node];
+                atomic_add_entry(args.BD + 2 * (static_cast<std::size_t>(fc) * pv.nv + node),
+                                 static_cast<double>(m.b[i].re) * rs, static_cast<double>(m.b[i].im) * rs);
+            }
+    }
+    if (bad)
+        atomicExch(args.error, ERR_DISTANCE);
+    __syncthreads();
+    R *A = matrix_of<R>(args);
+    auto flush = [&](const R *tile, std::uint32_t r0, std::uint32_t nr, std::uint32_t c0, std::uint32_t nc) {
+        for (std::uint32_t e = tid; e < nr * nc; e += kTileThreads) {
+            const std::uint32_t r = e % nr, c = e / nr;
+            const R re = tile[c * kStrideAB + 2 * r], im = tile[c * kStrideAB + 2 * r + 1];
+            if (re != R(0) || im != R(0)) {
+                const std::uint32_t row = cl.nodes[r0 + r], col = cl.nodes[c0 + c];
+                const R rs = static_cast<R>(args.row_scale[row]);
+                unsafeAtomicAdd(A + 2 * (static_cast<std::size_t>(col) * pv.nv + row), re * rs);
+                unsafeAtomicAdd(A + 2 * (static_cast<std::size_t>(col) * pv.nv + row) + 1, im * rs);
+            }
+        }
+    };
+    flush(tab, a0, nA, b0, nB);
+    if (!diag)
+        flush(tba, b0, nB, a0, nA);
 }
 
 template <class M> __global__ void mass_terms(AssemblyArgs args) {
@@ -1298,7 +1489,7 @@ void launch_near_operator(const NearOperatorLaunch &L, hipStream_t stream) {
         hipLaunchKernelGGL(regular_pairs<CsrSink>, dim3((L.regular_count + 255) / 256), dim3(256), 0, stream, L.args,
                            L.near, L.regular, L.regular_count, L.rules, with(L.regular_masks));
     if (L.touching_count)
-        hipLaunchKernelGGL(touching_jobs<CsrSink>, dim3((L.touching_count + 3) / 4), dim3(256), 0, stream, L.args,
+        hipLaunchKernelGGL(touching_jobs<CsrSink>, dim3(touching_groups(L.touching_count)), dim3(256), 0, stream, L.args,
                            L.touching, L.touching_count, L.gauss, L.singular_order, with(L.touching_masks));
     if (L.patch_count)
         hipLaunchKernelGGL((near_patches<double, CsrSink>), dim3((L.patch_count + 255) / 256), dim3(256), 0, stream,
@@ -1375,7 +1566,7 @@ void launch_regular(const AssemblyLaunch &L, hipStream_t stream) {
 void launch_touching(const AssemblyLaunch &L, hipStream_t stream) {
     if (!L.touching_count)
         return;
-    const dim3 grid((L.touching_count + 3) / 4);
+    const dim3 grid(touching_groups(L.touching_count));
     if (L.args.A32)
         hipLaunchKernelGGL(touching_jobs<DenseSink<float>>, grid, dim3(256), 0, stream, L.args, L.touching,
                            L.touching_count, L.gauss, L.singular_order, DenseSink<float>{});
@@ -1385,14 +1576,16 @@ void launch_touching(const AssemblyLaunch &L, hipStream_t stream) {
 }
 
 void launch_near(const AssemblyLaunch &L, hipStream_t stream) {
-    if (L.near_item_count) {
-        const dim3 grid((L.near_item_count + 255) / 256);
-        if (L.args.A32)
-            hipLaunchKernelGGL((near_patches<float, DenseSink<float>>), grid, dim3(256), 0, stream, L.args,
-                               L.near_items, L.near_item_count, L.patches, L.rules, DenseSink<float>{});
-        else
-            hipLaunchKernelGGL((near_patches<double, DenseSink<double>>), grid, dim3(256), 0, stream, L.args,
-                               L.near_items, L.near_item_count, L.patches, L.rules, DenseSink<double>{});
+    if (L.near_chunk_count) {
+        if (L.args.A32) {
+            static const TileRules<float> fixed = make_tile_rules<float>();
+            hipLaunchKernelGGL(near_tiles<float>, dim3(L.near_chunk_count), dim3(kTileThreads), 0, stream, L.args,
+                               L.clusters, L.near_chunks, L.near_items, L.patches, L.rules, fixed);
+        } else {
+            static const TileRules<double> fixed = make_tile_rules<double>();
+            hipLaunchKernelGGL(near_tiles<double>, dim3(L.near_chunk_count), dim3(kTileThreads), 0, stream, L.args,
+                               L.clusters, L.near_chunks, L.near_items, L.patches, L.rules, fixed);
+        }
     }
     if (L.near_count) {
         const dim3 grid((L.near_count + 3) / 4);

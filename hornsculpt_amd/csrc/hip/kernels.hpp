@@ -101,6 +101,13 @@ void launch_near_operator(const NearOperatorLaunch &launch, hipStream_t stream);
 void launch_csr_apply(const std::uint32_t *row_offsets, const std::uint32_t *columns, const double *values,
                       std::uint32_t rows, const double *x, double *y, hipStream_t stream);
 
+// A run of near_items whose panels lie in clusters a <= b, all of degree 8 or all of 14;
+// bit 1 of an item's swap: the test panel lies in b (and a != b).
+struct NearChunk {
+    std::uint32_t a, b, first, count;
+};
+inline constexpr std::uint32_t kNearSwap = 1, kNearTestInB = 2;
+
 struct AssemblyLaunch {
     AssemblyArgs args;
     ClusterView clusters;
@@ -116,8 +123,9 @@ struct AssemblyLaunch {
     unsigned singular_order;
     const NearJob *near_jobs;              // jobs with a projection-fan patch (per-job kernel)
     std::uint32_t near_count;
-    const NearPatchItem *near_items;       // tensor patches of the other jobs (per-patch kernel)
-    std::uint32_t near_item_count;
+    const NearPatchItem *near_items;       // tensor patches of the other jobs, grouped by cluster pair
+    const NearChunk *near_chunks;          // runs of one cluster pair and one rule
+    std::uint32_t near_chunk_count;
     const PairPatch *patches;
     // regular tiles: trial panels per wavefront block (4, 8 or 16) of the general and
     // of the far tiles

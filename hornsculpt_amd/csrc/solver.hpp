@@ -258,8 +258,9 @@ struct DevicePlan {
     InteractionPlan plan;
     DeviceBuffer<TouchingJob> touching;
     DeviceBuffer<NearJob> near;                // jobs with a projection-fan patch
-    DeviceBuffer<dev::NearPatchItem> near_items; // tensor patches of all other jobs
-    std::uint32_t near_job_count{}, near_item_count{};
+    DeviceBuffer<dev::NearPatchItem> near_items; // tensor patches of all other jobs, grouped by cluster pair
+    DeviceBuffer<dev::NearChunk> near_chunks;
+    std::uint32_t near_job_count{}, near_chunk_count{};
     DeviceBuffer<PairPatch> patches;
     DeviceBuffer<std::uint32_t> near_offsets, near_trials;
     DeviceBuffer<std::uint8_t> whole;
@@ -274,7 +275,7 @@ struct DevicePlan {
     std::uint64_t last_use{}; // plan cache recency (MeshSolver::plans_)
     std::uint64_t device_bytes() const {
         return touching.capacity_bytes() + near.capacity_bytes() + near_items.capacity_bytes() +
-               patches.capacity_bytes() + near_offsets.capacity_bytes() + near_trials.capacity_bytes() +
+               near_chunks.capacity_bytes() + patches.capacity_bytes() + near_offsets.capacity_bytes() + near_trials.capacity_bytes() +
                whole.capacity_bytes() + gauss.capacity_bytes() + tiles.capacity_bytes();
     }
 };
@@ -410,6 +411,7 @@ class MeshSolver {
     DeviceBuffer<std::uint32_t> cluster_panel_offsets_, cluster_panels_, cluster_node_offsets_, cluster_nodes_;
     DeviceBuffer<double> cluster_far_; // per cluster: the bounds of the far tiles' fixed-point scale
     std::uint32_t cluster_count_{};
+    std::vector<std::uint32_t> cluster_of_; // per panel
     std::vector<ClusterBounds> cluster_bounds_;
     std::map<std::tuple<unsigned, unsigned, double, double, unsigned, double, bool>, std::shared_ptr<DevicePlan>> plans_;
     std::mutex plan_mutex_;       // serialises plan and near-structure builds
