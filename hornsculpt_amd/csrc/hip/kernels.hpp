@@ -111,10 +111,11 @@ inline constexpr std::uint32_t kNearSwap = 1, kNearTestInB = 2;
 struct AssemblyLaunch {
     AssemblyArgs args;
     ClusterView clusters;
-    // (test cluster, trial cluster) tiles: the first far_tiles are far tiles whose
-    // pairs all qualify for degree 4 at this wavenumber (uniform path).
+    // (test cluster, trial cluster) tiles: the first separated_tiles are far tiles (no touching
+    // or near pair, at least three edges apart: degree 4 or 6), of which the first far_tiles
+    // have pairs of degree 4 only at this wavenumber.
     const std::uint32_t *tiles;
-    std::uint32_t tile_count, far_tiles;
+    std::uint32_t tile_count, far_tiles, separated_tiles;
     NearView near;
     const double *rules;                   // kRuleTableCount x 4 doubles
     const TouchingJob *touching;

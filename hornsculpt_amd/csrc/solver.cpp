@@ -687,6 +687,8 @@ dev::AssemblyLaunch MeshSolver::assembly_launch(const DevicePlan &p, const Numer
         std::upper_bound(p.far_tile_edge.begin(), p.far_tile_edge.end(), 0.0,
                          [k](double, double h) { return !(k * h <= .5); }) -
         p.far_tile_edge.begin());
+    // above k h = 2 a separated pair may take no regular rule: the plan lists no far tile then
+    L.separated_tiles = static_cast<std::uint32_t>(p.far_tile_edge.size());
     L.near = {p.near_offsets.data(), p.near_trials.data(), p.whole.size() ? p.whole.data() : nullptr};
     L.rules = rules_.data();
     L.touching = p.touching.data();
@@ -712,17 +714,22 @@ void MeshSolver::tune_regular_tiles(dev::AssemblyLaunch &L, bool mixed, hipStrea
     std::ostringstream key;
     key << "mesh " << std::hex << hash_ << std::dec << " (" << nt() << " panels) " << (mixed ? "fp32" : "fp64");
     auto tune = [&](bool far) {
-        const std::uint32_t count = far ? L.far_tiles : L.tile_count - L.far_tiles;
+        const std::uint32_t count = far ? L.separated_tiles : L.tile_count - L.separated_tiles;
         if (!count)
             return 8u;
         dev::AssemblyLaunch T = L;
         const std::uint32_t prefix = std::min(count, std::max(512u, count / 32));
         if (far) {
-            T.tile_count = T.far_tiles = prefix;
+            // the kind that most of the far tiles have
+            const bool low = 2 * L.far_tiles >= count;
+            const std::uint32_t first = low ? 0 : L.far_tiles, kind = low ? L.far_tiles : count - L.far_tiles;
+            T.tiles = L.tiles + 2 * static_cast<std::size_t>(first);
+            T.tile_count = T.separated_tiles = std::min(kind, prefix);
+            T.far_tiles = low ? T.tile_count : 0;
         } else {
-            T.tiles = L.tiles + 2 * static_cast<std::size_t>(L.far_tiles);
+            T.tiles = L.tiles + 2 * static_cast<std::size_t>(L.separated_tiles);
             T.tile_count = prefix;
-            T.far_tiles = 0;
+            T.far_tiles = T.separated_tiles = 0;
         }
         return autotune::choose(
             "tile_trial_block", key.str() + (far ? " far" : " general"), {4, 8, 16}, 8, s,
