@@ -1,17 +1,26 @@
-// Device-resident restart cycle of GMRES (one right-hand side).
+// Arnoldi steps of GMRES: the fused orthogonalization that every GMRES here runs (one
+// system, several at once, host-driven or captured), and the device-resident restart
+// cycle of one right-hand side.
 //
-// The Arnoldi step index j, the Hessenberg column, the Givens rotations, the
+// Orthogonalization. At the orders of a horn (500 to 20,000 unknowns) the basis is a few
+// MB, so a step is bound by its chain of dependent launches and not by bytes. CGS2, the
+// norm and v_{j+1} = w / |w| are therefore four launches: each reduction's partials are
+// summed by every workgroup of the launch that needs them (`blocks` x (j + 1) values out of
+// L2) instead of by a launch of their own, and each workgroup keeps its rows of w in LDS
+// from the subtraction to the next projection. As ten launches (two projections, two sums,
+// two subtractions, two norm launches, scaling, rotation) an iteration at n = 523 took
+// @OLD523 us with its product, and takes @NEW523 us now; at n = 10,373, @OLD10K us and @NEW10K us.
+//
+// Restart cycle. The Arnoldi step index j, the Hessenberg column, the Givens rotations, the
 // rotated right-hand side g and the stop decision live in device memory, so one
-// Arnoldi step is a fixed sequence of launches (current = v_j, the operator, CGS2
-// against v_0..v_j, the norm, v_{j+1}, the rotation) whose arguments never change:
+// Arnoldi step is a fixed sequence of launches (the operator's input from v_j, the
+// product, the orthogonalization, the rotation) whose arguments never change:
 // the host captures it once into a HIP graph and replays it once per iteration,
 // reading the state back only every few steps. Each kernel reads j from the state
 // and returns at once when the cycle has stopped (target met, breakdown or the
-// step limit), so replays queued past the stop cost only their launches.
-//
-// The arithmetic is that of the host-driven cycle: the same projection, subtraction
-// and norm reductions in the same order, and the rotation formulas of the host
-// Givens loop evaluated in FP64 on one lane.
+// step limit), so replays queued past the stop cost only their launches. The rotation
+// publishes the next j and the stop flag while other workgroups of its launch still run:
+// they read the copies that the step's first kernel made.
 #include "device.hpp"
 #include "kernels.hpp"
 
@@ -23,9 +32,17 @@
 namespace hsbem::dev {
 namespace {
 
-constexpr int kRows = 512; // rows per projection workgroup (as the host-driven cycle)
+enum : int { S_J = 0, S_DONE = 1, S_USED = 2, S_LIMIT = 3, S_ERROR = 4, S_STEP_J = 5, S_STEP_DONE = 6 };
 
-enum : int { S_J = 0, S_DONE = 1, S_USED = 2, S_LIMIT = 3, S_ERROR = 4 };
+constexpr int kThreads = 512, kWaves = kThreads / 64;
+constexpr std::uint32_t kColumns = 256; // basis columns whose coefficients are held in LDS at a time
+constexpr std::uint32_t kFinishRows = 256;
+
+// Rows per lane of a pass: 64 rows per workgroup up to n = 4096 (at most 64 workgroups),
+// 128 up to 16384 (at most 128), else 256, so that the partials that every workgroup sums
+// stay near 100 KB at 60 columns while small systems still spread over the chip.
+std::uint32_t rows_per_lane(std::uint32_t n) { return n <= 4096 ? 1 : n <= 16384 ? 2 : 4; }
+std::uint32_t pass_blocks(std::uint32_t n) { return (n + 64 * rows_per_lane(n) - 1) / (64 * rows_per_lane(n)); }
 
 struct Layout {
     std::uint32_t stride; // restart + 1
@@ -41,8 +58,6 @@ struct Layout {
     __host__ __device__ std::size_t total() const { return H() + 2 * static_cast<std::size_t>(stride) * stride; }
 };
 
-__device__ __forceinline__ bool stopped(const int *st) { return st[S_DONE] != 0; }
-
 __global__ void cycle_begin(int *st, double *small, Layout L, double beta, double target, std::uint32_t limit) {
     const std::uint32_t t = threadIdx.x;
     for (std::size_t i = t; i < 2 * static_cast<std::size_t>(L.stride); i += blockDim.x)
@@ -57,116 +72,225 @@ __global__ void cycle_begin(int *st, double *small, Layout L, double beta, doubl
         st[S_USED] = 0;
         st[S_LIMIT] = static_cast<int>(limit);
         st[S_ERROR] = 0;
+        st[S_STEP_J] = 0;
+        st[S_STEP_DONE] = st[S_DONE];
     }
 }
 
-__global__ void load_current(const double *basis, std::uint32_t n, const int *st, double *current) {
-    if (stopped(st))
-        return;
-    const std::size_t j = static_cast<std::size_t>(st[S_J]);
-    const std::uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < 2 * n)
-        current[i] = basis[2 * j * n + i];
+// The step index of this launch; false when the cycle has stopped.
+__device__ __forceinline__ bool step_index(const ArnoldiBatch &B, std::uint32_t &j) {
+    j = B.state ? static_cast<std::uint32_t>(B.state[S_STEP_J]) : B.j;
+    return !(B.state && B.state[S_STEP_DONE] != 0);
 }
 
-// part[b][c] = sum over rows of block b of conj(V[:, c]) w, c <= j (one wavefront per column).
-__global__ __launch_bounds__(256) void project_step(const double *V, std::uint32_t n, const int *st, const double *w,
-                                                   double *part) {
-    if (stopped(st))
-        return;
-    const std::uint32_t m = static_cast<std::uint32_t>(st[S_J]) + 1;
-    const std::uint32_t r0 = blockIdx.x * kRows;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x / 64;
-    const std::uint32_t c = blockIdx.y * 4 + wave;
-    if (c >= m)
-        return;
-    double re = 0, im = 0;
-    for (std::uint32_t r = r0 + lane; r < min(r0 + kRows, n); r += 64) {
-        const double vr = V[2 * (static_cast<std::size_t>(c) * n + r)], vi = V[2 * (static_cast<std::size_t>(c) * n + r) + 1];
-        const double xr = w[2 * r], xi = w[2 * r + 1];
-        re += vr * xr + vi * xi;
-        im += vr * xi - vi * xr;
+// First kernel of a step: j and the stop flag as the last rotation left them, copied for
+// the kernels that follow.
+__device__ __forceinline__ bool step_begin(const ArnoldiBatch &B, std::uint32_t &j) {
+    if (!B.state) {
+        j = B.j;
+        return true;
     }
-    re = wave_sum(re);
-    im = wave_sum(im);
-    if (lane == 0) {
-        part[2 * (static_cast<std::size_t>(blockIdx.x) * m + c)] = re;
-        part[2 * (static_cast<std::size_t>(blockIdx.x) * m + c) + 1] = im;
+    const int done = B.state[S_DONE], at = B.state[S_J];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        B.state[S_STEP_J] = at;
+        B.state[S_STEP_DONE] = done;
     }
+    j = static_cast<std::uint32_t>(at);
+    return done == 0;
 }
 
-__global__ void sum_step(const double *part, std::uint32_t blocks, const int *st, double *out) {
-    if (stopped(st))
+// in[a] = v_j of the a-th system of the batch.
+__global__ __launch_bounds__(256) void load_step(ArnoldiBatch B, double2 *in) {
+    std::uint32_t j;
+    if (!step_begin(B, j))
         return;
-    const std::uint32_t m = static_cast<std::uint32_t>(st[S_J]) + 1;
-    const std::uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= m)
-        return;
-    double re = 0, im = 0;
-    for (std::uint32_t b = 0; b < blocks; ++b) {
-        re += part[2 * (static_cast<std::size_t>(b) * m + c)];
-        im += part[2 * (static_cast<std::size_t>(b) * m + c) + 1];
-    }
-    out[2 * c] = re;
-    out[2 * c + 1] = im;
+    const std::uint32_t i = blockIdx.x * 256 + threadIdx.x, a = blockIdx.y;
+    if (i < B.n)
+        in[static_cast<std::size_t>(a) * B.n + i] =
+            reinterpret_cast<const double2 *>(B.basis + B.which[a] * B.basis_stride)[static_cast<std::size_t>(j) * B.n + i];
 }
 
-__global__ void subtract_step(const double *V, std::uint32_t n, const int *st, const double *h, double *w) {
-    if (stopped(st))
+// in[a] = M^{-1} v_j with the 64-wide block-Jacobi inverses: one workgroup per block and
+// system, each wavefront a quarter of the block's columns.
+__global__ __launch_bounds__(256) void jacobi_step(ArnoldiBatch B, const double2 *inverses, double2 *in) {
+    __shared__ double2 sv[64], red[4][64];
+    std::uint32_t j;
+    if (!step_begin(B, j))
         return;
-    const std::uint32_t m = static_cast<std::uint32_t>(st[S_J]) + 1;
-    const std::uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= n)
-        return;
-    double re = w[2 * r], im = w[2 * r + 1];
-    for (std::uint32_t c = 0; c < m; ++c) {
-        const double vr = V[2 * (static_cast<std::size_t>(c) * n + r)], vi = V[2 * (static_cast<std::size_t>(c) * n + r) + 1];
-        const double hr = h[2 * c], hi = h[2 * c + 1];
-        re -= vr * hr - vi * hi;
-        im -= vr * hi + vi * hr;
-    }
-    w[2 * r] = re;
-    w[2 * r + 1] = im;
-}
-
-__global__ __launch_bounds__(256) void norm_step_partial(const double *x, std::uint32_t n, const int *st, double *part) {
-    if (stopped(st))
-        return;
-    __shared__ double red[4];
-    double s = 0;
-    for (std::uint32_t r = blockIdx.x * 256 + threadIdx.x; r < n; r += gridDim.x * 256) {
-        const double a = x[2 * r] * 1.0, b = x[2 * r + 1] * 1.0;
-        s += a * a + b * b;
-    }
-    s = wave_sum(s);
-    if ((threadIdx.x & 63) == 0)
-        red[threadIdx.x / 64] = s;
+    const std::uint32_t blk = blockIdx.x, r0 = blk * 64, a = blockIdx.y;
+    const int i = threadIdx.x & 63, wave = threadIdx.x / 64;
+    const double2 *f = inverses + static_cast<std::size_t>(blk) * 4096 + 1024 * wave;
+    double2 c[16];
+#pragma unroll
+    for (int t = 0; t < 16; ++t)
+        c[t] = f[t * 64 + i];
+    if (wave == 0)
+        sv[i] = r0 + i < B.n ? reinterpret_cast<const double2 *>(B.basis + B.which[a] * B.basis_stride)
+                                   [static_cast<std::size_t>(j) * B.n + r0 + i]
+                             : double2{0, 0};
     __syncthreads();
-    if (threadIdx.x == 0)
-        part[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
+    double re = 0, im = 0;
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+        const double2 v = sv[16 * wave + t];
+        re += c[t].x * v.x - c[t].y * v.y;
+        im += c[t].x * v.y + c[t].y * v.x;
+    }
+    red[wave][i] = double2{re, im};
+    __syncthreads();
+    if (wave == 0 && r0 + i < B.n)
+        in[static_cast<std::size_t>(a) * B.n + r0 + i] =
+            double2{red[0][i].x + red[1][i].x + red[2][i].x + red[3][i].x,
+                    red[0][i].y + red[1][i].y + red[2][i].y + red[3][i].y};
 }
 
-__global__ void norm_step_finish(const double *part, std::uint32_t blocks, const int *st, double *out) {
-    if (stopped(st))
-        return;
-    double s = 0;
-    for (std::uint32_t b = threadIdx.x; b < blocks; b += 64)
-        s += part[b];
-    s = wave_sum(s);
-    if (threadIdx.x == 0)
-        out[0] = s;
+// Sum over the wavefront of eight values: lane l returns the sum of v[l & 7]. Three
+// exchanges halve the values a lane carries and three more add the lanes that carry the
+// same one: 10 exchanges where eight separate sums take 48.
+__device__ __forceinline__ double wave_sum8(const double *v, int lane) {
+    double a[4], b[2];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const bool hi = lane & 4;
+        a[i] = (hi ? v[i + 4] : v[i]) + __shfl_xor(hi ? v[i] : v[i + 4], 4, 64);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const bool hi = lane & 2;
+        b[i] = (hi ? a[i + 2] : a[i]) + __shfl_xor(hi ? a[i] : a[i + 2], 2, 64);
+    }
+    const bool hi = lane & 1;
+    double s = (hi ? b[1] : b[0]) + __shfl_xor(hi ? b[0] : b[1], 1, 64);
+#pragma unroll
+    for (int off = 8; off < 64; off <<= 1)
+        s += __shfl_xor(s, off, 64);
+    return s;
 }
 
-// v_{j+1} = w / |w| (0 when |w| = 0).
-__global__ void store_next(const double *w, std::uint32_t n, const int *st, const double *norm2, double *basis) {
-    if (stopped(st))
+// One pass over the rows of w = v_{j+1}'s slot, 64 RK rows per workgroup, blockIdx.y the
+// system. kGather: w = the product's column-chunk partials summed, then part1[b][c] = this
+// block's share of conj(v_c) w. kFirst: h1 = the sum of part1, w -= V h1, part2 likewise.
+// kSecond: h2 = the sum of part2, w -= V h2, part1[b] = this block's |w|^2. (part1 is read
+// by kFirst only, so kSecond may write it.) Rows are lanes and the wavefronts share the
+// columns in the subtraction; a wavefront takes four columns at a time in the projection.
+enum Pass { kGather, kFirst, kSecond };
+template <int RK, Pass PASS>
+__global__ __launch_bounds__(kThreads) void arnoldi_pass(ArnoldiBatch B, const double2 *y, std::uint32_t chunks) {
+    constexpr int R = 64 * RK;
+    __shared__ double2 sw[R], red[kWaves * R], sh[kColumns];
+    std::uint32_t j;
+    if (!step_index(B, j))
         return;
-    const std::size_t j = static_cast<std::size_t>(st[S_J]);
-    const std::uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= 2 * n)
-        return;
-    const double v = *norm2;
-    basis[2 * (j + 1) * n + i] = v > 0 ? w[i] / sqrt(v) : 0.0;
+    const std::uint32_t m = j + 1, n = B.n, ld = B.restart + 1, blocks = gridDim.x, a = blockIdx.y, e = B.which[a];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x / 64;
+    const std::uint32_t r0 = blockIdx.x * R;
+    const double2 *V = reinterpret_cast<const double2 *>(B.basis + e * B.basis_stride);
+    double2 *w = reinterpret_cast<double2 *>(B.basis + e * B.basis_stride) + static_cast<std::size_t>(m) * n;
+    double2 *part1 = reinterpret_cast<double2 *>(B.part) + 2 * static_cast<std::size_t>(a) * blocks * ld;
+    double2 *part2 = part1 + static_cast<std::size_t>(blocks) * ld;
+    double2 acc[RK] = {};
+    if constexpr (PASS == kGather) {
+        for (std::uint32_t c = wave; c < chunks; c += kWaves)
+#pragma unroll
+            for (int k = 0; k < RK; ++k) {
+                const std::uint32_t row = r0 + 64 * k + lane;
+                if (row < n) {
+                    const double2 v = y[(static_cast<std::size_t>(a) * chunks + c) * n + row];
+                    acc[k].x += v.x;
+                    acc[k].y += v.y;
+                }
+            }
+    } else {
+        const double2 *part = PASS == kFirst ? part1 : part2;
+        double2 *h = reinterpret_cast<double2 *>(B.small + e * B.small_stride) + (PASS == kFirst ? 0 : ld);
+        for (std::uint32_t c0 = 0; c0 < m; c0 += kColumns) {
+            const std::uint32_t cn = min(kColumns, m - c0);
+            for (std::uint32_t q = 0; q < cn; q += 64) {
+                double2 s = {};
+                if (q + lane < cn)
+#pragma unroll 8
+                    for (std::uint32_t b = wave; b < blocks; b += kWaves) {
+                        const double2 v = part[static_cast<std::size_t>(b) * ld + c0 + q + lane];
+                        s.x += v.x;
+                        s.y += v.y;
+                    }
+                red[wave * 64 + lane] = s;
+                __syncthreads();
+                if (wave == 0 && q + lane < cn) {
+#pragma unroll
+                    for (int t = 1; t < kWaves; ++t) {
+                        s.x += red[t * 64 + lane].x;
+                        s.y += red[t * 64 + lane].y;
+                    }
+                    sh[q + lane] = s;
+                    if (blockIdx.x == 0)
+                        h[c0 + q + lane] = s;
+                }
+                __syncthreads();
+            }
+#pragma unroll 4
+            for (std::uint32_t c = wave; c < cn; c += kWaves) {
+                const double2 hc = sh[c];
+                const double2 *col = V + static_cast<std::size_t>(c0 + c) * n;
+#pragma unroll
+                for (int k = 0; k < RK; ++k) {
+                    const std::uint32_t row = r0 + 64 * k + lane;
+                    const double2 v = row < n ? col[row] : double2{0, 0};
+                    acc[k].x += v.x * hc.x - v.y * hc.y;
+                    acc[k].y += v.x * hc.y + v.y * hc.x;
+                }
+            }
+            __syncthreads();
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < RK; ++k)
+        red[wave * R + 64 * k + lane] = acc[k];
+    __syncthreads();
+    for (int t = threadIdx.x; t < R; t += kThreads) {
+        double2 s = red[t];
+#pragma unroll
+        for (int q = 1; q < kWaves; ++q) {
+            s.x += red[q * R + t].x;
+            s.y += red[q * R + t].y;
+        }
+        if (r0 + t < n) {
+            if (PASS != kGather)
+                s = double2{w[r0 + t].x - s.x, w[r0 + t].y - s.y};
+            w[r0 + t] = s;
+        }
+        sw[t] = r0 + t < n ? s : double2{0, 0};
+    }
+    __syncthreads();
+    if constexpr (PASS == kSecond) {
+        if (wave == 0) {
+            double s = 0;
+#pragma unroll
+            for (int k = 0; k < RK; ++k)
+                s += sw[64 * k + lane].x * sw[64 * k + lane].x + sw[64 * k + lane].y * sw[64 * k + lane].y;
+            s = wave_sum(s);
+            if (lane == 0)
+                reinterpret_cast<double *>(part1)[blockIdx.x] = s;
+        }
+    } else {
+        double *out = reinterpret_cast<double *>((PASS == kGather ? part1 : part2) + static_cast<std::size_t>(blockIdx.x) * ld);
+        for (std::uint32_t c = 4 * wave; c < m; c += 4 * kWaves) {
+            double v[8] = {};
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int k = 0; k < RK; ++k) {
+                    const std::uint32_t row = r0 + 64 * k + lane;
+                    const double2 x = row < n && c + u < m ? V[static_cast<std::size_t>(c + u) * n + row] : double2{0, 0};
+                    const double2 wr = sw[64 * k + lane];
+                    v[2 * u] += x.x * wr.x + x.y * wr.y;
+                    v[2 * u + 1] += x.x * wr.y - x.y * wr.x;
+                }
+            const double s = wave_sum8(v, lane);
+            if (lane < 8 && c + lane / 2 < m)
+                out[2 * c + lane] = s;
+        }
+    }
 }
 
 struct Cx {
@@ -180,28 +304,46 @@ __device__ __forceinline__ Cx cneg(Cx a) { return {-a.re, -a.im}; }
 __device__ __forceinline__ double cabs(Cx a) { return hypot(a.re, a.im); }
 
 // Column j of the Hessenberg matrix from the two CGS passes and |w|, the earlier
-// rotations applied to it, the new rotation, g rotated, and the stop decision.
-__global__ void givens_step(int *st, double *small, Layout L) {
-    if (threadIdx.x != 0 || stopped(st))
-        return;
-    const std::uint32_t j = static_cast<std::uint32_t>(st[S_J]);
+// rotations applied to it, the new rotation, g rotated, and the stop decision. The chain
+// of rotations is one lane's work on staged values (through global memory the three loads
+// of each rotation were its time: about 15 us at 60 columns).
+__device__ void rotate_column(int *st, double *small, Layout L, std::uint32_t j, double norm2, Cx *scol, Cx *ssn,
+                              double *scs) {
     Cx *col = reinterpret_cast<Cx *>(small + L.H()) + static_cast<std::size_t>(j) * L.stride;
     const Cx *h1 = reinterpret_cast<const Cx *>(small + L.h1()), *h2 = reinterpret_cast<const Cx *>(small + L.h2());
     Cx *g = reinterpret_cast<Cx *>(small + L.g()), *sn = reinterpret_cast<Cx *>(small + L.sn());
     double *cs = small + L.cs();
-    for (std::uint32_t i = 0; i <= j; ++i)
-        col[i] = cadd(h1[i], h2[i]);
-    for (std::uint32_t i = j + 2; i < L.stride; ++i)
-        col[i] = {0.0, 0.0};
-    const double next = sqrt(small[L.nrm()]);
-    col[j + 1] = {next, 0.0};
-    const bool breakdown = !(next > 0);
-    for (std::uint32_t i = 0; i < j; ++i) {
-        const Cx t = cadd(cscale(col[i], cs[i]), cmul(sn[i], col[i + 1]));
-        col[i + 1] = cadd(cmul(cneg(cconj(sn[i])), col[i]), cscale(col[i + 1], cs[i]));
-        col[i] = t;
+    const std::uint32_t tid = threadIdx.x;
+    const double next = sqrt(norm2);
+    Cx cur = cadd(h1[0], h2[0]); // lane 0's: entry i of the column with the rotations before i applied
+    for (std::uint32_t i0 = 0; i0 < j; i0 += kColumns) {
+        const std::uint32_t in = min(kColumns, j - i0);
+        for (std::uint32_t i = tid; i < in; i += blockDim.x) {
+            scol[i] = cadd(h1[i0 + i + 1], h2[i0 + i + 1]);
+            ssn[i] = sn[i0 + i];
+            scs[i] = cs[i0 + i];
+        }
+        __syncthreads();
+        if (tid == 0)
+#pragma unroll 4
+            for (std::uint32_t i = 0; i < in; ++i) {
+                const Cx below = scol[i], s = ssn[i];
+                const double c = scs[i];
+                scol[i] = cadd(cscale(cur, c), cmul(s, below));
+                cur = cadd(cmul(cneg(cconj(s)), cur), cscale(below, c));
+            }
+        __syncthreads();
+        for (std::uint32_t i = tid; i < in; i += blockDim.x)
+            col[i0 + i] = scol[i];
+        __syncthreads();
     }
-    const Cx a = col[j], bb = col[j + 1];
+    for (std::uint32_t i = j + 2 + tid; i < L.stride; i += blockDim.x)
+        col[i] = {0.0, 0.0};
+    if (tid != 0)
+        return;
+    small[L.nrm()] = norm2;
+    const Cx a = cur, bb = {next, 0.0};
+    const bool breakdown = !(next > 0);
     const double absa = cabs(a), len = hypot(absa, cabs(bb));
     if (!(len > 0) || !isfinite(len)) {
         st[S_ERROR] = 1;
@@ -209,15 +351,17 @@ __global__ void givens_step(int *st, double *small, Layout L) {
         return;
     }
     const Cx phase = absa > 0 ? Cx{a.re / absa, a.im / absa} : Cx{1.0, 0.0};
-    cs[j] = absa / len;
-    const Cx s = cmul(phase, cconj(bb));
-    sn[j] = {s.re / len, s.im / len};
+    const double c = absa / len;
+    const Cx sp = cmul(phase, cconj(bb)), sj = {sp.re / len, sp.im / len};
+    cs[j] = c;
+    sn[j] = sj;
     col[j] = cscale(phase, len);
     col[j + 1] = {0.0, 0.0};
-    const Cx t = cadd(cscale(g[j], cs[j]), cmul(sn[j], g[j + 1]));
-    g[j + 1] = cadd(cmul(cneg(cconj(sn[j])), g[j]), cscale(g[j + 1], cs[j]));
-    g[j] = t;
-    const double resid = cabs(g[j + 1]);
+    const Cx gj = g[j], gn = g[j + 1];
+    const Cx gr = cadd(cmul(cneg(cconj(sj)), gj), cscale(gn, c));
+    g[j] = cadd(cscale(gj, c), cmul(sj, gn));
+    g[j + 1] = gr;
+    const double resid = cabs(gr);
     small[L.resid()] = resid;
     st[S_USED] = static_cast<int>(j + 1);
     st[S_J] = static_cast<int>(j + 1);
@@ -225,40 +369,75 @@ __global__ void givens_step(int *st, double *small, Layout L) {
         st[S_DONE] = 1;
 }
 
+// v_{j+1} = w / |w| (0 when |w| = 0) in place; every wavefront sums the norm's partials.
+// With a device cycle the last workgroup rotates the column instead, else |w|^2 goes
+// behind h1 and h2.
+__global__ __launch_bounds__(kFinishRows) void finish_step(ArnoldiBatch B, std::uint32_t blocks) {
+    __shared__ Cx scol[kColumns], ssn[kColumns];
+    __shared__ double scs[kColumns];
+    std::uint32_t j;
+    if (!step_index(B, j))
+        return;
+    const std::uint32_t n = B.n, ld = B.restart + 1, a = blockIdx.y, e = B.which[a], lane = threadIdx.x & 63;
+    const double *part = B.part + 4 * static_cast<std::size_t>(a) * blocks * ld;
+    double v = 0;
+    for (std::uint32_t b = lane; b < blocks; b += 64)
+        v += part[b];
+    v = wave_sum(v);
+    const std::uint32_t i = blockIdx.x * kFinishRows + threadIdx.x;
+    if (blockIdx.x * kFinishRows >= n) {
+        rotate_column(B.state, B.small, Layout{ld}, j, v, scol, ssn, scs);
+        return;
+    }
+    if (!B.state && i == 0)
+        B.small[e * B.small_stride + 4 * ld] = v;
+    if (i >= n)
+        return;
+    double2 *w = reinterpret_cast<double2 *>(B.basis + e * B.basis_stride) + static_cast<std::size_t>(j + 1) * n;
+    const double len = sqrt(v);
+    w[i] = v > 0 ? double2{w[i].x / len, w[i].y / len} : double2{0, 0};
+}
+
+template <int RK>
+void launch_passes(const ArnoldiBatch &B, const double *y, std::uint32_t chunks, hipStream_t s) {
+    const dim3 grid(pass_blocks(B.n), B.count), block(kThreads);
+    const double2 *yv = reinterpret_cast<const double2 *>(y);
+    hipLaunchKernelGGL((arnoldi_pass<RK, kGather>), grid, block, 0, s, B, yv, chunks);
+    hipLaunchKernelGGL((arnoldi_pass<RK, kFirst>), grid, block, 0, s, B, nullptr, 0u);
+    hipLaunchKernelGGL((arnoldi_pass<RK, kSecond>), grid, block, 0, s, B, nullptr, 0u);
+}
+
 } // namespace
 
 std::size_t gmres_cycle_small_doubles(std::uint32_t restart) { return Layout{restart + 1}.total(); }
-std::size_t gmres_cycle_scratch_doubles(std::uint32_t n, std::uint32_t restart) {
-    const std::size_t blocks = (n + kRows - 1) / kRows;
-    return std::max<std::size_t>(2 * blocks * (restart + 1) + 1024, 1024 + 2048);
+std::size_t arnoldi_part_doubles(std::uint32_t n, std::uint32_t restart) {
+    return 4 * static_cast<std::size_t>(pass_blocks(n)) * (restart + 1);
 }
 std::size_t gmres_cycle_h_offset(std::uint32_t restart) { return Layout{restart + 1}.H(); }
 std::size_t gmres_cycle_g_offset(std::uint32_t restart) { return Layout{restart + 1}.g(); }
 
-void gmres_cycle_begin(const GmresDeviceCycle &c, double beta, double target, std::uint32_t limit, hipStream_t s) {
+void gmres_cycle_begin(const ArnoldiBatch &c, double beta, double target, std::uint32_t limit, hipStream_t s) {
     hipLaunchKernelGGL(cycle_begin, dim3(1), dim3(256), 0, s, c.state, c.small, Layout{c.restart + 1}, beta, target,
                        limit);
 }
 
-void gmres_cycle_load(const GmresDeviceCycle &c, hipStream_t s) {
-    hipLaunchKernelGGL(load_current, dim3((2 * c.n + 255) / 256), dim3(256), 0, s, c.basis, c.n, c.state, c.current);
+void arnoldi_load(const ArnoldiBatch &B, double *in, hipStream_t s) {
+    hipLaunchKernelGGL(load_step, dim3((B.n + 255) / 256, B.count), dim3(256), 0, s, B, reinterpret_cast<double2 *>(in));
 }
 
-void gmres_cycle_orthogonalize(const GmresDeviceCycle &c, hipStream_t s) {
-    const Layout L{c.restart + 1};
-    const std::uint32_t n = c.n, blocks = (n + kRows - 1) / kRows, groups = (c.restart + 1 + 3) / 4;
-    for (const std::size_t h : {L.h1(), L.h2()}) {
-        hipLaunchKernelGGL(project_step, dim3(blocks, groups), dim3(256), 0, s, c.basis, n, c.state, c.w, c.scratch);
-        hipLaunchKernelGGL(sum_step, dim3((c.restart + 1 + 63) / 64), dim3(64), 0, s, c.scratch, blocks, c.state,
-                           c.small + h);
-        hipLaunchKernelGGL(subtract_step, dim3((n + 255) / 256), dim3(256), 0, s, c.basis, n, c.state, c.small + h, c.w);
+void arnoldi_precondition(const ArnoldiBatch &B, const double *inverses, double *in, hipStream_t s) {
+    hipLaunchKernelGGL(jacobi_step, dim3((B.n + 63) / 64, B.count), dim3(256), 0, s, B,
+                       reinterpret_cast<const double2 *>(inverses), reinterpret_cast<double2 *>(in));
+}
+
+void arnoldi_orthogonalize(const ArnoldiBatch &B, const double *y, std::uint32_t chunks, hipStream_t s) {
+    switch (rows_per_lane(B.n)) {
+    case 1: launch_passes<1>(B, y, chunks, s); break;
+    case 2: launch_passes<2>(B, y, chunks, s); break;
+    default: launch_passes<4>(B, y, chunks, s);
     }
-    const std::uint32_t nblocks = std::min<std::uint32_t>(1024, (n + 255) / 256);
-    hipLaunchKernelGGL(norm_step_partial, dim3(nblocks), dim3(256), 0, s, c.w, n, c.state, c.scratch);
-    hipLaunchKernelGGL(norm_step_finish, dim3(1), dim3(64), 0, s, c.scratch, nblocks, c.state, c.small + L.nrm());
-    hipLaunchKernelGGL(store_next, dim3((2 * n + 255) / 256), dim3(256), 0, s, c.w, n, c.state, c.small + L.nrm(),
-                       c.basis);
-    hipLaunchKernelGGL(givens_step, dim3(1), dim3(64), 0, s, c.state, c.small, L);
+    hipLaunchKernelGGL(finish_step, dim3((B.n + kFinishRows - 1) / kFinishRows + (B.state ? 1 : 0), B.count),
+                       dim3(kFinishRows), 0, s, B, pass_blocks(B.n));
 }
 
 } // namespace hsbem::dev

@@ -171,23 +171,24 @@ void launch_flux_rhs(const double *BD, std::uint32_t nv, std::uint32_t nd, const
 
 // y[:, e] = A x[:, e] for e < nvec (A n x n complex, column-major, FP64 or FP32
 // when fp32 != 0; vectors and accumulation FP64); y may not alias x.
-// skip (device int, single-vector products only): when nonzero at run time the
-// kernels return at once (a captured solver step after its loop has finished).
 void launch_gemv(const void *A, bool fp32, std::uint32_t n, const double *x, double *y, std::uint32_t nvec,
-                 double *scratch, hipStream_t stream, const int *skip = nullptr);
+                 double *scratch, hipStream_t stream);
+// The same for nvec <= 8 without the last sum: scratch[(e chunks + c) n ..] holds the
+// share of column chunk c; returns chunks. y is written only where a product of one
+// vector has its shape tuned first. skip (device int): when nonzero at run time the
+// kernels return at once (a captured solver step after its loop has finished).
+std::uint32_t launch_gemv_partials(const void *A, bool fp32, std::uint32_t n, const double *x, double *y,
+                                   std::uint32_t nvec, double *scratch, hipStream_t stream, const int *skip = nullptr);
 // Scratch doubles launch_gemv needs for n and nvec.
 std::size_t gemv_scratch_doubles(std::uint32_t n, std::uint32_t nvec);
 
-// out[j] = V[:, j]^H w for j < m (V n x m column-major); out complex m.
-void launch_project(const double *V, std::uint32_t n, std::uint32_t m, const double *w, double *out,
-                    double *scratch, hipStream_t stream);
 // w -= V h (h complex m).
 void launch_subtract_combination(const double *V, std::uint32_t n, std::uint32_t m, const double *h, double *w,
                                  hipStream_t stream);
 // out[0] = ||x||_2^2 (one complex vector of length n, weighted by mass if given).
 void launch_norm2(const double *x, std::uint32_t n, const double *weight, double *out, double *scratch,
                   hipStream_t stream);
-std::size_t reduction_scratch_doubles(std::uint32_t n, std::uint32_t m);
+inline constexpr std::size_t kNormScratchDoubles = 1024;
 
 // Complex LU with partial pivoting in place (A n x n), pivots n. info (cleared by the caller):
 // the first zero pivot's column + 1, or negative when the panel's workgroups gave up waiting
@@ -200,32 +201,40 @@ void check_lu_status(int info, const char *singular);
 void lu_solve(const double *LU, std::uint32_t n, const std::int32_t *pivots, double *B, std::uint32_t nrhs,
               hipStream_t stream);
 
+// One Arnoldi step of up to 8 systems at once. System e (the a-th of the step is
+// which[a]) has its basis at basis + e basis_stride (column c: n complex at 2 n c; column
+// j + 1 receives v_{j+1}) and at small + e small_stride h1 and h2 (restart + 1 complex
+// each) and |w|^2. part: count x arnoldi_part_doubles. j is the host's, or with `state`
+// that of the device-resident restart cycle below (one system).
+struct ArnoldiBatch {
+    double *basis, *small, *part;
+    std::size_t basis_stride, small_stride;
+    int *state;
+    std::uint32_t n, restart, j, count;
+    std::uint32_t which[8];
+};
+std::size_t arnoldi_part_doubles(std::uint32_t n, std::uint32_t restart);
+// The operator's input, in[a] = v_j, or M^{-1} v_j with the 64-wide block-Jacobi
+// inverses; with `state` one of these is the step's first launch.
+void arnoldi_load(const ArnoldiBatch &B, double *in, hipStream_t s);
+void arnoldi_precondition(const ArnoldiBatch &B, const double *inverses, double *in, hipStream_t s);
+// w_a = the sum over `chunks` of y[(a chunks + c) n ..] (chunks = 1: y is the product, and
+// may be the basis column itself for one system), CGS2 of w against v_0..v_j,
+// v_{j+1} = w / |w|; with `state` the column is rotated and j advances.
+void arnoldi_orthogonalize(const ArnoldiBatch &B, const double *y, std::uint32_t chunks, hipStream_t s);
+
 // Device-resident GMRES restart cycle (one right-hand side): the step index, the
 // Hessenberg columns, the Givens rotations, g and the stop flag live in `small` /
-// `state`, so one Arnoldi step (load, operator, orthogonalize) is a fixed launch
+// `state`, so one Arnoldi step (input, operator, orthogonalize) is a fixed launch
 // sequence a HIP graph can replay; every kernel of a step returns at once after the
-// cycle has stopped. state: [j, done, used, limit, error]; small layout: h1 at 0
-// ((restart+1) complex, reused for the cycle's y), g and H at the offsets below
-// (H column-major, stride restart+1).
-struct GmresDeviceCycle {
-    double *basis;    // (restart + 1) x n complex
-    double *current;  // n complex: v_j
-    double *w;        // n complex: the operator's output being orthogonalized
-    double *scratch;  // >= gmres_cycle_scratch_doubles(n, restart)
-    double *small;    // gmres_cycle_small_doubles(restart)
-    int *state;       // 5 ints
-    std::uint32_t n, restart;
-};
+// cycle has stopped. state: [j, done, used, limit, error, the step's j and done]; small
+// layout (gmres_cycle_small_doubles): h1 at 0 ((restart+1) complex, reused for the
+// cycle's y), g and H at the offsets below (H column-major, stride restart+1).
 std::size_t gmres_cycle_small_doubles(std::uint32_t restart);
-std::size_t gmres_cycle_scratch_doubles(std::uint32_t n, std::uint32_t restart);
 std::size_t gmres_cycle_h_offset(std::uint32_t restart);
 std::size_t gmres_cycle_g_offset(std::uint32_t restart);
 // Starts a cycle: g = (beta, 0, ...), the absolute target, at most `limit` steps.
-void gmres_cycle_begin(const GmresDeviceCycle &c, double beta, double target, std::uint32_t limit, hipStream_t s);
-// current = v_j.
-void gmres_cycle_load(const GmresDeviceCycle &c, hipStream_t s);
-// CGS2 of w against v_0..v_j, v_{j+1} = w / |w|, column j rotated, j += 1.
-void gmres_cycle_orthogonalize(const GmresDeviceCycle &c, hipStream_t s);
+void gmres_cycle_begin(const ArnoldiBatch &c, double beta, double target, std::uint32_t limit, hipStream_t s);
 
 // LU factorization and solve (as lu_factor + lu_solve) whose pivots and status
 // word live in a static device array instead of allocated memory: A (n x n,
@@ -270,8 +279,6 @@ void launch_axpy(std::uint32_t n, const double *alpha, const double *x, double *
 void launch_add(std::uint32_t n, const double *x, double *y, hipStream_t stream);
 // r = b - r (complex vectors of length n).
 void launch_subtract_from(std::uint32_t n, const double *b, double *r, hipStream_t stream);
-// y = x / sqrt(*norm2) (device-resident squared norm; zero vector when it is 0).
-void launch_normalize(std::uint32_t n, const double *norm2, const double *x, double *y, hipStream_t stream);
 void launch_scale(std::uint32_t n, double s, const double *x, double *y, hipStream_t stream);
 
 // ---- fields (field.hip) ----

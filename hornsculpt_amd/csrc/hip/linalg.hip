@@ -197,45 +197,6 @@ __global__ void gemv_reduce(const double *part, std::uint32_t n, std::uint32_t c
     y[2 * idx + 1] = im;
 }
 
-// Projection partials: workgroup (b, g) reduces rows [b*kProjectRows, ...) for the
-// columns j = 4g + wave, one wavefront per column, into part[b][j].
-constexpr int kProjectRows = 512;
-__global__ __launch_bounds__(256) void project_partial(const double *V, std::uint32_t n, std::uint32_t m,
-                                                      const double *w, double *part) {
-    constexpr int kRows = kProjectRows;
-    const std::uint32_t r0 = blockIdx.x * kRows;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x / 64;
-    const std::uint32_t j = blockIdx.y * 4 + wave;
-    if (j >= m)
-        return;
-    double re = 0, im = 0;
-    for (std::uint32_t r = r0 + lane; r < min(r0 + kRows, n); r += 64) {
-        const double vr = V[2 * (static_cast<std::size_t>(j) * n + r)], vi = V[2 * (static_cast<std::size_t>(j) * n + r) + 1];
-        const double xr = w[2 * r], xi = w[2 * r + 1];
-        re += vr * xr + vi * xi; // conj(v) * x
-        im += vr * xi - vi * xr;
-    }
-    re = wave_sum(re);
-    im = wave_sum(im);
-    if (lane == 0) {
-        part[2 * (static_cast<std::size_t>(blockIdx.x) * m + j)] = re;
-        part[2 * (static_cast<std::size_t>(blockIdx.x) * m + j) + 1] = im;
-    }
-}
-
-__global__ void sum_columns(const double *part, std::uint32_t blocks, std::uint32_t m, double *out) {
-    const std::uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= m)
-        return;
-    double re = 0, im = 0;
-    for (std::uint32_t b = 0; b < blocks; ++b) {
-        re += part[2 * (static_cast<std::size_t>(b) * m + j)];
-        im += part[2 * (static_cast<std::size_t>(b) * m + j) + 1];
-    }
-    out[2 * j] = re;
-    out[2 * j + 1] = im;
-}
-
 __global__ void subtract_combination(const double *V, std::uint32_t n, std::uint32_t m, const double *h, double *w) {
     const std::uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= n)
@@ -298,15 +259,6 @@ __global__ void subtract_from_kernel(std::uint32_t n, const double *b, double *r
     if (i >= 2 * n)
         return;
     r[i] = b[i] - r[i];
-}
-
-// y = x / sqrt(*norm2) with the squared norm read on the device (0 when the norm is 0).
-__global__ void normalize_kernel(std::uint32_t n, const double *norm2, const double *x, double *y) {
-    const std::uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= 2 * n)
-        return;
-    const double v = *norm2;
-    y[i] = v > 0 ? x[i] / sqrt(v) : 0.0;
 }
 
 __global__ void scale_kernel(std::uint32_t n, double s, const double *x, double *y) {
@@ -766,9 +718,10 @@ std::size_t gemv_scratch_doubles(std::uint32_t n, std::uint32_t nvec) {
 
 namespace {
 
+// The partial products of the column chunks; returns the number of chunks.
 template <int COLS>
-void launch_gemv_one(const void *A, bool fp32, std::uint32_t n, const double *x, double *y, double *scratch,
-                     hipStream_t stream, const int *skip, std::uint32_t rows) {
+std::uint32_t launch_gemv_one(const void *A, bool fp32, std::uint32_t n, const double *x, double *scratch,
+                              hipStream_t stream, const int *skip, std::uint32_t rows) {
     const std::uint32_t chunks = (n + COLS - 1) / COLS;
     const dim3 grid((n + kGemvRows - 1) / kGemvRows, chunks);
     if (fp32 && rows == 4 && n % 4 == 0)
@@ -785,22 +738,27 @@ void launch_gemv_one(const void *A, bool fp32, std::uint32_t n, const double *x,
     else
         hipLaunchKernelGGL((gemv_partial<1, double2, COLS>), grid, dim3(kGemvRows * kGemvWaves), 0, stream,
                            static_cast<const double2 *>(A), n, x, chunks, scratch, skip);
-    hipLaunchKernelGGL(gemv_reduce, dim3((n + 255) / 256), dim3(256), 0, stream, scratch, n, chunks, 1u, y, skip);
+    return chunks;
 }
 
 // A product shape: the column chunk (512 / 1024 / 2048, low 16 bits) and, for an FP32
 // matrix whose order they divide, the rows per lane (1, 2 or 4; bits 16 and up).
 constexpr std::uint32_t gemv_shape(std::uint32_t cols, std::uint32_t rows) { return cols | rows << 16; }
 
-void launch_gemv_cols(std::uint32_t shape, const void *A, bool fp32, std::uint32_t n, const double *x, double *y,
-                      double *scratch, hipStream_t stream, const int *skip = nullptr) {
+std::uint32_t launch_gemv_cols(std::uint32_t shape, const void *A, bool fp32, std::uint32_t n, const double *x,
+                               double *scratch, hipStream_t stream, const int *skip = nullptr) {
     const std::uint32_t cols = shape & 0xffffu, rows = std::max(shape >> 16, 1u);
     if (cols == 2048)
-        launch_gemv_one<2048>(A, fp32, n, x, y, scratch, stream, skip, rows);
-    else if (cols == 1024)
-        launch_gemv_one<1024>(A, fp32, n, x, y, scratch, stream, skip, rows);
-    else
-        launch_gemv_one<kGemvCols>(A, fp32, n, x, y, scratch, stream, skip, rows);
+        return launch_gemv_one<2048>(A, fp32, n, x, scratch, stream, skip, rows);
+    if (cols == 1024)
+        return launch_gemv_one<1024>(A, fp32, n, x, scratch, stream, skip, rows);
+    return launch_gemv_one<kGemvCols>(A, fp32, n, x, scratch, stream, skip, rows);
+}
+
+void launch_gemv_reduce(std::uint32_t n, std::uint32_t chunks, std::uint32_t nvec, const double *scratch, double *y,
+                        hipStream_t stream, const int *skip) {
+    const std::size_t count = static_cast<std::size_t>(n) * nvec;
+    hipLaunchKernelGGL(gemv_reduce, dim3((count + 255) / 256), dim3(256), 0, stream, scratch, n, chunks, nvec, y, skip);
 }
 
 // Shape of the one-vector product per (n, precision), chosen by the autotuner among
@@ -832,58 +790,51 @@ std::uint32_t gemv_columns(const void *A, bool fp32, std::uint32_t n, const doub
     const std::string key = "n=" + std::to_string(n) + (fp32 ? " fp32" : " fp64");
     return autotune::choose(
         "gemv_shape", key, shapes, kGemvCols, stream,
-        [&](std::uint32_t shape) { launch_gemv_cols(shape, A, fp32, n, x, y, scratch, stream); }, 3, pinned);
+        [&](std::uint32_t shape) {
+            launch_gemv_reduce(n, launch_gemv_cols(shape, A, fp32, n, x, scratch, stream), 1, scratch, y, stream, nullptr);
+        },
+        3, pinned);
 }
 
 } // namespace
 
-void launch_gemv(const void *A, bool fp32, std::uint32_t n, const double *x, double *y, std::uint32_t nvec,
-                 double *scratch, hipStream_t stream, const int *skip) {
-    if (nvec == 1) {
-        launch_gemv_cols(gemv_columns(A, fp32, n, x, y, scratch, stream), A, fp32, n, x, y, scratch, stream, skip);
-        return;
-    }
+std::uint32_t launch_gemv_partials(const void *A, bool fp32, std::uint32_t n, const double *x, double *y,
+                                   std::uint32_t nvec, double *scratch, hipStream_t stream, const int *skip) {
+    if (nvec == 1)
+        return launch_gemv_cols(gemv_columns(A, fp32, n, x, y, scratch, stream), A, fp32, n, x, scratch, stream, skip);
     const std::uint32_t chunks = (n + kGemvCols - 1) / kGemvCols;
-    for (std::uint32_t v0 = 0; v0 < nvec; v0 += kMaxVec) {
-        const std::uint32_t nv = std::min<std::uint32_t>(kMaxVec, nvec - v0);
-        const dim3 grid((n + kGemvRows - 1) / kGemvRows, chunks);
-        const double *xs = x + 2 * static_cast<std::size_t>(v0) * n;
-        switch (nv) {
+    const dim3 grid((n + kGemvRows - 1) / kGemvRows, chunks);
+    switch (nvec) {
 #define HS_GEMV_CASE(N)                                                                                          \
     case N:                                                                                                      \
         if (fp32)                                                                                                \
-            hipLaunchKernelGGL((gemv_partial<N, float2>), grid, dim3(kGemvRows * kGemvWaves), 0, stream,                      \
-                               static_cast<const float2 *>(A), n, xs, chunks, scratch, nullptr);                 \
+            hipLaunchKernelGGL((gemv_partial<N, float2>), grid, dim3(kGemvRows * kGemvWaves), 0, stream,         \
+                               static_cast<const float2 *>(A), n, x, chunks, scratch, skip);                     \
         else                                                                                                     \
-            hipLaunchKernelGGL((gemv_partial<N, double2>), grid, dim3(kGemvRows * kGemvWaves), 0, stream,                     \
-                               static_cast<const double2 *>(A), n, xs, chunks, scratch, nullptr);                \
+            hipLaunchKernelGGL((gemv_partial<N, double2>), grid, dim3(kGemvRows * kGemvWaves), 0, stream,        \
+                               static_cast<const double2 *>(A), n, x, chunks, scratch, skip);                    \
         break;
-            HS_GEMV_CASE(1)
-            HS_GEMV_CASE(2)
-            HS_GEMV_CASE(3)
-            HS_GEMV_CASE(4)
-            HS_GEMV_CASE(5)
-            HS_GEMV_CASE(6)
-            HS_GEMV_CASE(7)
-            HS_GEMV_CASE(8)
+        HS_GEMV_CASE(2)
+        HS_GEMV_CASE(3)
+        HS_GEMV_CASE(4)
+        HS_GEMV_CASE(5)
+        HS_GEMV_CASE(6)
+        HS_GEMV_CASE(7)
+        HS_GEMV_CASE(8)
 #undef HS_GEMV_CASE
-        }
-        const std::size_t count = static_cast<std::size_t>(n) * nv;
-        hipLaunchKernelGGL(gemv_reduce, dim3((count + 255) / 256), dim3(256), 0, stream, scratch, n, chunks, nv,
-                           y + 2 * static_cast<std::size_t>(v0) * n, nullptr);
+    default: throw std::invalid_argument("a matrix product takes 1 to 8 vectors at a time");
     }
+    return chunks;
 }
 
-std::size_t reduction_scratch_doubles(std::uint32_t n, std::uint32_t m) {
-    const std::size_t blocks = (n + kProjectRows - 1) / kProjectRows;
-    return 2 * blocks * std::max<std::uint32_t>(m, 1) + 1024;
-}
-
-void launch_project(const double *V, std::uint32_t n, std::uint32_t m, const double *w, double *out, double *scratch,
-                    hipStream_t stream) {
-    const std::uint32_t blocks = (n + kProjectRows - 1) / kProjectRows;
-    hipLaunchKernelGGL(project_partial, dim3(blocks, (m + 3) / 4), dim3(256), 0, stream, V, n, m, w, scratch);
-    hipLaunchKernelGGL(sum_columns, dim3((m + 63) / 64), dim3(64), 0, stream, scratch, blocks, m, out);
+void launch_gemv(const void *A, bool fp32, std::uint32_t n, const double *x, double *y, std::uint32_t nvec,
+                 double *scratch, hipStream_t stream) {
+    for (std::uint32_t v0 = 0; v0 < nvec; v0 += kMaxVec) {
+        const std::uint32_t nv = nvec == 1 ? 1 : std::min<std::uint32_t>(kMaxVec, nvec - v0);
+        const std::size_t at = 2 * static_cast<std::size_t>(v0) * n;
+        const std::uint32_t chunks = launch_gemv_partials(A, fp32, n, x + at, y + at, nv, scratch, stream);
+        launch_gemv_reduce(n, chunks, nv, scratch, y + at, stream, nullptr);
+    }
 }
 
 void launch_subtract_combination(const double *V, std::uint32_t n, std::uint32_t m, const double *h, double *w,
@@ -908,10 +859,6 @@ void launch_subtract_from(std::uint32_t n, const double *b, double *r, hipStream
 
 void launch_axpy(std::uint32_t n, const double *alpha, const double *x, double *y, hipStream_t stream) {
     hipLaunchKernelGGL(axpy_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, n, alpha, x, y);
-}
-
-void launch_normalize(std::uint32_t n, const double *norm2, const double *x, double *y, hipStream_t stream) {
-    hipLaunchKernelGGL(normalize_kernel, dim3((2 * n + 255) / 256), dim3(256), 0, stream, n, norm2, x, y);
 }
 
 void launch_scale(std::uint32_t n, double s, const double *x, double *y, hipStream_t stream) {

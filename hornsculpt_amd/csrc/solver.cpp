@@ -799,7 +799,6 @@ void GmresWorkspace::release() {
         (void)hipGraphExecDestroy(step_graph);
     step_graph = nullptr;
     step_key = {};
-    cycle_current.release();
     cycle_w.release();
     cycle_z.release();
     cycle_small.release();
@@ -860,12 +859,11 @@ void dense_gmres_graph(hipStream_t s, const void *A, bool fp32, std::uint32_t n,
         ws.basis.resize(vec * stride);
     if (ws.r.size() < vec)
         ws.r.resize(vec);
-    for (auto *buf : {&ws.cycle_current, &ws.cycle_w, &ws.cycle_z})
+    for (auto *buf : {&ws.cycle_w, &ws.cycle_z})
         if (buf->size() < vec)
             buf->resize(vec);
-    const std::size_t scratch =
-        std::max({dev::gemv_scratch_doubles(n, 1), dev::gmres_cycle_scratch_doubles(n, restart),
-                  dev::reduction_scratch_doubles(n, 1)});
+    const std::size_t products = std::max(dev::gemv_scratch_doubles(n, 1), dev::kNormScratchDoubles);
+    const std::size_t scratch = products + dev::arnoldi_part_doubles(n, restart);
     if (ws.scratch.size() < scratch)
         ws.scratch.resize(scratch);
     if (ws.cycle_small.size() < dev::gmres_cycle_small_doubles(restart))
@@ -888,8 +886,14 @@ void dense_gmres_graph(hipStream_t s, const void *A, bool fp32, std::uint32_t n,
         hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "event create");
         ws.cycle_events.push_back(e);
     }
-    const dev::GmresDeviceCycle cyc{ws.basis.data(), ws.cycle_current.data(), ws.cycle_w.data(), ws.scratch.data(),
-                                    ws.cycle_small.data(), ws.cycle_state.data(), n, restart};
+    dev::ArnoldiBatch cyc{};
+    cyc.basis = ws.basis.data();
+    cyc.small = ws.cycle_small.data();
+    cyc.part = ws.scratch.data() + products;
+    cyc.state = ws.cycle_state.data();
+    cyc.n = n;
+    cyc.restart = restart;
+    cyc.count = 1;
     double *nrm = ws.small.data();
     auto norm = [&](const double *v) {
         dev::launch_norm2(v, n, nullptr, nrm, ws.scratch.data(), s);
@@ -911,14 +915,19 @@ void dense_gmres_graph(hipStream_t s, const void *A, bool fp32, std::uint32_t n,
         hip_check(hipStreamSynchronize(s), "product warm-up");
         hipGraph_t graph = nullptr;
         hip_check(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "capture begin");
-        dev::gmres_cycle_load(cyc, s);
-        const double *in = ws.cycle_current.data();
-        if (jacobi) {
-            apply_block_jacobi(jacobi, n, in, ws.cycle_z.data(), s);
-            in = ws.cycle_z.data();
+        const double *in = ws.cycle_z.data();
+        if (jacobi && jacobi.width == 64) {
+            dev::arnoldi_precondition(cyc, jacobi.inverses, ws.cycle_z.data(), s);
+        } else {
+            dev::arnoldi_load(cyc, ws.cycle_z.data(), s);
+            if (jacobi) {
+                apply_block_jacobi(jacobi, n, ws.cycle_z.data(), ws.cycle_w.data(), s);
+                in = ws.cycle_w.data();
+            }
         }
-        dev::launch_gemv(A, fp32, n, in, ws.cycle_w.data(), 1, ws.scratch.data(), s, ws.cycle_state.data() + 1);
-        dev::gmres_cycle_orthogonalize(cyc, s);
+        const std::uint32_t chunks = dev::launch_gemv_partials(A, fp32, n, in, ws.r.data(), 1, ws.scratch.data(), s,
+                                                               ws.cycle_state.data() + 1);
+        dev::arnoldi_orthogonalize(cyc, ws.scratch.data(), chunks, s);
         const hipError_t captured = hipStreamEndCapture(s, &graph);
         hip_check(captured, "capture end");
         const hipError_t made = hipGraphInstantiate(&ws.step_graph, graph, nullptr, nullptr, 0);
@@ -1088,7 +1097,8 @@ void dense_gmres_multi(hipStream_t s, const void *A, bool fp32, std::uint32_t n,
         ws.multi_out.resize(nrhs * vec);
     if (ws.multi_small.size() < nrhs * slot)
         ws.multi_small.resize(nrhs * slot);
-    const std::size_t scratch = std::max(dev::gemv_scratch_doubles(n, nrhs), dev::reduction_scratch_doubles(n, stride));
+    const std::size_t products = std::max(dev::gemv_scratch_doubles(n, nrhs), dev::kNormScratchDoubles);
+    const std::size_t scratch = products + nrhs * dev::arnoldi_part_doubles(n, restart);
     if (ws.scratch.size() < scratch)
         ws.scratch.resize(scratch);
     if (ws.multi_pinned_doubles < nrhs * slot) {
@@ -1103,8 +1113,6 @@ void dense_gmres_multi(hipStream_t s, const void *A, bool fp32, std::uint32_t n,
            *out = ws.multi_out.data(), *small0 = ws.multi_small.data(), *pinned = ws.multi_pinned;
     auto basis = [&](std::uint32_t e, std::uint32_t j) { return basis0 + (e * stride + j) * vec; };
     auto h1 = [&](std::uint32_t e) { return small0 + e * slot; };
-    auto h2 = [&](std::uint32_t e) { return small0 + e * slot + 2 * stride; };
-    auto nrm = [&](std::uint32_t e) { return small0 + e * slot + 4 * stride; };
     auto cell = [&](std::uint32_t e) { return small0 + e * slot + column; };
     auto xe = [&](std::uint32_t e) { return x + e * vec; };
     auto re = [&](std::uint32_t e) { return out + e * vec; }; // residuals live in the output pack between cycles
@@ -1173,25 +1181,26 @@ void dense_gmres_multi(hipStream_t s, const void *A, bool fp32, std::uint32_t n,
                 throw Cancelled();
             }
             const auto c = static_cast<std::uint32_t>(active.size());
-            for (std::uint32_t a = 0; a < c; ++a) { // pack M^{-1} v_j of the active systems
-                if (jacobi)
+            dev::ArnoldiBatch step{};
+            step.basis = basis0;
+            step.basis_stride = stride * vec;
+            step.small = small0;
+            step.small_stride = slot;
+            step.part = sc + products;
+            step.n = n;
+            step.restart = restart;
+            step.j = j;
+            step.count = c;
+            std::copy(active.begin(), active.end(), step.which);
+            if (jacobi && jacobi.width == 64) // in: M^{-1} v_j of the active systems
+                dev::arnoldi_precondition(step, jacobi.inverses, in, s);
+            else if (jacobi)
+                for (std::uint32_t a = 0; a < c; ++a)
                     apply_block_jacobi(jacobi, n, basis(active[a], j), in + a * vec, s);
-                else
-                    hip_check(hipMemcpyAsync(in + a * vec, basis(active[a], j), sizeof(double) * vec,
-                                             hipMemcpyDeviceToDevice, s), "pack");
-            }
-            dev::launch_gemv(A, fp32, n, in, out, c, sc, s);
-            for (std::uint32_t a = 0; a < c; ++a) {
-                const std::uint32_t e = active[a];
-                double *w = basis(e, j + 1);
-                hip_check(hipMemcpyAsync(w, out + a * vec, sizeof(double) * vec, hipMemcpyDeviceToDevice, s), "unpack");
-                dev::launch_project(basis(e, 0), n, j + 1, w, h1(e), sc, s);
-                dev::launch_subtract_combination(basis(e, 0), n, j + 1, h1(e), w, s);
-                dev::launch_project(basis(e, 0), n, j + 1, w, h2(e), sc, s);
-                dev::launch_subtract_combination(basis(e, 0), n, j + 1, h2(e), w, s);
-                dev::launch_norm2(w, n, nullptr, nrm(e), sc, s);
-                dev::launch_normalize(n, nrm(e), w, w, s);
-            }
+            else
+                dev::arnoldi_load(step, in, s);
+            const std::uint32_t chunks = dev::launch_gemv_partials(A, fp32, n, in, out, c, sc, s);
+            dev::arnoldi_orthogonalize(step, sc, chunks, s);
             hip_check(hipMemcpyAsync(pinned, small0, sizeof(double) * nrhs * slot, hipMemcpyDeviceToHost, s),
                       "arnoldi download");
             hip_check(hipStreamSynchronize(s), "arnoldi sync");
@@ -1272,7 +1281,8 @@ void gmres(hipStream_t s, const KrylovOperator &op, std::uint32_t n, const doubl
         r_.resize(2 * static_cast<std::size_t>(n));
     if (jacobi && ws.z.size() < 2 * static_cast<std::size_t>(n))
         ws.z.resize(2 * static_cast<std::size_t>(n));
-    const std::size_t scratch = std::max(dev::gemv_scratch_doubles(n, 1), dev::reduction_scratch_doubles(n, restart + 1));
+    const std::size_t scratch = // shared: a step's partial sums do not outlive it
+        std::max({dev::gemv_scratch_doubles(n, 1), dev::kNormScratchDoubles, dev::arnoldi_part_doubles(n, restart)});
     if (scratch_.size() < scratch)
         scratch_.resize(scratch);
     const std::size_t column = 4 * (restart + 1) + 1; // h1, h2 (complex, restart + 1 each) and |w|^2
@@ -1292,7 +1302,7 @@ void gmres(hipStream_t s, const KrylovOperator &op, std::uint32_t n, const doubl
         ws.events.push_back(e);
     }
     auto &small = ws.small;
-    double *h1 = small.data(), *h2 = small.data() + 2 * (restart + 1), *nrm = small.data() + 4 * (restart + 1);
+    double *h1 = small.data(), *nrm = small.data() + 4 * (restart + 1);
     auto norm = [&](const double *v) {
         dev::launch_norm2(v, n, nullptr, nrm, scratch_.data(), s);
         double out = 0;
@@ -1324,12 +1334,15 @@ void gmres(hipStream_t s, const KrylovOperator &op, std::uint32_t n, const doubl
             vj = ws.z.data();
         }
         op.apply(vj, w, s);
-        dev::launch_project(basis_.data(), n, j + 1, w, h1, scratch_.data(), s);
-        dev::launch_subtract_combination(basis_.data(), n, j + 1, h1, w, s);
-        dev::launch_project(basis_.data(), n, j + 1, w, h2, scratch_.data(), s);
-        dev::launch_subtract_combination(basis_.data(), n, j + 1, h2, w, s);
-        dev::launch_norm2(w, n, nullptr, nrm, scratch_.data(), s);
-        dev::launch_normalize(n, nrm, w, w, s);
+        dev::ArnoldiBatch step{};
+        step.basis = basis_.data();
+        step.small = small.data();
+        step.part = scratch_.data();
+        step.n = n;
+        step.restart = restart;
+        step.j = j;
+        step.count = 1;
+        dev::arnoldi_orthogonalize(step, w, 1, s);
         hip_check(hipMemcpyAsync(ws.pinned + column * j, small.data(), sizeof(double) * column, hipMemcpyDeviceToHost, s),
                   "arnoldi download");
         hip_check(hipEventRecord(ws.events[j], s), "arnoldi event");
@@ -1511,7 +1524,7 @@ std::shared_ptr<PreparedRequest> MeshSolver::prepare(const Request &req) const {
     const std::uint64_t nobs = P->observers.size();
     const bool fmm = num.acceleration == 1;
     const std::uint64_t scratch = std::max({dev::gemv_scratch_doubles(nv, std::min<std::uint32_t>(ne, 8)),
-                                            dev::reduction_scratch_doubles(nv, num.gmres_restart + 1), std::size_t{4096},
+                                            std::size_t{4096},
                                             lu && !fmm ? dev::kLuWorkDoubles : 0});
     std::uint64_t bytes = (fmm ? 0 : (mixed ? 8 : 16) * nv2) + 16 * nv * nd1 + 16 * nd1 * ne + 3 * 16ull * nv * ne +
                           16ull * nt * ne + 8 * scratch + 4ull * nt;
@@ -1522,7 +1535,7 @@ std::shared_ptr<PreparedRequest> MeshSolver::prepare(const Request &req) const {
         // per node on a 10k-node horn, 203 KB on a 59k-node flanged horn at 16 kHz)
         const std::uint64_t measured = const_cast<MeshSolver *>(this)->fmm_point_bytes(num);
         bytes += measured ? measured + measured / 10 : 16ull * nv * 12288 + (64ull << 20);
-        bytes += 16ull * nv * (num.fmm_restart + 2) + 16ull * nv + 8ull * (4 * (num.fmm_restart + 2) + 8) +
+        bytes += 8 * dev::arnoldi_part_doubles(nv, num.fmm_restart) + 16ull * nv * (num.fmm_restart + 2) + 16ull * nv + 8ull * (4 * (num.fmm_restart + 2) + 8) +
                  8 * (num.fmm_block_width == 64 ? dev::jacobi_factor_doubles(nv)
                                                 : 2 * dev::jacobi_wide_doubles(nv, num.fmm_block_width));
     }
@@ -1530,6 +1543,7 @@ std::shared_ptr<PreparedRequest> MeshSolver::prepare(const Request &req) const {
         bytes += 16 * nv2 + 4ull * nv;
     else
         bytes += 16ull * nv * (num.gmres_restart + 2) + 16ull * nv + 8 * scratch + 8ull * (4 * (num.gmres_restart + 2) + 8) +
+                 8 * std::min<std::uint32_t>(ne, kGmresBatch) * dev::arnoldi_part_doubles(nv, num.gmres_restart) +
                  (ne > 1 ? 16ull * nv * std::min<std::uint32_t>(ne, kGmresBatch) * (num.gmres_restart + 3) +
                                8ull * std::min<std::uint32_t>(ne, kGmresBatch) * (4 * (num.gmres_restart + 2) + 16) +
                                8 * dev::gemv_scratch_doubles(nv, std::min<std::uint32_t>(ne, kGmresBatch))
@@ -1568,7 +1582,7 @@ void MeshSolver::bind(const PreparedRequest &P, Workspace &ws) {
     ws.flux_column.upload(P.flux_column, ws.stream);
     const bool lu = !fmm && !mixed && num.solver == 0;
     const std::size_t scratch = std::max({dev::gemv_scratch_doubles(nv, std::min<std::uint32_t>(ne, 8)),
-                                          dev::reduction_scratch_doubles(nv, num.gmres_restart + 1), std::size_t{4096},
+                                          std::size_t{4096},
                                           lu ? dev::kLuWorkDoubles : 0});
     ws.scratch.resize(scratch);
     if (lu) {

@@ -168,9 +168,9 @@ struct GmresWorkspace {
     DeviceBuffer<double> multi_basis, multi_in, multi_out, multi_small;
     double *multi_pinned{};
     std::size_t multi_pinned_doubles{};
-    // device-resident cycles (dense_gmres): v_j and the operator output, the cycle
+    // device-resident cycles (dense_gmres): the operator input (two for a wide block-Jacobi), the cycle
     // state, the captured Arnoldi step and what it was captured for, pinned state reads
-    DeviceBuffer<double> cycle_current, cycle_w, cycle_z, cycle_small;
+    DeviceBuffer<double> cycle_w, cycle_z, cycle_small;
     DeviceBuffer<int> cycle_state;
     hipGraphExec_t step_graph{};
     std::tuple<const void *, bool, std::uint32_t, std::uint32_t, const double *, std::uint32_t, const double *,
