@@ -7,9 +7,11 @@
 // norm and v_{j+1} = w / |w| are therefore four launches: each reduction's partials are
 // summed by every workgroup of the launch that needs them (`blocks` x (j + 1) values out of
 // L2) instead of by a launch of their own, and each workgroup keeps its rows of w in LDS
-// from the subtraction to the next projection. As ten launches (two projections, two sums,
-// two subtractions, two norm launches, scaling, rotation) an iteration at n = 523 took
-// @OLD523 us with its product, and takes @NEW523 us now; at n = 10,373, @OLD10K us and @NEW10K us.
+// from the subtraction to the next projection. Against ten launches a step (two
+// projections, two sums, two subtractions, two norm launches, scaling, rotation), whole
+// solves with the rest unchanged: mixed form on a horn of edge 20 mm (4 frequencies, about
+// 37 steps each) 16.0 -> 12.9 ms; four systems at once on the horn of edge 8 mm
+// 45.2 -> 35.8 ms; one system on that of 5.2 mm (10,373 unknowns, 86 steps) 77.4 -> 74.0 ms.
 //
 // Restart cycle. The Arnoldi step index j, the Hessenberg column, the Givens rotations, the
 // rotated right-hand side g and the stop decision live in device memory, so one
