@@ -389,19 +389,14 @@ std::unique_ptr<FmmOperator> MeshSolver::build_fmm(const Numerics &n, double k_m
 
     // ---- translation links
     t0 = Clock::now();
-    // one rotation plan per (direction, order class): a launch's kernels are chosen by
-    // its largest order (<= 32, <= 40, <= 48, <= 64, <= 128), so narrower levels never
-    // share a plan with a wider one
+    // one rotation plan per (direction, order class: <= 32, <= 40, <= 48, <= 64, <= 128), so
+    // that narrower levels never share a wider one's tables
     std::map<std::pair<Triple, int>, std::uint32_t> direction_index;
     std::vector<Triple> directions;
     std::vector<int> direction_order;
     auto direction = [&](Triple t, int ord) {
         t = reduced(t);
-        const int order_class = ord > dev::kMaxWideOrder    ? 4
-                                : ord > dev::kMidFmmOrder   ? 3
-                                : ord > dev::kMaxFmmOrder   ? 2
-                                : ord > dev::kSmallFmmOrder ? 1
-                                                            : 0;
+        const int order_class = ord > 64 ? 4 : ord > dev::kMidFmmOrder ? 3 : ord > 40 ? 2 : ord > 32 ? 1 : 0;
         auto [it, fresh] = direction_index.emplace(std::make_pair(t, order_class),
                                                    static_cast<std::uint32_t>(directions.size()));
         if (fresh) {
@@ -443,8 +438,8 @@ std::unique_ptr<FmmOperator> MeshSolver::build_fmm(const Numerics &n, double k_m
     // indices; each gets a workspace slot for the larger of its two orders.
     std::vector<dev::FmmDestination> destinations;
     std::vector<dev::FmmLink> links;
-    std::vector<std::uint32_t> link_order, axial_order;
-    std::vector<dev::FmmChunk> chunks, axial_chunks;
+    std::vector<std::uint32_t> link_order;
+    std::vector<dev::FmmChunk> chunks;
     std::uint32_t launch_link_base = 0;
     std::uint64_t slot = 0, workspace = 0;
     auto begin_destination = [&](std::uint64_t target, int ord) {
@@ -459,38 +454,36 @@ std::unique_ptr<FmmOperator> MeshSolver::build_fmm(const Numerics &n, double k_m
         slot += static_cast<std::uint64_t>(big + 1) * (big + 1);
         ++destinations.back().link_count;
     };
-    // Chunks of at most kFmmChunk launch links sharing key(link), in key order;
-    // chunk.first indexes the launch's own slice of the order array.
-    auto make_chunks = [&](std::uint32_t count, auto key, std::vector<std::uint32_t> &order_out,
-                           std::vector<dev::FmmChunk> &chunks_out) {
+    // Chunks of at most kFmmChunk launch links sharing a rotation and a coaxial plan (so
+    // also both orders); chunk.first indexes the launch's own slice of the order array.
+    auto make_chunks = [&](std::uint32_t count) {
         std::vector<std::uint32_t> idx(count);
         std::iota(idx.begin(), idx.end(), 0u);
-        std::stable_sort(idx.begin(), idx.end(), [&](std::uint32_t a, std::uint32_t b) {
-            return key(links[launch_link_base + a]) < key(links[launch_link_base + b]);
-        });
-        for (std::uint32_t i = 0; i < idx.size();) {
-            const std::uint32_t kv = key(links[launch_link_base + idx[i]]);
-            dev::FmmChunk ch{kv, i, 0, 0};
-            while (i < idx.size() && ch.count < static_cast<std::uint32_t>(dev::kFmmChunk) &&
-                   key(links[launch_link_base + idx[i]]) == kv) {
+        auto key = [&](std::uint32_t i) {
+            const dev::FmmLink &lk = links[launch_link_base + i];
+            return static_cast<std::uint64_t>(lk.rotation) << 32 | lk.axial;
+        };
+        std::stable_sort(idx.begin(), idx.end(), [&](std::uint32_t a, std::uint32_t b) { return key(a) < key(b); });
+        std::uint64_t base = 0;
+        for (std::uint32_t i = 0; i < count;) {
+            dev::FmmChunk ch{links[launch_link_base + idx[i]].rotation, i, 0, 0, base};
+            while (i < count && ch.count < static_cast<std::uint32_t>(dev::kFmmChunk) && key(idx[i]) == key(idx[ch.first])) {
                 const auto &lk = links[launch_link_base + idx[i]];
-                ch.max_order = std::max({ch.max_order, lk.source_order, lk.target_order});
+                const std::uint64_t big = std::max(lk.source_order, lk.target_order);
+                base += (big + 1) * (big + 1);
                 ++ch.count;
                 ++i;
             }
-            chunks_out.push_back(ch);
+            chunks.push_back(ch);
         }
-        order_out.insert(order_out.end(), idx.begin(), idx.end());
+        link_order.insert(link_order.end(), idx.begin(), idx.end());
     };
     auto end_launch = [&](std::uint32_t first) {
         FmmOperator::Launch L{first, static_cast<std::uint32_t>(destinations.size()) - first, launch_link_base,
                               static_cast<std::uint32_t>(links.size()) - launch_link_base,
-                              static_cast<std::uint32_t>(chunks.size()), 0,
-                              static_cast<std::uint32_t>(axial_chunks.size()), 0};
-        make_chunks(L.link_count, [](const dev::FmmLink &lk) { return lk.rotation; }, link_order, chunks);
-        make_chunks(L.link_count, [](const dev::FmmLink &lk) { return lk.axial; }, axial_order, axial_chunks);
+                              static_cast<std::uint32_t>(chunks.size()), 0, 0};
+        make_chunks(L.link_count);
         L.chunk_count = static_cast<std::uint32_t>(chunks.size()) - L.first_chunk;
-        L.axial_chunk_count = static_cast<std::uint32_t>(axial_chunks.size()) - L.first_axial_chunk;
         workspace = std::max(workspace, slot);
         slot = 0;
         launch_link_base = static_cast<std::uint32_t>(links.size());
@@ -686,12 +679,12 @@ std::unique_ptr<FmmOperator> MeshSolver::build_fmm(const Numerics &n, double k_m
         }
     }
 
-    // the kernels of a launch are chosen by the largest order it touches: its links'
-    // orders and the orders of the (level-shared) rotation plans it applies
+    // the largest order a launch touches: its links' orders and the orders of the
+    // (level-shared) rotation plans it applies
     for (FmmOperator::Launch &L : op->translate_)
-        for (std::uint32_t c = L.first_chunk; c < L.first_chunk + L.chunk_count; ++c)
-            L.max_order = std::max({L.max_order, chunks[c].max_order,
-                                    static_cast<std::uint32_t>(direction_order[chunks[c].rotation])});
+        for (std::uint32_t i = L.first_link; i < L.first_link + L.link_count; ++i)
+            L.max_order = std::max({L.max_order, links[i].source_order, links[i].target_order,
+                                    static_cast<std::uint32_t>(direction_order[links[i].rotation])});
 
     // ---- rotation and coaxial plans (host, in parallel)
     const TranslationPlanCacheStatistics cache_before = translation_plans_.statistics();
@@ -811,8 +804,6 @@ std::unique_ptr<FmmOperator> MeshSolver::build_fmm(const Numerics &n, double k_m
     upload_nonempty(op->links_, links, s);
     upload_nonempty(op->chunks_, chunks, s);
     upload_nonempty(op->link_order_, link_order, s);
-    upload_nonempty(op->axial_chunks_, axial_chunks, s);
-    upload_nonempty(op->axial_order_, axial_order, s);
     op->work_y_.resize(2 * std::max<std::uint64_t>(workspace, 1));
     op->work_z_.resize(2 * std::max<std::uint64_t>(workspace, 1));
     upload_nonempty(op->rotations_, rot_table, s);
@@ -1030,9 +1021,7 @@ void FmmOperator::apply_in(const double *x, double *y, hipStream_t s, bool fp32)
             T.links = links_.data() + L.first_link;
             T.order = link_order_.data() + L.first_link;
             T.chunks = chunks_.data() + L.first_chunk;
-            T.axial_order = axial_order_.data() + L.first_link;
-            T.axial_chunks = axial_chunks_.data() + L.first_axial_chunk;
-            dev::launch_translate(T, L.destination_count, L.link_count, L.chunk_count, L.axial_chunk_count, L.max_order,
+            dev::launch_translate(T, L.destination_count, L.link_count, L.chunk_count, L.max_order,
                                   split_target_, s);
         } else if (stage.kind == StageKind::angular) {
             const HfLaunch &A = angular_[stage.index];

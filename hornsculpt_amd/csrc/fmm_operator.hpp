@@ -108,7 +108,7 @@ class FmmOperator {
     friend class MeshSolver;
     struct Launch {
         std::uint32_t first_destination{}, destination_count{}, first_link{}, link_count{}, first_chunk{},
-            chunk_count{}, first_axial_chunk{}, axial_chunk_count{}, max_order{};
+            chunk_count{}, max_order{};
     };
     std::uint32_t n_{};
     FmmStatistics stats_;
@@ -120,8 +120,7 @@ class FmmOperator {
     DeviceBuffer<dev::FmmDestination> destinations_;
     DeviceBuffer<dev::FmmLink> links_;
     DeviceBuffer<dev::FmmChunk> chunks_;
-    DeviceBuffer<std::uint32_t> link_order_, axial_order_;
-    DeviceBuffer<dev::FmmChunk> axial_chunks_;
+    DeviceBuffer<std::uint32_t> link_order_;
     mutable DeviceBuffer<double> work_y_, work_z_;
     DeviceBuffer<dev::FmmRotation> rotations_;
     DeviceBuffer<double> small_d_, azimuth_, axial_;

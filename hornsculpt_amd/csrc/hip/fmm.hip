@@ -300,20 +300,8 @@ __device__ __forceinline__ void split_index(int e, int &l, int &t) {
 
 // Offset of the |m| block of a coaxial plan: sum_{j<m} (pt+1-j)(ps+1-j).
 __device__ __forceinline__ std::size_t axial_block(int m, int ps, int pt) {
-    std::size_t off = 0;
-    for (int j = 0; j < m; ++j)
-        off += static_cast<std::size_t>(pt + 1 - j) * (ps + 1 - j);
-    return off;
-}
-
-// Position of coefficient (l, m) of an order-p expansion in |m|-major order: blocks
-// |m| = 0..p, each holding l = |m|..p for +|m| and then (|m| > 0) for -|m|; block |m|
-// starts at (2|m|-1)(p+1) - (|m|-1)|m| (0 for |m| = 0). The forward rotation writes
-// the rotated source in this order so the coaxial products read contiguous columns.
-__device__ __forceinline__ std::size_t m_major(int p, int l, int m) {
-    const int a = m < 0 ? -m : m;
-    const std::size_t block = a ? static_cast<std::size_t>(2 * a - 1) * (p + 1) - static_cast<std::size_t>(a - 1) * a : 0;
-    return block + (m < 0 ? p - a + 1 : 0) + (l - a);
+    const std::size_t j = m, a = pt + 1, b = ps + 1, first = j ? j * (j - 1) / 2 : 0; // sum of the j below m
+    return j * a * b - (a + b) * first + (j ? first * (2 * j - 1) / 3 : 0);
 }
 
 // Offset of degree l in a rotation's small-d table: sum_{j<l} (2j+1)^2 = l(2l-1)(2l+1)/3.
@@ -322,667 +310,279 @@ __device__ __forceinline__ std::size_t degree_block(int l) {
 }
 
 // Translations run as four passes over the links of one level:
-//   rotate    per chunk of links sharing a direction: the Wigner blocks d_l are
-//             staged in LDS degree by degree and applied to every source of the
-//             chunk (Y = d^T e^{i m phi} X, stored |m|-major);
-//   coaxial   one wavefront per link: per-|m| block product Z = T Y;
-//   back      per chunk again: W = e^{-i m phi} d Z;
+//   rotate    per chunk of links sharing a direction and a coaxial plan: the Wigner blocks
+//             d_l applied to every source of the chunk (Y = d^T e^{i m phi} X);
+//   coaxial   per-|m| block product Z = T Y;
+//   back      W = e^{-i m phi} d Z;
 //   gather    one block per destination: the sum of its links' W.
-// Y and W share one workspace slot per link, Z uses a second.
-// Two degrees per stage, l and top - l: their Wigner blocks d_l and the chunk's
-// slices of both degrees are staged in LDS together, so every stage carries about
-// the same work ((2l+1)^2 + (2(top-l)+1)^2 multiply-adds per link) and the number of
-// barrier pairs halves; the next stage's values are loaded into registers while the
-// current one is computed. Workgroup (chunk, y) takes the stages h = y, y + Y, ... of
-// its chunk (Y = gridDim.y): the degrees are independent, so a level with few chunks
-// spreads its stages over more workgroups instead of running them one after another.
-// Instantiated for orders up to kP = 32, 40 and 48 (LDS and registers sized to kP, so
-// the common orders 24-32 keep three workgroups per CU).
-template <int kP, class E>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kP <= 32 ? 3 : 1))) void rotate_links(FmmTranslateLaunch L, bool back) {
-    using CE = Cx<E>;
-    constexpr int kStage = (2 * kP + 1) * (2 * kP + 1) + 1; // >= n_a^2 + n_b^2 for n_a + n_b <= 2 kP + 2
-    constexpr int kStagePerThread = (kStage + 255) / 256;
-    constexpr int kSliceWidth = 2 * kP + 2;                 // >= n_a + n_b
-    constexpr int kSlicePerThread = (kFmmChunk * kSliceWidth + 255) / 256;
-    __shared__ E dl[kStage];
-    __shared__ CE xs[kFmmChunk][kSliceWidth]; // rows >= count: stale, their results are dropped
-    __shared__ CE ph[2 * kP + 1];
-    __shared__ std::uint64_t src_off[kFmmChunk], dst_off[kFmmChunk];
-    __shared__ int ord[kFmmChunk];
-    const FmmChunk ch = L.chunks[blockIdx.x];
-    const int split = static_cast<int>(blockIdx.y), splits = static_cast<int>(gridDim.y);
-    if (split > static_cast<int>(ch.max_order) / 2)
-        return; // this chunk has fewer stages than the launch has splits
-    const FmmRotation rot = L.rotations[ch.rotation];
-    const C2 *az = reinterpret_cast<const C2 *>(L.azimuth) + rot.azimuth;
-    for (int m = threadIdx.x; m <= 2 * static_cast<int>(rot.order); m += blockDim.x)
-        ph[m] = to_cx<E>(az[m]);
-    if (threadIdx.x < ch.count) {
-        const FmmLink lk = L.links[L.order[ch.first + threadIdx.x]];
-        src_off[threadIdx.x] = back ? lk.slot : lk.source;
-        dst_off[threadIdx.x] = lk.slot;
-        ord[threadIdx.x] = static_cast<int>(back ? lk.target_order : lk.source_order);
+// Y and Z hold a chunk's links interleaved (coefficient (l, m) of link j at
+// base + (l^2 + l + m) count + j), W each link's expansion in its slot.
+//
+// Rotations and coaxial products are small matrix products (a block of 2l + 1 or
+// p + 1 - |m| rows against up to 16 links), on the matrix cores in 16 x 16 x 4 steps with
+// the operands loaded straight from memory into lanes: a block is read once per chunk by one
+// wavefront and a link's values once per wavefront, so nothing is staged, no barrier
+// holds wavefronts together and their number per CU hides the latency. (With the blocks and
+// slices staged in LDS and FP64 vector products, the products were bound by LDS reads: 12
+// reads of 16 bytes for 24 multiply-adds.) Each wavefront takes whole degrees l (orders |m|);
+// each step
+// reads and writes rows of 16 count bytes, so that no pass touches part of a line in one
+// order and the rest in another.
+// One level of a 20.7k-triangle horn (41k links of order 26, FP64), forward, coaxial, back:
+// 620 + 657 + 551 us before, 275 + 377 + 405 us now (Y, Z and W are 480 MB each: 2.2 to 3.6
+// TB/s); the whole operator 3.96 -> 2.72 ms. What gave how much: tiles alone about nothing (the
+// |m|-major Y and strided Z wrote 2 to 2.4 times their bytes in parts of lines), the
+// interleaved layout and dies that share a direction 4.5 -> 3.5 ms, four wavefronts per SIMD
+// and d by rows 3.0 ms, 16-byte stores 2.7 ms.
+template <class E> struct Tile16;
+template <> struct Tile16<double> {
+    typedef double V __attribute__((ext_vector_type(4)));
+    // row of a lane's i-th value of D (column lane & 15)
+    static __device__ __forceinline__ int row(int lane, int i) { return (lane >> 4) + 4 * i; }
+    static __device__ __forceinline__ V mac(double a, double b, V c) {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
     }
-    __syncthreads();
-    const CE *in = reinterpret_cast<const CE *>(back ? L.work_z : L.source_expansions);
-    CE *out = reinterpret_cast<CE *>(L.work_y);
-    const int count = static_cast<int>(ch.count), P = static_cast<int>(rot.order), top = static_cast<int>(ch.max_order);
-    const int stages = top / 2 + 1; // stage h: degrees h and top - h (one degree when they coincide)
-    // degrees of stage h and their sizes; nb = 0 when the stage holds one degree
-    auto degrees = [&](int h, int &la, int &lb, int &na, int &nb) {
-        la = h;
-        lb = top - h;
-        na = 2 * la + 1;
-        nb = lb > la ? 2 * lb + 1 : 0;
-    };
-    E pd[kStagePerThread];
-    CE px[kSlicePerThread];
-    auto fetch = [&](int h) {
-        int la, lb, na, nb;
-        degrees(h, la, lb, na, nb);
-        const double *srca = L.small_d + rot.small_d + degree_block(la);
-        const double *srcb = L.small_d + rot.small_d + degree_block(lb);
+};
+template <> struct Tile16<float> {
+    typedef float V __attribute__((ext_vector_type(4)));
+    static __device__ __forceinline__ int row(int lane, int i) { return 4 * (lane >> 4) + i; }
+    static __device__ __forceinline__ V mac(float a, float b, V c) {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+};
+
+// The value of the neighbouring lane (lane ^ 1).
+__device__ __forceinline__ float neighbour(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xb1, 0xf, 0xf, true));
+}
+__device__ __forceinline__ double neighbour(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0xb1, 0xf, 0xf, true),
+              hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0xb1, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+
+// Two values of a lane pair (lane even: real parts, odd: imaginary parts) as one complex
+// value per lane, the first for the even lane and the second for the odd one.
+template <class E> __device__ __forceinline__ Cx<E> pair_values(E first, E second, int part) {
+    const E other = neighbour(part ? first : second);
+    return part ? Cx<E>{other, second} : Cx<E>{first, other};
+}
+
+// The two column tiles of a chunk: lane & 15 = 2 (link & 7) + (0 real, 1 imaginary). Where
+// coefficient e of the lane's link is: first + e step (complex values).
+struct LinkColumns {
+    std::uint64_t in[2], out[2];
+    std::uint32_t in_step, out_step;
+    bool live[2];
+};
+
+// RT row tiles from row0 of degree l for CT column tiles. Both directions read the block by
+// rows q, a row per 16 lanes: back takes d[t][q] = (-1)^(t - q) d[q][t], because columns of it
+// would be 16 separate lines a load (that pass took 1.5 times the forward one).
+template <class E, bool BACK, int RT, int CT>
+__device__ __forceinline__ void rotate_rows(const double *d, const C2 *phase, int l, int row0, const LinkColumns &at,
+                                            const Cx<E> *in, Cx<E> *out) {
+    using CE = Cx<E>;
+    using T = Tile16<E>;
+    const int lane = threadIdx.x & 63, n = 2 * l + 1, part = lane & 1;
+    const std::size_t base = static_cast<std::size_t>(l) * l;
+    typename T::V acc[RT][CT] = {};
+    int row[RT];
 #pragma unroll
-        for (int i = 0; i < kStagePerThread; ++i) {
-            const int e = threadIdx.x + 256 * i;
-            pd[i] = static_cast<E>(e < na * na ? srca[e] : e < na * na + nb * nb ? srcb[e - na * na] : 0.0);
+    for (int r = 0; r < RT; ++r)
+        row[r] = min(row0 + 16 * r + (lane & 15), n - 1); // rows beyond n: results dropped
+#pragma unroll 2
+    for (int q0 = 0; q0 < n; q0 += 4) {
+        const int q = q0 + (lane >> 4), qc = min(q, n - 1); // beyond n: zeros in the other operand
+        E a[RT], b[CT];
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+            a[r] = static_cast<E>(d[qc * n + row[r]]);
+#pragma unroll
+        for (int c = 0; c < CT; ++c) {
+            CE x{0, 0};
+            if (q < n && at.live[c])
+                x = in[at.in[c] + (base + q) * at.in_step];
+            if (!BACK)
+                x = to_cx<E>(phase[qc - l]) * x;
+            b[c] = part ? x.im : x.re;
+            if (BACK && (q & 1))
+                b[c] = -b[c];
         }
-        const int w = na + nb;
 #pragma unroll
-        for (int i = 0; i < kSlicePerThread; ++i) {
-            const int e = threadIdx.x + 256 * i;
-            CE v{0, 0};
-            if (e < count * w) {
-                const int j = e / w, q = e % w;
-                const int l = q < na ? la : lb, qq = q < na ? q : q - na;
-                if (l <= ord[j])
-                    v = in[src_off[j] + static_cast<std::size_t>(l) * l + qq];
-            }
-            px[i] = v;
-        }
-    };
-    fetch(split);
-    for (int h = split; h < stages; h += splits) {
-        int la, lb, na, nb;
-        degrees(h, la, lb, na, nb);
-        const int w = na + nb;
-        __syncthreads();
+        for (int r = 0; r < RT; ++r)
 #pragma unroll
-        for (int i = 0; i < kStagePerThread; ++i) {
-            const int e = threadIdx.x + 256 * i;
-            if (e < na * na + nb * nb)
-                dl[e] = pd[i];
-        }
+            for (int c = 0; c < CT; ++c)
+                acc[r][c] = T::mac(a[r], b[c], acc[r][c]);
+    }
 #pragma unroll
-        for (int i = 0; i < kSlicePerThread; ++i) {
-            const int e = threadIdx.x + 256 * i;
-            if (e < count * w) {
-                const int j = e / w, q = e % w;
-                const int l = q < na ? la : lb, qq = q < na ? q : q - na;
-                xs[j][q] = back ? px[i] : ph[P + qq - l] * px[i];
-            }
-        }
-        __syncthreads();
-        if (h + splits < stages)
-            fetch(h + splits);
-        // thread = (output t of one of the two degrees, group of 4 links): one Wigner
-        // load feeds 4 accumulators
-        const int groups = (count + 3) / 4;
-        for (int e = threadIdx.x; e < groups * w; e += blockDim.x) {
-            const int g = e / w, tq = e % w, j0 = 4 * g;
-            const bool first = tq < na;
-            const int l = first ? la : lb, n = first ? na : nb, t = first ? tq : tq - na, x0 = first ? 0 : na;
-            const E *dbl = dl + (first ? 0 : na * na);
-            CE s0{0, 0}, s1{0, 0}, s2{0, 0}, s3{0, 0};
-            const int stride = back ? 1 : n;
-            const E *drow = back ? dbl + t * n : dbl + t;
-            // three steps per pass: their 15 LDS reads are issued before the products
-            // (three, not four, keeps the order-32 kernel within the 168 registers of
-            // three waves per SIMD: measured 4.18 ms per horn apply against 4.57 ms)
-            constexpr int kSteps = 3;
-            int q = 0;
-            for (; q + kSteps <= n; q += kSteps) {
-                E d[kSteps];
-                CE x[kSteps][4];
+    for (int r = 0; r < RT; ++r)
 #pragma unroll
-                for (int u = 0; u < kSteps; ++u) {
-                    d[u] = drow[(q + u) * stride];
+        for (int i = 0; i < 4; i += 2) {
+            const int t = row0 + 16 * r + T::row(lane, i + part); // the lane's value of the two
+            const CE ph = BACK ? to_cx<E>(phase[min(t, n - 1) - l]) : CE{1, 0};
 #pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        x[u][i] = xs[j0 + i][x0 + q + u];
+            for (int c = 0; c < CT; ++c) {
+                CE v = pair_values<E>(acc[r][c][i], acc[r][c][i + 1], part);
+                if (BACK) {
+                    v = conj(ph) * v;
+                    if (t & 1)
+                        v = CE{-v.re, -v.im};
                 }
-#pragma unroll
-                for (int u = 0; u < kSteps; ++u) {
-                    s0 = s0 + d[u] * x[u][0];
-                    s1 = s1 + d[u] * x[u][1];
-                    s2 = s2 + d[u] * x[u][2];
-                    s3 = s3 + d[u] * x[u][3];
-                }
-            }
-            for (; q < n; ++q) {
-                const E d = drow[q * stride];
-                s0 = s0 + d * xs[j0][x0 + q];
-                s1 = s1 + d * xs[j0 + 1][x0 + q];
-                s2 = s2 + d * xs[j0 + 2][x0 + q];
-                s3 = s3 + d * xs[j0 + 3][x0 + q];
-            }
-            const CE sv[4] = {s0, s1, s2, s3};
-            const CE rot_back = back ? conj(ph[P + t - l]) : CE{1, 0};
-            const std::size_t base = static_cast<std::size_t>(l) * l;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int j = j0 + i;
-                if (j < count && l <= ord[j])
-                    out[dst_off[j] + (back ? base + t : m_major(ord[j], l, t - l))] = back ? rot_back * sv[i] : sv[i];
+                if (t < n && at.live[c])
+                    out[at.out[c] + (base + t) * at.out_step] = v;
             }
         }
+}
+
+template <class E, bool BACK, int CT>
+__device__ __forceinline__ void rotate_degrees(const FmmTranslateLaunch &L, const FmmChunk &ch, int top,
+                                               const LinkColumns &at) {
+    const FmmRotation rot = L.rotations[ch.rotation];
+    const C2 *phase = reinterpret_cast<const C2 *>(L.azimuth) + rot.azimuth + rot.order; // of m = 0
+    const Cx<E> *in = reinterpret_cast<const Cx<E> *>(BACK ? L.work_z : L.source_expansions);
+    Cx<E> *out = reinterpret_cast<Cx<E> *>(L.work_y);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    for (int l = 4 * blockIdx.y + wave; l <= top; l += 4 * gridDim.y) {
+        const double *d = L.small_d + rot.small_d + degree_block(l);
+        for (int row0 = 0; row0 < 2 * l + 1; row0 += 64)
+            switch (min((2 * l + 1 - row0 + 15) / 16, 4)) {
+            case 1: rotate_rows<E, BACK, 1, CT>(d, phase, l, row0, at, in, out); break;
+            case 2: rotate_rows<E, BACK, 2, CT>(d, phase, l, row0, at, in, out); break;
+            case 3: rotate_rows<E, BACK, 3, CT>(d, phase, l, row0, at, in, out); break;
+            default: rotate_rows<E, BACK, 4, CT>(d, phase, l, row0, at, in, out);
+            }
     }
 }
 
-// Z = T Y per |m| block for a chunk of links sharing one coaxial plan, two blocks per
-// stage (|m| = h and mm - h, which balances the rows x columns of the two): the blocks
-// T_m and the chunk's order-m columns of Y are staged in LDS, the next stage's values
-// prefetched into registers during the current products. Workgroup (chunk, y) takes
-// the stages y, y + Y, ... (Y = gridDim.y) of its chunk's stage sequence.
-// T_m rows are stored with an odd stride (cols | 1) of 16-byte values, so the
-// consecutive rows read by consecutive lanes fall in distinct bank groups.
-template <int kP, class E>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kP <= 32 ? 4 : 1))) void coaxial_links(FmmTranslateLaunch L) {
-    using CE = Cx<E>;
-    constexpr int kAxialRows = kP + 1;
-    // A stage pairs |m| = h with mm - h while their columns fit kColumns (always when
-    // ps <= pt: cols_a + cols_b = ps + 2), else holds one block. Its blocks hold at most
-    // (pt + 1)(ps + 2) <= kAxialRows^2 + kAxialRows values, stored with odd row strides
-    // (at most rows_a + rows_b <= 2 kAxialRows more).
-    constexpr int kBlockElems = kAxialRows * kAxialRows + kAxialRows;
-    constexpr int kBlock = kAxialRows * (kAxialRows + 3);
-    constexpr int kBlockPerThread = (kBlockElems + 255) / 256;
-    constexpr int kColumns = kAxialRows + 1;
-    constexpr int kColumnPerThread = (kFmmChunk * 2 * kColumns + 255) / 256;
-    __shared__ CE tm[kBlock];
-    __shared__ CE ys[kFmmChunk][2][kColumns];
-    __shared__ std::uint64_t slot[kFmmChunk];
-    const FmmChunk ch = L.axial_chunks[blockIdx.x];
-    const int split = static_cast<int>(blockIdx.y), splits = static_cast<int>(gridDim.y);
-    const FmmLink first = L.links[L.axial_order[ch.first]];
-    const int ps = static_cast<int>(first.source_order), pt = static_cast<int>(first.target_order), mm = min(ps, pt);
-    const C2 *T = reinterpret_cast<const C2 *>(L.axial) + L.axial_offsets[first.axial];
-    const CE *y = reinterpret_cast<const CE *>(L.work_y);
-    CE *z = reinterpret_cast<CE *>(L.work_z);
-    const int count = static_cast<int>(ch.count);
-    if (threadIdx.x < count)
-        slot[threadIdx.x] = L.links[L.axial_order[ch.first + threadIdx.x]].slot;
-    // degrees above min(ps, pt) in |m| have no source: those outputs are zero
-    const int nct = (pt + 1) * (pt + 1);
-    __syncthreads();
-    if (split == 0)
-        for (int e = threadIdx.x; e < count * nct; e += blockDim.x) {
-            const int j = e / nct, c = e % nct;
-            int l, t;
-            split_index(c, l, t);
-            if (abs(t - l) > mm)
-                z[slot[j] + c] = {0, 0};
-        }
-    struct Pair {
-        int ma, mb, ra, ca, rb, cb; // rb = cb = 0 when the stage holds one block
-        int lo, hi;                 // the |m| still to do after this stage: lo .. hi
-    };
-    // the stage that starts with |m| in lo .. hi still to do
-    auto blocks = [&](int lo, int hi) {
-        Pair q;
-        q.ma = lo;
-        q.ra = pt - lo + 1;
-        q.ca = ps - lo + 1;
-        const bool two = hi > lo && q.ca + (ps - hi + 1) <= kColumns;
-        q.mb = two ? hi : lo;
-        q.rb = two ? pt - hi + 1 : 0;
-        q.cb = two ? ps - hi + 1 : 0;
-        q.lo = lo + 1;
-        q.hi = two ? hi - 1 : hi;
-        return q;
-    };
-    CE pt_[kBlockPerThread], py[kColumnPerThread];
-    auto fetch = [&](const Pair &q) {
-        const C2 *Ta = T + axial_block(q.ma, ps, pt), *Tb = T + axial_block(q.mb, ps, pt);
-        const int sa = q.ra * q.ca, sb = q.rb * q.cb;
-#pragma unroll
-        for (int i = 0; i < kBlockPerThread; ++i) {
-            const int e = threadIdx.x + 256 * i;
-            pt_[i] = to_cx<E>(e < sa ? Ta[e] : e < sa + sb ? Tb[e - sa] : C2{0, 0});
-        }
-        const int w = q.ca + q.cb;
-#pragma unroll
-        for (int i = 0; i < kColumnPerThread; ++i) {
-            const int e = threadIdx.x + 256 * i;
-            const bool live = e < count * 2 * w;
-            const int ee = live ? e : 0;
-            const int j = ee / (2 * w), r = ee % (2 * w), sgn = r / w, c = r % w;
-            const int m = c < q.ca ? q.ma : q.mb, n = m + (c < q.ca ? c : c - q.ca);
-            py[i] = live ? y[slot[j] + m_major(ps, n, sgn ? -m : m)] : CE{0, 0};
-        }
-    };
-    // the stage `steps` stages after p; false when the sequence ends first
-    auto advance = [&](Pair &p, int steps) {
-        for (int i = 0; i < steps; ++i) {
-            if (p.lo > p.hi)
-                return false;
-            p = blocks(p.lo, p.hi);
-        }
-        return true;
-    };
-    Pair q = blocks(0, mm);
-    if (!advance(q, split))
+// Chunk of a workgroup: the chip's 8 dies take workgroups in turn, so each gets a run of
+// consecutive chunks, which share their direction's blocks in its L2.
+__device__ __forceinline__ std::uint32_t chunk_of(std::uint32_t block, std::uint32_t chunks) {
+    const std::uint32_t die = block % 8, per = chunks / 8, more = chunks % 8;
+    return die * per + min(die, more) + block / 8;
+}
+
+// Workgroup (chunk, y) takes the degrees 4 y .. 4 y + 3, 4 (y + Y) .., (Y = gridDim.y), so a
+// level with few chunks spreads its degrees over more workgroups.
+template <class E, bool BACK> __global__ __launch_bounds__(256, 3) void rotate_links(FmmTranslateLaunch L) {
+    const FmmChunk ch = L.chunks[chunk_of(blockIdx.x, gridDim.x)];
+    const FmmLink first = L.links[L.order[ch.first]]; // its orders are the chunk's
+    const int top = static_cast<int>(BACK ? first.target_order : first.source_order);
+    if (4 * static_cast<int>(blockIdx.y) > top)
         return;
-    fetch(q);
-    for (;;) {
-        const int sa = q.ra * q.ca, w = q.ca + q.cb;
-        const int stride_a = q.ca | 1, stride_b = q.cb | 1, base_b = q.ra * stride_a;
-        __syncthreads();
+    LinkColumns at;
+    at.in_step = BACK ? ch.count : 1;
+    at.out_step = BACK ? 1 : ch.count;
 #pragma unroll
-        for (int i = 0; i < kBlockPerThread; ++i) {
-            const int e = threadIdx.x + 256 * i;
-            if (e < sa)
-                tm[(e / q.ca) * stride_a + e % q.ca] = pt_[i];
-            else if (e < sa + q.rb * q.cb)
-                tm[base_b + ((e - sa) / q.cb) * stride_b + (e - sa) % q.cb] = pt_[i];
-        }
+    for (std::uint32_t c = 0; c < 2; ++c) {
+        const std::uint32_t j = 8 * c + (threadIdx.x & 15) / 2;
+        at.live[c] = j < ch.count;
+        const FmmLink lk = L.links[L.order[ch.first + (at.live[c] ? j : 0)]];
+        at.in[c] = BACK ? ch.base + j : lk.source;
+        at.out[c] = BACK ? lk.slot : ch.base + j;
+    }
+    if (ch.count > 8)
+        rotate_degrees<E, BACK, 2>(L, ch, top, at);
+    else
+        rotate_degrees<E, BACK, 1>(L, ch, top, at);
+}
+
+// Rows row0 .. row0 + 16 RT of Z = T Y for order |m|, both signs, CT column tiles.
+template <class E, int RT, int CT>
+__device__ __forceinline__ void axial_rows(const C2 *T, int m, int ps, int pt, int row0, std::uint64_t base, int count,
+                                           const Cx<E> *y, Cx<E> *z) {
+    using CE = Cx<E>;
+    using M = Tile16<E>;
+    const int lane = threadIdx.x & 63, rows = pt + 1 - m, cols = ps + 1 - m, part = lane & 1, j0 = (lane & 15) / 2;
+    typename M::V acc[RT][CT][2] = {};
+    int row[RT];
 #pragma unroll
-        for (int i = 0; i < kColumnPerThread; ++i) {
-            const int e = threadIdx.x + 256 * i;
-            if (e < count * 2 * w) {
-                const int j = e / (2 * w), r = e % (2 * w), sgn = r / w;
-                ys[j][sgn][r % w] = py[i];
-            }
-        }
-        __syncthreads();
-        Pair next = q;
-        const bool more = advance(next, splits);
-        if (more)
-            fetch(next);
-        // thread = (row of one of the two blocks, sign, group of 4 links): one T load
-        // feeds 4 accumulators
-        const int groups = (count + 3) / 4, rows2 = 2 * (q.ra + q.rb);
-        for (int e = threadIdx.x; e < groups * rows2; e += blockDim.x) {
-            const int g = e / rows2, r = e % rows2, j0 = 4 * g;
-            const int half = r < 2 * q.ra ? 0 : 1;
-            const int rr = half ? r - 2 * q.ra : r, rows = half ? q.rb : q.ra;
-            const int sgn = rr / rows, m = half ? q.mb : q.ma, l = m + rr % rows;
-            if (sgn && !m)
-                continue;
-            const int cols = half ? q.cb : q.ca, c0 = half ? q.ca : 0;
-            const CE *trow = tm + (half ? base_b + (l - m) * stride_b : (l - m) * stride_a);
-            CE s0{0, 0}, s1{0, 0}, s2{0, 0}, s3{0, 0};
-            // two columns per pass: their 10 LDS reads are issued before the products (two,
-            // not four, keeps the order-32 kernel within the 128 registers of four waves
-            // per SIMD, which its LDS allows; both measured alike on the horn apply)
-            constexpr int kSteps = 2;
-            int c = 0;
-            for (; c + kSteps <= cols; c += kSteps) {
-                CE tv[kSteps], yv[kSteps][4];
+    for (int r = 0; r < RT; ++r)
+        row[r] = min(row0 + 16 * r + (lane & 15), rows - 1);
+#pragma unroll 2
+    for (int q0 = 0; q0 < cols; q0 += 4) {
+        const int q = q0 + (lane >> 4), qc = min(q, cols - 1), l = m + q;
+        CE a[RT];
 #pragma unroll
-                for (int u = 0; u < kSteps; ++u) {
-                    tv[u] = trow[c + u];
+        for (int r = 0; r < RT; ++r)
+            a[r] = to_cx<E>(T[row[r] * cols + qc]);
 #pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        yv[u][i] = ys[j0 + i][sgn][c0 + c + u];
-                }
+        for (int c = 0; c < CT; ++c)
 #pragma unroll
-                for (int u = 0; u < kSteps; ++u) {
-                    s0 = s0 + tv[u] * yv[u][0];
-                    s1 = s1 + tv[u] * yv[u][1];
-                    s2 = s2 + tv[u] * yv[u][2];
-                    s3 = s3 + tv[u] * yv[u][3];
+            for (int sgn = 0; sgn < 2; ++sgn) {
+                if (sgn && m == 0)
+                    continue;
+                CE v{0, 0};
+                if (q < cols && j0 + 8 * c < count)
+                    v = y[base + static_cast<std::size_t>(l * (l + 1) + (sgn ? -m : m)) * count + j0 + 8 * c];
+                const E direct = part ? v.im : v.re, crossed = part ? v.re : -v.im;
+#pragma unroll
+                for (int r = 0; r < RT; ++r) {
+                    acc[r][c][sgn] = M::mac(a[r].re, direct, acc[r][c][sgn]);
+                    acc[r][c][sgn] = M::mac(a[r].im, crossed, acc[r][c][sgn]);
                 }
             }
-            for (; c < cols; ++c) {
-                const CE tv = trow[c];
-                s0 = s0 + tv * ys[j0][sgn][c0 + c];
-                s1 = s1 + tv * ys[j0 + 1][sgn][c0 + c];
-                s2 = s2 + tv * ys[j0 + 2][sgn][c0 + c];
-                s3 = s3 + tv * ys[j0 + 3][sgn][c0 + c];
-            }
-            const CE sv[4] = {s0, s1, s2, s3};
-            const std::size_t idx = static_cast<std::size_t>(l) * l + l + (sgn ? -m : m);
+    }
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if (j0 + i < count)
-                    z[slot[j0 + i] + idx] = sv[i];
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int i = 0; i < 4; i += 2) {
+            const int t = row0 + 16 * r + M::row(lane, i + part), l = m + t;
+#pragma unroll
+            for (int c = 0; c < CT; ++c) {
+                const CE plus = pair_values<E>(acc[r][c][0][i], acc[r][c][0][i + 1], part),
+                         minus = pair_values<E>(acc[r][c][1][i], acc[r][c][1][i + 1], part);
+                if (t < rows && j0 + 8 * c < count) {
+                    CE *at = z + base + static_cast<std::size_t>(l * (l + 1)) * count + j0 + 8 * c;
+                    at[m * count] = plus;
+                    if (m)
+                        at[-m * count] = minus;
+                }
+            }
         }
-        if (!more)
-            break;
-        q = next;
+}
+
+template <class E, int CT>
+__device__ __forceinline__ void axial_orders(const FmmTranslateLaunch &L, const C2 *T, int ps, int pt,
+                                             const FmmChunk &ch) {
+    const Cx<E> *y = reinterpret_cast<const Cx<E> *>(L.work_y);
+    Cx<E> *z = reinterpret_cast<Cx<E> *>(L.work_z);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), mm = min(ps, pt);
+    for (int m = 4 * blockIdx.y + wave; m <= mm; m += 4 * gridDim.y) {
+        const C2 *block = T + axial_block(m, ps, pt);
+        const int rows = pt + 1 - m, count = static_cast<int>(ch.count);
+        for (int row0 = 0; row0 < rows; row0 += 32)
+            if (rows - row0 > 16)
+                axial_rows<E, 2, CT>(block, m, ps, pt, row0, ch.base, count, y, z);
+            else
+                axial_rows<E, 1, CT>(block, m, ps, pt, row0, ch.base, count, y, z);
     }
 }
 
-// Orders above kMaxFmmOrder (up to kMaxWideOrder): the same two passes with the
-// Wigner block staged in column (forward) or row (back) tiles of kWideTile and no
-// register prefetch; one workgroup per chunk holds ~100 KB of LDS.
-constexpr int kWideN = 2 * kMaxWideOrder + 1;
-constexpr int kWideTile = kMaxWideOrder + 1;
-
-__global__ __launch_bounds__(256) void rotate_links_wide(FmmTranslateLaunch L, bool back) {
-    __shared__ double dt[kWideN * kWideTile];
-    __shared__ C2 xs[kFmmChunk][kWideN];
-    __shared__ C2 ph[kWideN];
-    __shared__ std::uint64_t src_off[kFmmChunk], dst_off[kFmmChunk];
-    __shared__ int ord[kFmmChunk];
-    const FmmChunk ch = L.chunks[blockIdx.x];
-    const FmmRotation rot = L.rotations[ch.rotation];
-    const C2 *az = reinterpret_cast<const C2 *>(L.azimuth) + rot.azimuth;
-    for (int m = threadIdx.x; m <= 2 * static_cast<int>(rot.order); m += blockDim.x)
-        ph[m] = az[m];
-    if (threadIdx.x < ch.count) {
-        const FmmLink lk = L.links[L.order[ch.first + threadIdx.x]];
-        src_off[threadIdx.x] = back ? lk.slot : lk.source;
-        dst_off[threadIdx.x] = lk.slot;
-        ord[threadIdx.x] = static_cast<int>(back ? lk.target_order : lk.source_order);
-    }
-    __syncthreads();
-    const C2 *in = reinterpret_cast<const C2 *>(back ? L.work_z : L.source_expansions);
-    C2 *out = reinterpret_cast<C2 *>(L.work_y);
-    const int count = static_cast<int>(ch.count), P = static_cast<int>(rot.order), top = static_cast<int>(ch.max_order);
-    const int groups = (count + 3) / 4;
-    for (int l = 0; l <= top; ++l) {
-        const int n = 2 * l + 1;
-        const std::size_t base = static_cast<std::size_t>(l) * l;
-        const double *dl = L.small_d + rot.small_d + static_cast<std::size_t>(l) * (2 * l - 1) * (2 * l + 1) / 3;
-        __syncthreads();
-        for (int e = threadIdx.x; e < count * n; e += blockDim.x) {
-            const int j = e / n, q = e % n;
-            C2 v{0, 0};
-            if (l <= ord[j]) {
-                v = in[src_off[j] + base + q];
-                if (!back)
-                    v = ph[P + q - l] * v;
-            }
-            xs[j][q] = v;
-        }
-        for (int t0 = 0; t0 < n; t0 += kWideTile) {
-            const int tw = min(kWideTile, n - t0);
-            __syncthreads();
-            // forward: dt[q][t - t0] = d[q][t]; back: dt[t - t0][q] = d[t][q]
-            for (int e = threadIdx.x; e < n * tw; e += blockDim.x) {
-                if (back) {
-                    const int t = e / n, q = e % n;
-                    dt[t * n + q] = dl[static_cast<std::size_t>(t0 + t) * n + q];
-                } else {
-                    const int q = e / tw, t = e % tw;
-                    dt[q * tw + t] = dl[static_cast<std::size_t>(q) * n + t0 + t];
-                }
-            }
-            __syncthreads();
-            for (int e = threadIdx.x; e < groups * tw; e += blockDim.x) {
-                const int g = e / tw, tt = e % tw, t = t0 + tt, j0 = 4 * g;
-                C2 s0{0, 0}, s1{0, 0}, s2{0, 0}, s3{0, 0};
-                const int stride = back ? 1 : tw;
-                const double *drow = back ? dt + tt * n : dt + tt;
-                for (int q = 0; q < n; ++q) {
-                    const double d = drow[q * stride];
-                    s0 = s0 + d * xs[j0][q];
-                    s1 = s1 + d * xs[min(j0 + 1, kFmmChunk - 1)][q];
-                    s2 = s2 + d * xs[min(j0 + 2, kFmmChunk - 1)][q];
-                    s3 = s3 + d * xs[min(j0 + 3, kFmmChunk - 1)][q];
-                }
-                const C2 sv[4] = {s0, s1, s2, s3};
-                const C2 rot_back = back ? conj(ph[P + t - l]) : C2{1, 0};
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int j = j0 + i;
-                    if (j < count && l <= ord[j])
-                        out[dst_off[j] + (back ? base + t : m_major(ord[j], l, t - l))] = back ? rot_back * sv[i] : sv[i];
-                }
-            }
-        }
-    }
-}
-
-constexpr int kWideRows = kMaxWideOrder + 1;
-
-__global__ __launch_bounds__(256) void coaxial_links_wide(FmmTranslateLaunch L) {
-    __shared__ C2 tm[kWideRows * kWideRows];
-    __shared__ C2 ys[kFmmChunk][2][kWideRows];
-    __shared__ std::uint64_t slot[kFmmChunk];
-    const FmmChunk ch = L.axial_chunks[blockIdx.x];
-    const FmmLink first = L.links[L.axial_order[ch.first]];
+// Z = T Y per |m| block; workgroup (chunk, y) takes the orders 4 y .. 4 y + 3, 4 (y + Y) .. of
+// the chunk.
+template <class E> __global__ __launch_bounds__(256, 4) void coaxial_links(FmmTranslateLaunch L) {
+    const FmmChunk ch = L.chunks[chunk_of(blockIdx.x, gridDim.x)];
+    const FmmLink first = L.links[L.order[ch.first]];
     const int ps = static_cast<int>(first.source_order), pt = static_cast<int>(first.target_order), mm = min(ps, pt);
     const C2 *T = reinterpret_cast<const C2 *>(L.axial) + L.axial_offsets[first.axial];
-    const C2 *y = reinterpret_cast<const C2 *>(L.work_y);
-    C2 *z = reinterpret_cast<C2 *>(L.work_z);
-    const int count = static_cast<int>(ch.count);
-    if (threadIdx.x < count)
-        slot[threadIdx.x] = L.links[L.axial_order[ch.first + threadIdx.x]].slot;
-    const int nct = (pt + 1) * (pt + 1);
-    __syncthreads();
-    for (int e = threadIdx.x; e < count * nct; e += blockDim.x) {
-        const int j = e / nct, c = e % nct;
-        int l, t;
-        split_index(c, l, t);
-        if (abs(t - l) > mm)
-            z[slot[j] + c] = {0, 0};
-    }
-    std::size_t off = 0;
-    const int groups = (count + 3) / 4;
-    for (int m = 0; m <= mm; ++m) {
-        const int rows = pt - m + 1, cols = ps - m + 1;
-        __syncthreads();
-        const int stride = cols | 1;
-        for (int e = threadIdx.x; e < rows * cols; e += blockDim.x)
-            tm[(e / cols) * stride + e % cols] = T[off + e];
-        for (int e = threadIdx.x; e < kFmmChunk * 2 * cols; e += blockDim.x) {
-            const int j = e / (2 * cols), r = e % (2 * cols), sgn = r / cols, n = m + r % cols;
-            ys[j][sgn][r % cols] = j < count ? y[slot[j] + m_major(ps, n, sgn ? -m : m)]
-                                             : C2{0, 0};
-        }
-        __syncthreads();
-        off += static_cast<std::size_t>(rows) * cols;
-        for (int e = threadIdx.x; e < groups * 2 * rows; e += blockDim.x) {
-            const int g = e / (2 * rows), r = e % (2 * rows), sgn = r / rows, l = m + r % rows, j0 = 4 * g;
-            if (sgn && !m)
-                continue;
-            C2 s0{0, 0}, s1{0, 0}, s2{0, 0}, s3{0, 0};
-            const C2 *trow = tm + (l - m) * stride;
-            for (int c = 0; c < cols; ++c) {
-                const C2 tv = trow[c];
-                s0 = s0 + tv * ys[j0][sgn][c];
-                s1 = s1 + tv * ys[j0 + 1][sgn][c];
-                s2 = s2 + tv * ys[j0 + 2][sgn][c];
-                s3 = s3 + tv * ys[j0 + 3][sgn][c];
-            }
-            const C2 sv[4] = {s0, s1, s2, s3};
-            const std::size_t idx = static_cast<std::size_t>(l) * l + l + (sgn ? -m : m);
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if (j0 + i < count)
-                    z[slot[j0 + i] + idx] = sv[i];
+    // orders above min(ps, pt) have no source: those outputs are zero
+    if (blockIdx.y == 0 && pt > mm) {
+        Cx<E> *z = reinterpret_cast<Cx<E> *>(L.work_z) + ch.base;
+        const int count = static_cast<int>(ch.count);
+        for (int e = threadIdx.x; e < count * (pt + 1) * (pt + 1); e += blockDim.x) {
+            int l, t;
+            split_index(e / count, l, t);
+            if (abs(t - l) > mm)
+                z[e] = {0, 0};
         }
     }
-}
-
-// Orders above kMaxWideOrder (up to kMaxBigOrder): no staging of a whole Wigner or
-// coaxial block fits in LDS, so the reduction index is tiled. Rotations: per degree,
-// all of the chunk's inputs (one half of the chunk, 8 links, at a time) stay in LDS
-// while 32-row slabs of d_l pass through; every thread keeps the running sums of
-// its (t, 4-link group) items in registers. Coaxial products: per |m| block the
-// chunk's columns stay in LDS while 16-column slabs of T_m pass through.
-constexpr int kBigN = 2 * kMaxBigOrder + 1;
-constexpr int kBigHalf = 8; // links per pass (a chunk of kFmmChunk links takes kFmmChunk / 8 passes)
-constexpr int kBigSlab = 32;
-constexpr int kBigItems = (kBigN * (kBigHalf / 4) + 255) / 256; // (t, group) items per thread
-
-__global__ __launch_bounds__(256) void rotate_links_big(FmmTranslateLaunch L, bool back) {
-    __shared__ C2 xs[kBigHalf][kBigN];
-    __shared__ double dt[kBigSlab * kBigN];
-    __shared__ C2 ph[kBigN];
-    __shared__ std::uint64_t src_off[kFmmChunk], dst_off[kFmmChunk];
-    __shared__ int ord[kFmmChunk];
-    const FmmChunk ch = L.chunks[blockIdx.x];
-    const FmmRotation rot = L.rotations[ch.rotation];
-    const C2 *az = reinterpret_cast<const C2 *>(L.azimuth) + rot.azimuth;
-    for (int m = threadIdx.x; m <= 2 * static_cast<int>(rot.order); m += blockDim.x)
-        ph[m] = az[m];
-    if (threadIdx.x < ch.count) {
-        const FmmLink lk = L.links[L.order[ch.first + threadIdx.x]];
-        src_off[threadIdx.x] = back ? lk.slot : lk.source;
-        dst_off[threadIdx.x] = lk.slot;
-        ord[threadIdx.x] = static_cast<int>(back ? lk.target_order : lk.source_order);
-    }
-    __syncthreads();
-    const C2 *in = reinterpret_cast<const C2 *>(back ? L.work_z : L.source_expansions);
-    C2 *out = reinterpret_cast<C2 *>(L.work_y);
-    const int count = static_cast<int>(ch.count), P = static_cast<int>(rot.order), top = static_cast<int>(ch.max_order);
-    for (int h = 0; h * kBigHalf < count; ++h) {
-        const int j_first = h * kBigHalf, hc = min(kBigHalf, count - j_first);
-        for (int l = 0; l <= top; ++l) {
-            const int n = 2 * l + 1;
-            const std::size_t base = static_cast<std::size_t>(l) * l;
-            const double *dl = L.small_d + rot.small_d + static_cast<std::size_t>(l) * (2 * l - 1) * (2 * l + 1) / 3;
-            __syncthreads();
-            for (int e = threadIdx.x; e < kBigHalf * n; e += blockDim.x) {
-                const int jj = e / n, q = e % n, j = j_first + jj;
-                C2 v{0, 0};
-                if (jj < hc && l <= ord[j]) {
-                    v = in[src_off[j] + base + q];
-                    if (!back)
-                        v = ph[P + q - l] * v;
-                }
-                xs[jj][q] = v;
-            }
-            C2 acc[kBigItems][4];
-#pragma unroll
-            for (int it = 0; it < kBigItems; ++it)
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    acc[it][i] = {0, 0};
-            const int items = n * (kBigHalf / 4);
-            for (int q0 = 0; q0 < n; q0 += kBigSlab) {
-                const int qw = min(kBigSlab, n - q0);
-                __syncthreads();
-                // dt[qq][t] = d[q][t] (forward) or d[t][q] (back), q = q0 + qq
-                for (int e = threadIdx.x; e < qw * n; e += blockDim.x) {
-                    if (back) {
-                        const int t = e / qw, qq = e % qw;
-                        dt[qq * n + t] = dl[static_cast<std::size_t>(t) * n + q0 + qq];
-                    } else {
-                        const int qq = e / n, t = e % n;
-                        dt[qq * n + t] = dl[static_cast<std::size_t>(q0 + qq) * n + t];
-                    }
-                }
-                __syncthreads();
-#pragma unroll
-                for (int it = 0; it < kBigItems; ++it) {
-                    const int e = threadIdx.x + 256 * it;
-                    if (e >= items)
-                        continue;
-                    const int g = e / n, t = e % n, j0 = 4 * g;
-                    for (int qq = 0; qq < qw; ++qq) {
-                        const double d = dt[qq * n + t];
-                        const int q = q0 + qq;
-#pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            acc[it][i] = acc[it][i] + d * xs[j0 + i][q];
-                    }
-                }
-            }
-#pragma unroll
-            for (int it = 0; it < kBigItems; ++it) {
-                const int e = threadIdx.x + 256 * it;
-                if (e >= items)
-                    continue;
-                const int g = e / n, t = e % n;
-                const C2 rot_back = back ? conj(ph[P + t - l]) : C2{1, 0};
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int jj = 4 * g + i, j = j_first + jj;
-                    if (jj < hc && l <= ord[j])
-                        out[dst_off[j] + (back ? base + t : m_major(ord[j], l, t - l))] =
-                            back ? rot_back * acc[it][i] : acc[it][i];
-                }
-            }
-        }
-    }
-}
-
-constexpr int kBigRows = kMaxBigOrder + 1;
-constexpr int kBigCols = 16;
-constexpr int kBigCoaxItems = (kBigRows * 2 * (kFmmChunk / 4) + 255) / 256; // (row, sign, group) per thread
-
-__global__ __launch_bounds__(256) void coaxial_links_big(FmmTranslateLaunch L) {
-    __shared__ C2 ys[kFmmChunk][2][kBigCols]; // the current column tile of every link's +m / -m sources
-    __shared__ C2 tm[kBigRows * kBigCols];
-    __shared__ std::uint64_t slot[kFmmChunk];
-    const FmmChunk ch = L.axial_chunks[blockIdx.x];
-    const FmmLink first = L.links[L.axial_order[ch.first]];
-    const int ps = static_cast<int>(first.source_order), pt = static_cast<int>(first.target_order), mm = min(ps, pt);
-    const C2 *T = reinterpret_cast<const C2 *>(L.axial) + L.axial_offsets[first.axial];
-    const C2 *y = reinterpret_cast<const C2 *>(L.work_y);
-    C2 *z = reinterpret_cast<C2 *>(L.work_z);
-    const int count = static_cast<int>(ch.count);
-    if (threadIdx.x < count)
-        slot[threadIdx.x] = L.links[L.axial_order[ch.first + threadIdx.x]].slot;
-    const int nct = (pt + 1) * (pt + 1);
-    __syncthreads();
-    for (int e = threadIdx.x; e < count * nct; e += blockDim.x) {
-        const int j = e / nct, c = e % nct;
-        int l, t;
-        split_index(c, l, t);
-        if (abs(t - l) > mm)
-            z[slot[j] + c] = {0, 0};
-    }
-    std::size_t off = 0;
-    for (int m = 0; m <= mm; ++m) {
-        const int rows = pt - m + 1, cols = ps - m + 1;
-        C2 acc[kBigCoaxItems][4];
-#pragma unroll
-        for (int it = 0; it < kBigCoaxItems; ++it)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                acc[it][i] = {0, 0};
-        const int items = rows * 2 * (kFmmChunk / 4);
-        for (int c0 = 0; c0 < cols; c0 += kBigCols) {
-            const int cw = min(kBigCols, cols - c0);
-            __syncthreads();
-            for (int e = threadIdx.x; e < rows * cw; e += blockDim.x) {
-                const int r = e / cw, cc = e % cw;
-                tm[r * kBigCols + cc] = T[off + static_cast<std::size_t>(r) * cols + c0 + cc];
-            }
-            for (int e = threadIdx.x; e < kFmmChunk * 2 * cw; e += blockDim.x) {
-                const int j = e / (2 * cw), r = e % (2 * cw), sgn = r / cw, cc = r % cw, n = m + c0 + cc;
-                ys[j][sgn][cc] = j < count ? y[slot[j] + m_major(ps, n, sgn ? -m : m)] : C2{0, 0};
-            }
-            __syncthreads();
-#pragma unroll
-            for (int it = 0; it < kBigCoaxItems; ++it) {
-                const int e = threadIdx.x + 256 * it;
-                if (e >= items)
-                    continue;
-                const int g = e / (2 * rows), r = e % (2 * rows), sgn = r / rows, row = r % rows, j0 = 4 * g;
-                if (sgn && !m)
-                    continue;
-                for (int cc = 0; cc < cw; ++cc) {
-                    const C2 tv = tm[row * kBigCols + cc];
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        acc[it][i] = acc[it][i] + tv * ys[j0 + i][sgn][cc];
-                }
-            }
-        }
-#pragma unroll
-        for (int it = 0; it < kBigCoaxItems; ++it) {
-            const int e = threadIdx.x + 256 * it;
-            if (e >= items)
-                continue;
-            const int g = e / (2 * rows), r = e % (2 * rows), sgn = r / rows, l = m + r % rows, j0 = 4 * g;
-            if (sgn && !m)
-                continue;
-            const std::size_t idx = static_cast<std::size_t>(l) * l + l + (sgn ? -m : m);
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if (j0 + i < count)
-                    z[slot[j0 + i] + idx] = acc[it][i];
-        }
-        off += static_cast<std::size_t>(rows) * cols;
-    }
+    if (4 * static_cast<int>(blockIdx.y) > mm)
+        return;
+    if (ch.count > 8)
+        axial_orders<E, 2>(L, T, ps, pt, ch);
+    else
+        axial_orders<E, 1>(L, T, ps, pt, ch);
 }
 
 // target = sum of the destination's link results.
@@ -1299,53 +899,30 @@ void launch_leaf_test(const FmmLeaf *leaves, std::uint32_t leaf_count, const std
                            expansions, y);
 }
 
-// The order-templated translations of one launch (orders up to kMidFmmOrder) in scalar E.
-template <class E>
-void launch_links(const FmmTranslateLaunch &launch, std::uint32_t max_order, dim3 rot_grid, dim3 axial_grid,
-                  hipStream_t stream) {
-    if (max_order > kMaxFmmOrder) {
-        hipLaunchKernelGGL((rotate_links<kMidFmmOrder, E>), rot_grid, dim3(256), 0, stream, launch, false);
-        hipLaunchKernelGGL((coaxial_links<kMidFmmOrder, E>), axial_grid, dim3(256), 0, stream, launch);
-        hipLaunchKernelGGL((rotate_links<kMidFmmOrder, E>), rot_grid, dim3(256), 0, stream, launch, true);
-    } else if (max_order > kSmallFmmOrder) {
-        hipLaunchKernelGGL((rotate_links<kMaxFmmOrder, E>), rot_grid, dim3(256), 0, stream, launch, false);
-        hipLaunchKernelGGL((coaxial_links<kMaxFmmOrder, E>), axial_grid, dim3(256), 0, stream, launch);
-        hipLaunchKernelGGL((rotate_links<kMaxFmmOrder, E>), rot_grid, dim3(256), 0, stream, launch, true);
-    } else {
-        hipLaunchKernelGGL((rotate_links<kSmallFmmOrder, E>), rot_grid, dim3(256), 0, stream, launch, false);
-        hipLaunchKernelGGL((coaxial_links<kSmallFmmOrder, E>), axial_grid, dim3(256), 0, stream, launch);
-        hipLaunchKernelGGL((rotate_links<kSmallFmmOrder, E>), rot_grid, dim3(256), 0, stream, launch, true);
-    }
+// The translations of one launch in scalar E.
+template <class E> void launch_links(const FmmTranslateLaunch &launch, dim3 grid, hipStream_t stream) {
+    hipLaunchKernelGGL((rotate_links<E, false>), grid, dim3(256), 0, stream, launch);
+    hipLaunchKernelGGL((coaxial_links<E>), grid, dim3(256), 0, stream, launch);
+    hipLaunchKernelGGL((rotate_links<E, true>), grid, dim3(256), 0, stream, launch);
 }
 
 void launch_translate(const FmmTranslateLaunch &launch, std::uint32_t destination_count, std::uint32_t link_count,
-                      std::uint32_t chunk_count, std::uint32_t axial_chunk_count, std::uint32_t max_order,
-                      std::uint32_t split_target, hipStream_t stream) {
+                      std::uint32_t chunk_count, std::uint32_t max_order, std::uint32_t split_target,
+                      hipStream_t stream) {
     if (!destination_count)
         return;
-    // Levels with few chunks spread each chunk's stages over up to `splits` workgroups,
-    // so that a launch holds about split_target workgroups (a rotation chunk has
-    // max_order / 2 + 1 stages, a coaxial chunk at most as many); 0 = no split.
-    auto splits = [&](std::uint32_t chunks) {
-        const std::uint32_t stages = max_order / 2 + 1;
-        return chunks && split_target ? std::max(1u, std::min(stages, (split_target + chunks - 1) / chunks)) : 1u;
-    };
-    const dim3 rot_grid(chunk_count, splits(chunk_count)), axial_grid(axial_chunk_count, splits(axial_chunk_count));
     if (launch.fp32 && link_count && max_order > kMidFmmOrder)
         throw std::invalid_argument("FP32 translations take orders up to 48 only");
-    if (link_count && max_order > kMaxWideOrder) {
-        hipLaunchKernelGGL(rotate_links_big, dim3(chunk_count), dim3(256), 0, stream, launch, false);
-        hipLaunchKernelGGL(coaxial_links_big, dim3(axial_chunk_count), dim3(256), 0, stream, launch);
-        hipLaunchKernelGGL(rotate_links_big, dim3(chunk_count), dim3(256), 0, stream, launch, true);
-    } else if (link_count && max_order > kMidFmmOrder) {
-        hipLaunchKernelGGL(rotate_links_wide, dim3(chunk_count), dim3(256), 0, stream, launch, false);
-        hipLaunchKernelGGL(coaxial_links_wide, dim3(axial_chunk_count), dim3(256), 0, stream, launch);
-        hipLaunchKernelGGL(rotate_links_wide, dim3(chunk_count), dim3(256), 0, stream, launch, true);
-    } else if (link_count && launch.fp32) {
-        launch_links<float>(launch, max_order, rot_grid, axial_grid, stream);
-    } else if (link_count) {
-        launch_links<double>(launch, max_order, rot_grid, axial_grid, stream);
-    }
+    // Levels with few chunks spread each chunk's degrees (orders), four at a time, over up
+    // to `splits` workgroups, so that a launch holds about split_target workgroups; 0 = no split.
+    const std::uint32_t stages = max_order / 4 + 1,
+                        splits = chunk_count && split_target
+                                     ? std::max(1u, std::min(stages, (split_target + chunk_count - 1) / chunk_count))
+                                     : 1u;
+    if (link_count && launch.fp32)
+        launch_links<float>(launch, dim3(chunk_count, splits), stream);
+    else if (link_count)
+        launch_links<double>(launch, dim3(chunk_count, splits), stream);
     if (launch.fp32)
         hipLaunchKernelGGL(gather_links<float>, dim3(destination_count), dim3(256), 0, stream, launch);
     else

@@ -11,12 +11,9 @@ namespace hsbem::dev {
 
 inline constexpr int kMaxLeafOrder = 64;   // leaf orders with the smaller radial register table (up to kMaxBigOrder)
 inline constexpr int kMaxLeafDofs = 512;   // P1 DOFs of one leaf
-inline constexpr int kSmallFmmOrder = 32;  // smaller instantiation of the staged translations
-inline constexpr int kMaxFmmOrder = 40;    // translations with the whole d_l block staged: (2p+1)^2 doubles
-inline constexpr int kMidFmmOrder = 48;    // largest whole-block instantiation (one workgroup per CU)
-inline constexpr int kMaxWideOrder = 64;   // tiled d_l stage above kMidFmmOrder
-inline constexpr int kMaxBigOrder = 128;   // any translated expansion (reduction-tiled kernels above kMaxWideOrder)
-inline constexpr int kFmmChunk = 16;       // links per rotation chunk
+inline constexpr int kMidFmmOrder = 48;    // largest order of the FP32 translations
+inline constexpr int kMaxBigOrder = 128;   // any translated expansion
+inline constexpr int kFmmChunk = 16;       // links per chunk: the columns of two matrix tiles
 inline constexpr int kFmmJacobi = 64;      // block width served by the LDS factorisation (others: the wide path)
 
 // One leaf of the support tree with P1 DOFs. Offsets count complex values.
@@ -69,9 +66,11 @@ struct FmmLink {
     std::uint32_t source_order, target_order, rotation, axial;
 };
 
-// Consecutive links (in the direction-sorted order) sharing one rotation.
+// Consecutive links (in the sorted order) sharing one rotation and one coaxial plan, and
+// where their interleaved values start in the workspaces (complex offset).
 struct FmmChunk {
-    std::uint32_t rotation, first, count, max_order;
+    std::uint32_t rotation, first, count, pad;
+    std::uint64_t base;
 };
 
 struct FmmDestination {
@@ -83,10 +82,8 @@ struct FmmDestination {
 struct FmmTranslateLaunch {
     const FmmDestination *destinations; // of this launch
     const FmmLink *links;               // of this launch (destination order)
-    const std::uint32_t *order;         // link indices sorted by rotation
-    const FmmChunk *chunks;             // rotation chunks
-    const std::uint32_t *axial_order;   // link indices sorted by coaxial plan
-    const FmmChunk *axial_chunks;       // chunks sharing a coaxial plan (rotation field = plan)
+    const std::uint32_t *order;         // link indices sorted by rotation and coaxial plan
+    const FmmChunk *chunks;
     double *work_y, *work_z;            // link workspaces (complex)
     const FmmRotation *rotations;
     const double *small_d;
@@ -258,14 +255,13 @@ void launch_leaf_emit(const FmmLeaf *leaves, std::uint32_t leaf_count, const std
 void launch_leaf_test(const FmmLeaf *leaves, std::uint32_t leaf_count, const std::uint32_t *leaf_dofs,
                       const double *testing, const double *expansions, double *y, hipStream_t stream,
                       bool fp32 = false);
-// max_order: largest source or target order of the launch's links and rotation plans
-// (selects the tiled kernels above kMaxFmmOrder and the reduction-tiled ones above
-// kMaxWideOrder; at most kMaxBigOrder).
-// split_target: a level with few chunks spreads each chunk's degree / |m| stages over
+// max_order: largest source or target order of the launch's links and rotation plans (at
+// most kMaxBigOrder).
+// split_target: a level with few chunks spreads each chunk's degrees / orders |m| over
 // more workgroups, up to about split_target workgroups per launch (0: one per chunk).
 void launch_translate(const FmmTranslateLaunch &launch, std::uint32_t destination_count, std::uint32_t link_count,
-                      std::uint32_t chunk_count, std::uint32_t axial_chunk_count, std::uint32_t max_order,
-                      std::uint32_t split_target, hipStream_t stream);
+                      std::uint32_t chunk_count, std::uint32_t max_order, std::uint32_t split_target,
+                      hipStream_t stream);
 // blocks (zeroed, n rounded up to width) from the near CSR in tree order;
 // position[dof] = index of dof in order.
 void launch_gather_blocks(const std::uint32_t *row_offsets, const std::uint32_t *columns, const double *values,
