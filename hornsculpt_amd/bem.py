@@ -33,6 +33,11 @@ WALL, DRIVEN = 0, 1
 ACCELERATION_DENSE, ACCELERATION_FAST_MULTIPOLE = 0, 1
 
 
+class LuLimits(ctypes.Structure):
+    """Limits of the LU's shared panels and on-chip permutation (0: the library's own), and the status it starts from."""
+    _fields_ = [("panel_groups", ctypes.c_uint32), ("permute_rows", ctypes.c_uint32), ("status", ctypes.c_int32)]
+
+
 class _FmmSettings(ctypes.Structure):
     _fields_ = [("leaf_capacity", ctypes.c_uint32), ("maximum_depth", ctypes.c_uint32), ("separation", ctypes.c_double),
                 ("near_ratio", ctypes.c_double), ("accuracy_seed", ctypes.c_double),
@@ -223,6 +228,7 @@ def library() -> ctypes.CDLL:
                 "hsbem_dense_gmres": (ctypes.c_int, [P, U32, D, D, D, U32, U32, ctypes.c_double, D,
                                                      ctypes.POINTER(U32)]),
                 "hsbem_dense_lu_solve": (ctypes.c_int, [P, U32, D, U32, D]),
+                "hsbem_dense_lu_solve_limited": (ctypes.c_int, [P, U32, D, U32, D, ctypes.POINTER(LuLimits)]),
                 "hsbem_dense_lu_solve_noalloc": (ctypes.c_int, [P, U32, D, U32, D]),
                 "hsbem_server_create": (ctypes.c_int, [P, ctypes.POINTER(_ServerOptions), ctypes.POINTER(P)]),
                 "hsbem_server_destroy": (ctypes.c_int, [P]),
@@ -1436,7 +1442,8 @@ def dense_gmres(A: np.ndarray, b: np.ndarray, restart: int, maximum_iterations: 
     return x.view(np.complex128), res.value, its.value
 
 
-def dense_lu_solve(A: np.ndarray, B: np.ndarray, context: Optional[Context] = None) -> np.ndarray:
+def dense_lu_solve(A: np.ndarray, B: np.ndarray, context: Optional[Context] = None,
+                   limits: Optional[LuLimits] = None) -> np.ndarray:
     """Device partial-pivot complex LU solve of A X = B."""
     lib = library()
     ctx = context or Context.default()
@@ -1446,6 +1453,7 @@ def dense_lu_solve(A: np.ndarray, B: np.ndarray, context: Optional[Context] = No
     Bm = B.reshape(n, -1)
     Af = np.ascontiguousarray(A.T).astype(np.complex128).view(np.float64).copy()
     Bf = np.ascontiguousarray(Bm.T).view(np.float64).copy()
-    _check(lib.hsbem_dense_lu_solve(ctx.handle, n, _dptr(Af), Bm.shape[1], _dptr(Bf)))
+    _check(lib.hsbem_dense_lu_solve_limited(ctx.handle, n, _dptr(Af), Bm.shape[1], _dptr(Bf),
+                                            None if limits is None else ctypes.byref(limits)))
     X = Bf.view(np.complex128).reshape(Bm.shape[1], n).T
     return X[:, 0].copy() if single else X.copy()

@@ -193,13 +193,20 @@ inline constexpr std::size_t kNormScratchDoubles = 1024;
 // Complex LU with partial pivoting in place (A n x n), pivots n. info (cleared by the caller):
 // the first zero pivot's column + 1, or negative when the panel's workgroups gave up waiting
 // for each other (see check_lu_status). work: kLuWorkDoubles doubles of this call's own.
-inline constexpr std::size_t kLuWorkDoubles = 4 * 120 * 132 + 64;
-void lu_factor(double *A, std::uint32_t n, std::int32_t *pivots, int *info, double *work, hipStream_t stream);
+inline constexpr std::uint32_t kLuPanelGroups = 120, kLuPermuteRows = 16384;
+inline constexpr std::size_t kLuWorkDoubles = 4 * kLuPanelGroups * 132 + 64;
+// What a factorization and its solves may use of that: workgroups of one panel (panels of more
+// than 128 rows for each take one workgroup and 4 columns at a time), rows of a permutation in LDS.
+struct LuLimits {
+    std::uint32_t panel_groups = kLuPanelGroups, permute_rows = kLuPermuteRows;
+};
+void lu_factor(double *A, std::uint32_t n, std::int32_t *pivots, int *info, double *work, hipStream_t stream,
+               const LuLimits &limits = {});
 // Throws std::runtime_error for a nonzero info: `singular` and the column, or the failed wait.
 void check_lu_status(int info, const char *singular);
 // Solve with the factors for nrhs right-hand sides in place (B n x nrhs).
 void lu_solve(const double *LU, std::uint32_t n, const std::int32_t *pivots, double *B, std::uint32_t nrhs,
-              hipStream_t stream);
+              hipStream_t stream, const LuLimits &limits = {});
 
 // One Arnoldi step of up to 8 systems at once. System e (the a-th of the step is
 // which[a]) has its basis at basis + e basis_stride (column c: n complex at 2 n c; column

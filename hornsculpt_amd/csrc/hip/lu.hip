@@ -27,7 +27,7 @@ constexpr int kPanelRows = 128;    // rows per panel workgroup: two per lane
 // once. Two fit on a compute unit (512 threads, at most 128 registers), and at most four
 // streams' kernels are dispatched at a time (four hardware queues), so 4 x 120 <= 2 x 256
 // always fit; panels of more rows take the one-workgroup path below.
-constexpr std::uint32_t kMaxPanelGroups = 120;
+constexpr std::uint32_t kMaxPanelGroups = kLuPanelGroups;
 constexpr std::uint32_t kRing = 4;                      // exchange slots per workgroup
 constexpr std::uint32_t kSlotWords = 4 + 2 * kBlock;     // size, position, 64 complex entries, the pivot's inverse
 static_assert(kLuWorkDoubles == kRing * kMaxPanelGroups * kSlotWords + kBlock);
@@ -63,6 +63,20 @@ __device__ __forceinline__ u64 wait_word(const u64 *w, int *late) {
         } while (b == kEmpty);
     }
     return b;
+}
+
+// The status word: 0, the first zero pivot's column + 1, or kWaitFailed, which no pivot replaces.
+// Workgroups of one launch read and write it at the same time, on several dies.
+__device__ __forceinline__ bool gave_up(const int *info) {
+    return __hip_atomic_load(info, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < 0;
+}
+__device__ __forceinline__ void report_wait_failed(int *info) {
+    __hip_atomic_fetch_min(info, kWaitFailed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void report_zero_pivot(int *info, int column) {
+    int expected = 0;
+    __hip_atomic_compare_exchange_strong(info, &expected, column, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Every outstanding access of this wavefront has completed (stores acknowledged, loads in registers).
@@ -115,7 +129,7 @@ struct PanelShared {
     double2 inverse;         // of the pivot
     double2 factor[kPanelRows];
     std::uint32_t at;        // this group's candidate
-    std::uint32_t other_at, other_group, singular, late;
+    std::uint32_t other_at, other_group, singular, late, quit;
     std::uint32_t pivot[kBlock];
 };
 
@@ -181,8 +195,6 @@ __device__ __forceinline__ void factor_panel(double2 *A, std::uint32_t n, const 
                                              PanelShared &S) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const std::uint32_t k0 = P.k0, nb = P.nb, groups = P.groups, first = k0 + g * kPanelRows;
-    if (*P.info < 0)
-        return; // an earlier panel gave up waiting: nothing here is valid any more
     std::uint32_t pos[2];
     bool open[2];
     double2 v[2][kColumns];
@@ -196,10 +208,14 @@ __device__ __forceinline__ void factor_panel(double2 *A, std::uint32_t n, const 
         for (int c = 0; c < kColumns; ++c) // beyond n and nb: a valid entry that is never stored
             v[h][c] = mine[static_cast<std::size_t>(min(wave * kColumns + c, static_cast<int>(nb) - 1)) * n];
     }
-    if (threadIdx.x == 0)
+    if (threadIdx.x == 0) {
         S.late = 0;
+        S.quit = gave_up(P.info);
+    }
     drain_memory(); // the rows are in registers before anything of this group is published
     __syncthreads();
+    if (S.quit) // a group gave up waiting: nothing is valid any more. (One read for all wavefronts: the word
+        return; // may change between two, and those that went on would miss what the others publish.)
     auto ring_of = [&](std::uint32_t j) {
         return P.exchange + static_cast<std::size_t>((k0 + j) & (kRing - 1)) * kMaxPanelGroups * kSlotWords;
     };
@@ -290,10 +306,10 @@ __device__ __forceinline__ void factor_panel(double2 *A, std::uint32_t n, const 
             __syncthreads();
             at = S.other_at;
             late = S.late;
-            if (late) { // nothing valid will come: keep every index in range and let the caller raise
+            if (late) { // nothing valid will come: keep this group's positions in range; see lu_rows
                 at = k0 + j;
                 if (threadIdx.x == 0)
-                    *P.info = kWaitFailed;
+                    report_wait_failed(P.info);
             }
             if (moves) {
                 const std::uint32_t winner = S.other_group;
@@ -360,10 +376,12 @@ __device__ __forceinline__ void factor_panel(double2 *A, std::uint32_t n, const 
         }
     }
     __syncthreads();
+    if (threadIdx.x == 0 && S.late) // also where the last column's row did not come
+        report_wait_failed(P.info);
     if (g == 0 && threadIdx.x < nb)
         P.piv[k0 + threadIdx.x] = static_cast<std::int32_t>(S.pivot[threadIdx.x]);
-    if (g == 0 && threadIdx.x == 0 && singular && *P.info == 0)
-        *P.info = static_cast<int>(singular);
+    if (g == 0 && threadIdx.x == 0 && singular)
+        report_zero_pivot(P.info, static_cast<int>(singular));
     // v[i] is the wavefront's column (i + its active steps) mod 8; every group has read its rows long ago
     const int steps = max(0, min(static_cast<int>(nb) - wave * kColumns, kColumns));
 #pragma unroll
@@ -561,13 +579,18 @@ __device__ __forceinline__ Interchange net_interchange(std::uint32_t p, std::uin
 // whole solve is products on the matrix cores, each wavefront 16 columns that stay in
 // registers: the D layout of one product is the B layout of the next. 25 us at n = 4099,
 // bound by the latency of its dependent loads and of the chain of products.
+// Nothing is done once a panel has given up waiting: its groups then disagree about the positions
+// of their rows, so some of `moves` may never have been written. (No other kernel takes an index
+// from what a panel wrote.)
 __global__ __launch_bounds__(256) void lu_rows(double *A, std::uint32_t n, std::uint32_t k0, std::uint32_t nb,
-                                               const PanelMoves *moves) {
+                                               const PanelMoves *moves, const int *info) {
     __shared__ double2 X[kBlock][kBlock + 1];  // X[q][i] = row k0 + i of column c0 + q
     __shared__ double2 L[kBlock][kBlock + 1];  // L[c][r] = A[k0 + r][k0 + c]
     __shared__ double2 inverse[4][16][17];     // [block][c][r]
     __shared__ std::uint32_t inside[kBlock], out[kBlock], moved;
     double2 *A2 = reinterpret_cast<double2 *>(A);
+    if (gave_up(info))
+        return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const std::uint32_t left = k0 / kBlock;
     const bool right = blockIdx.x >= left;
@@ -726,8 +749,8 @@ __global__ __launch_bounds__(kPanelThreads) void lu_leaf(double *A, std::uint32_
             u[tid] = at(j + tid, p);
         if (tid == 0) {
             piv[j] = static_cast<std::int32_t>(p);
-            if (!(v > 0) && *info == 0)
-                *info = static_cast<int>(j) + 1;
+            if (!(v > 0))
+                report_zero_pivot(info, static_cast<int>(j) + 1);
         }
         __syncthreads(); // (2): every thread has p and the pivot row's leaf entries
         const double2 d = u[0];
@@ -825,7 +848,7 @@ __global__ __launch_bounds__(64) void lu_trsm(double *A, std::uint32_t n, std::u
 // permutation is composed in LDS, the net effect of 16 panels at a time found by 16
 // wavefronts and applied in order, and the entries move once: 78 us at n = 4099, where the
 // chain of single interchanges in memory below took 1.4 ms.
-constexpr std::uint32_t kPermuteRows = 16384;
+constexpr std::uint32_t kPermuteRows = kLuPermuteRows;
 __global__ __launch_bounds__(1024) void permute_rows(double *B, std::uint32_t n, const std::int32_t *piv) {
     __shared__ std::uint16_t at[kPermuteRows];
     __shared__ std::uint16_t to[16][2 * kBlock], from[16][2 * kBlock];
@@ -1056,7 +1079,9 @@ void factor_panel_leaves(double *A, std::uint32_t n, std::uint32_t k0, std::uint
 
 } // namespace
 
-void lu_factor(double *A, std::uint32_t n, std::int32_t *piv, int *info, double *work, hipStream_t stream) {
+void lu_factor(double *A, std::uint32_t n, std::int32_t *piv, int *info, double *work, hipStream_t stream,
+               const LuLimits &limits) {
+    const std::uint32_t most = std::clamp(limits.panel_groups, 1u, kMaxPanelGroups) * kPanelRows;
     // While more rows are left than the panel's workgroups hold: pairs of 32-column panels
     // P1 = [k0, e1), P2 = [e1, e2), factored on one workgroup leaf by leaf, with one rank-64
     // trailing update. P1 is factored, its interchanges applied and its U rows solved over every
@@ -1065,7 +1090,7 @@ void lu_factor(double *A, std::uint32_t n, std::int32_t *piv, int *info, double 
     // P1's update reaches P2's U rows, P2's U rows are solved, and the rows below P2 take
     // both panels' updates at once.
     std::uint32_t k0 = 0;
-    for (; n - k0 > kMaxPanelGroups * kPanelRows; k0 += 2 * kPanel) {
+    for (; n - k0 > most; k0 += 2 * kPanel) {
         const std::uint32_t e1 = k0 + kPanel, e2 = e1 + kPanel;
         factor_panel_leaves(A, n, k0, kPanel, piv, info, stream);
         hipLaunchKernelGGL(lu_swap, dim3((n + 63) / 64), dim3(64), 0, stream, A, n, k0, kPanel, piv);
@@ -1101,7 +1126,7 @@ void lu_factor(double *A, std::uint32_t n, std::int32_t *piv, int *info, double 
         const std::uint32_t nb = std::min<std::uint32_t>(kBlock, n - k0), e = k0 + nb;
         const std::uint32_t others = k0 / kBlock + (n - e + kBlock - 1) / kBlock;
         if (others)
-            hipLaunchKernelGGL(lu_rows, dim3(others), dim3(256), 0, stream, A, n, k0, nb, moves);
+            hipLaunchKernelGGL(lu_rows, dim3(others), dim3(256), 0, stream, A, n, k0, nb, moves, info);
         if (e == n)
             break;
         const std::uint32_t next = std::min<std::uint32_t>(kBlock, n - e);
@@ -1112,8 +1137,8 @@ void lu_factor(double *A, std::uint32_t n, std::int32_t *piv, int *info, double 
 }
 
 void lu_solve(const double *LU, std::uint32_t n, const std::int32_t *piv, double *B, std::uint32_t nrhs,
-              hipStream_t stream) {
-    if (n <= kPermuteRows)
+              hipStream_t stream, const LuLimits &limits) {
+    if (n <= std::min(limits.permute_rows, kPermuteRows))
         hipLaunchKernelGGL(permute_rows, dim3(nrhs), dim3(1024), 0, stream, B, n, piv);
     else
         hipLaunchKernelGGL(apply_pivots, dim3((nrhs + 63) / 64), dim3(64), 0, stream, B, n, piv, nrhs);

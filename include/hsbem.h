@@ -544,6 +544,15 @@ HSBEM_API int hsbem_dense_gmres(hsbem_context *context, uint32_t n, const double
                                 double *relative_residual, uint32_t *iterations);
 /* Partial-pivot complex LU of a dense n x n matrix and solve of nrhs right-hand sides in place. */
 HSBEM_API int hsbem_dense_lu_solve(hsbem_context *context, uint32_t n, const double *A, uint32_t nrhs, double *B);
+/* The same with the factorization's limits set by the caller, for tests and measurements of the paths
+ * that only large orders take otherwise (null, or a zero member: the library's own). */
+typedef struct hsbem_lu_limits {
+    uint32_t panel_groups; /* workgroups that may factor a panel together, 128 rows each (120) */
+    uint32_t permute_rows; /* rows whose interchanges are composed on chip (16384) */
+    int32_t status;        /* status the factorization starts from: negative as if its workgroups had given up waiting */
+} hsbem_lu_limits;
+HSBEM_API int hsbem_dense_lu_solve_limited(hsbem_context *context, uint32_t n, const double *A, uint32_t nrhs, double *B,
+                                           const hsbem_lu_limits *limits);
 /* The same LU solve on caller-owned DEVICE buffers, allocating no device memory: the pivots and the
  * singular-pivot status and the factorization's exchange words live in a static device array of the
  * library (752 KiB per GPU, held until the process ends). No counterpart in the reference: it is for callers that cannot allocate
