@@ -34,8 +34,10 @@ ACCELERATION_DENSE, ACCELERATION_FAST_MULTIPOLE = 0, 1
 
 
 class LuLimits(ctypes.Structure):
-    """Limits of the LU's shared panels and on-chip permutation (0: the library's own), and the status it starts from."""
-    _fields_ = [("panel_groups", ctypes.c_uint32), ("permute_rows", ctypes.c_uint32), ("status", ctypes.c_int32)]
+    """Limits of the LU's shared panels and on-chip permutation (0: the library's own), the status it starts from and
+    whether a second attempt is left out."""
+    _fields_ = [("panel_groups", ctypes.c_uint32), ("permute_rows", ctypes.c_uint32), ("status", ctypes.c_int32),
+                ("once", ctypes.c_uint32)]
 
 
 class _FmmSettings(ctypes.Structure):

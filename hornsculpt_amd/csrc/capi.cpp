@@ -1507,24 +1507,23 @@ int hsbem_dense_lu_solve_limited(hsbem_context *c, uint32_t n, const double *A, 
         hsbem::hip_check(hipSetDevice(c->ctx.device), "set device");
         hipStream_t s = c->ctx.stream;
         hsbem::dev::LuLimits limits;
-        const int status = given ? given->status : 0;
-        if (given && given->panel_groups)
-            limits.panel_groups = given->panel_groups;
-        if (given && given->permute_rows)
-            limits.permute_rows = given->permute_rows;
+        if (given) {
+            limits.panel_groups = given->panel_groups ? given->panel_groups : limits.panel_groups;
+            limits.permute_rows = given->permute_rows ? given->permute_rows : limits.permute_rows;
+            limits.status = given->status;
+            limits.once = given->once != 0;
+        }
         const std::size_t nn = static_cast<std::size_t>(n) * n;
         hsbem::DeviceBuffer<double> dA(2 * nn), dB(2 * static_cast<std::size_t>(n) * nrhs);
         hsbem::DeviceBuffer<std::int32_t> piv(n);
         hsbem::DeviceBuffer<int> info(1);
         hsbem::DeviceBuffer<double> work(hsbem::dev::kLuWorkDoubles);
-        hsbem::hip_check(hipMemcpyAsync(dA.data(), A, dA.bytes(), hipMemcpyHostToDevice, s), "A upload");
         hsbem::hip_check(hipMemcpyAsync(dB.data(), B, dB.bytes(), hipMemcpyHostToDevice, s), "B upload");
-        hsbem::hip_check(hipMemcpyAsync(info.data(), &status, sizeof(int), hipMemcpyHostToDevice, s), "status upload");
-        hsbem::dev::lu_factor(dA.data(), n, piv.data(), info.data(), work.data(), s, limits);
-        int code = 0;
-        hsbem::hip_check(hipMemcpyAsync(&code, info.data(), sizeof(int), hipMemcpyDeviceToHost, s), "info download");
-        hsbem::hip_check(hipStreamSynchronize(s), "LU sync");
-        hsbem::dev::check_lu_status(code, "LU factorization failed at pivot ");
+        auto upload = [&] {
+            hsbem::hip_check(hipMemcpyAsync(dA.data(), A, dA.bytes(), hipMemcpyHostToDevice, s), "A upload");
+        };
+        hsbem::dev::lu_factor(upload, dA.data(), n, piv.data(), info.data(), work.data(), s,
+                              "LU factorization failed at pivot ", limits);
         hsbem::dev::lu_solve(dA.data(), n, piv.data(), dB.data(), nrhs, s, limits);
         hsbem::hip_check(hipMemcpyAsync(B, dB.data(), dB.bytes(), hipMemcpyDeviceToHost, s), "B download");
         hsbem::hip_check(hipStreamSynchronize(s), "LU solve sync");

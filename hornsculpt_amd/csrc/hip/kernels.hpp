@@ -7,6 +7,7 @@
 #include <hip/hip_runtime_api.h>
 
 #include <cstdint>
+#include <functional>
 
 namespace hsbem::dev {
 
@@ -190,20 +191,25 @@ void launch_norm2(const double *x, std::uint32_t n, const double *weight, double
                   hipStream_t stream);
 inline constexpr std::size_t kNormScratchDoubles = 1024;
 
-// Complex LU with partial pivoting in place (A n x n), pivots n. info (cleared by the caller):
-// the first zero pivot's column + 1, or negative when the panel's workgroups gave up waiting
-// for each other (see check_lu_status). work: kLuWorkDoubles doubles of this call's own.
+// Complex LU with partial pivoting of the n x n matrix that fill() puts into A on the stream
+// (null: it is there), in place; waits for the stream. Pivots n, info one status word, work
+// kLuWorkDoubles doubles of this call's own. A zero pivot throws std::runtime_error with
+// `singular` and its column + 1.
+// The workgroups of a panel wait for each other, for at most 10 s: this process reserves them
+// among its streams, but kernels of another process may keep some from becoming resident. The
+// matrix is then filled and factored again on one workgroup per panel; without fill() or with
+// limits.once the call throws std::runtime_error.
 inline constexpr std::uint32_t kLuPanelGroups = 120, kLuPermuteRows = 16384;
 inline constexpr std::size_t kLuWorkDoubles = 4 * kLuPanelGroups * 132 + 64;
-// What a factorization and its solves may use of that: workgroups of one panel (panels of more
-// than 128 rows for each take one workgroup and 4 columns at a time), rows of a permutation in LDS.
 struct LuLimits {
-    std::uint32_t panel_groups = kLuPanelGroups, permute_rows = kLuPermuteRows;
+    std::uint32_t panel_groups = kLuPanelGroups;  // workgroups of one panel (panels of more than 128 rows
+                                                  // for each take one workgroup, 4 columns at a time)
+    std::uint32_t permute_rows = kLuPermuteRows;  // rows of a permutation composed in LDS
+    bool once{};                                  // no second attempt
+    int status{};                                 // of the first attempt when it starts
 };
-void lu_factor(double *A, std::uint32_t n, std::int32_t *pivots, int *info, double *work, hipStream_t stream,
-               const LuLimits &limits = {});
-// Throws std::runtime_error for a nonzero info: `singular` and the column, or the failed wait.
-void check_lu_status(int info, const char *singular);
+void lu_factor(const std::function<void()> &fill, double *A, std::uint32_t n, std::int32_t *pivots, int *info,
+               double *work, hipStream_t stream, const char *singular, const LuLimits &limits = {});
 // Solve with the factors for nrhs right-hand sides in place (B n x nrhs).
 void lu_solve(const double *LU, std::uint32_t n, const std::int32_t *pivots, double *B, std::uint32_t nrhs,
               hipStream_t stream, const LuLimits &limits = {});

@@ -7,9 +7,14 @@
 //              column) while the others apply the previous panel to the rest of the
 //              matrix on the FP64 matrix cores.
 //   lu_solve   64-row blocks, one launch per block and sweep.
+#include "../solver.hpp"
 #include "device.hpp"
 
 #include <algorithm>
+#include <array>
+#include <chrono>
+#include <condition_variable>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 
@@ -23,16 +28,16 @@ constexpr int kStepThreads = 512;
 constexpr int kColumns = 8;        // columns a panel wavefront holds
 constexpr int kPart = 32;          // columns of L staged at a time in an update
 constexpr int kPanelRows = 128;    // rows per panel workgroup: two per lane
-// The workgroups of a panel wait for each other, so all of them have to be resident at
-// once. Two fit on a compute unit (512 threads, at most 128 registers), and at most four
-// streams' kernels are dispatched at a time (four hardware queues), so 4 x 120 <= 2 x 256
-// always fit; panels of more rows take the one-workgroup path below.
+// The workgroups of a panel wait for each other, so all of them have to be resident at once:
+// each factorization reserves them (PanelGroups below) and takes panels of more rows than it
+// got on one workgroup. Most at a time: the whole of a matrix of 15,360 rows, on half of the
+// 256 compute units.
 constexpr std::uint32_t kMaxPanelGroups = kLuPanelGroups;
 constexpr std::uint32_t kRing = 4;                      // exchange slots per workgroup
 constexpr std::uint32_t kSlotWords = 4 + 2 * kBlock;     // size, position, 64 complex entries, the pivot's inverse
 static_assert(kLuWorkDoubles == kRing * kMaxPanelGroups * kSlotWords + kBlock);
 constexpr u64 kEmpty = ~0ull;                           // an exchange word nobody has written
-constexpr u64 kWaitTicks = 1000000000ull;               // 10 s of the 100 MHz clock
+constexpr u64 kWaitTicks = 1000000000ull;               // 10 s of the 100 MHz clock: only other processes can cause it
 constexpr int kWaitFailed = -1;                         // info: a panel workgroup waited that long
 
 
@@ -528,6 +533,8 @@ __global__ __launch_bounds__(256) void lu_update_small(double *A, std::uint32_t 
             A2[static_cast<std::size_t>(c) * n + r] = double2{cold[v].x - (re[v] + re2[v]), cold[v].y - (im[v] + im2[v])};
     }
 }
+
+__global__ void set_status(int *info, int value) { *info = value; }
 
 __global__ void clear_exchange(u64 *exchange, std::uint32_t words) {
     const std::uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1038,14 +1045,73 @@ __global__ __launch_bounds__(256) void solve_step(const double *LU, std::uint32_
 
 } // namespace
 
-void check_lu_status(int info, const char *singular) {
-    if (info == kWaitFailed)
-        throw std::runtime_error("LU factorization: the panel's workgroups did not all become resident");
-    if (info)
-        throw std::runtime_error(singular + std::to_string(info));
+namespace {
+
+// Panel workgroups of this process that may wait for each other, per device: one per compute
+// unit. (Two fit on an empty one, but a workgroup that was placed beside another kernel's may
+// leave its LDS in two parts, neither large enough for a second.) Counted in whole rounds of
+// the dies that take workgroups in turn, so that no die gets more than its compute units.
+constexpr std::uint32_t kDies = 8;
+constexpr int kMaxDevices = 64;
+struct PanelBudget {
+    std::mutex mutex;
+    std::condition_variable freed;
+    std::uint32_t capacity{}, used{};
+};
+
+PanelBudget &budget_of(int device) {
+    static std::array<PanelBudget, kMaxDevices> budgets;
+    if (device < 0 || device >= kMaxDevices)
+        throw std::invalid_argument("device ordinal out of range for the LU factorization");
+    PanelBudget &b = budgets[device];
+    std::lock_guard lock(b.mutex);
+    if (!b.capacity) {
+        int units = 0, resident = 0;
+        hip_check(hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, device), "compute units");
+        hip_check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, lu_step, kStepThreads, 0), "LU occupancy");
+        b.capacity = resident > 0 ? std::max(units, 1) : 1;
+    }
+    return b;
 }
 
-namespace {
+// The workgroups that a factorization of n rows may use for a panel, reserved until this object
+// goes. Waits for others to finish theirs, but not for ever: after two seconds it takes what
+// is left, if need be one, which waits for nobody.
+class PanelGroups {
+  public:
+    PanelGroups(std::uint32_t n, std::uint32_t limit) {
+        const std::uint32_t wanted = std::min((n + kPanelRows - 1) / kPanelRows, std::clamp(limit, 1u, kMaxPanelGroups));
+        if (wanted <= 1)
+            return;
+        int device = 0;
+        hip_check(hipGetDevice(&device), "current device");
+        budget_ = &budget_of(device);
+        std::unique_lock lock(budget_->mutex);
+        const std::uint32_t whole = std::min((wanted + kDies - 1) / kDies * kDies, budget_->capacity);
+        budget_->freed.wait_for(lock, std::chrono::seconds(2),
+                                [&] { return budget_->used + whole <= budget_->capacity; });
+        const std::uint32_t left = budget_->capacity - budget_->used;
+        reserved_ = left >= whole ? whole : left / kDies * kDies;
+        count_ = std::clamp(reserved_, 1u, wanted);
+        budget_->used += reserved_;
+    }
+    ~PanelGroups() {
+        if (!reserved_)
+            return;
+        {
+            std::lock_guard lock(budget_->mutex);
+            budget_->used -= reserved_;
+        }
+        budget_->freed.notify_all();
+    }
+    PanelGroups(const PanelGroups &) = delete;
+    PanelGroups &operator=(const PanelGroups &) = delete;
+    std::uint32_t count() const { return count_; }
+
+  private:
+    PanelBudget *budget_{};
+    std::uint32_t reserved_{}, count_{1};
+};
 
 void step(double *A, std::uint32_t n, const PanelArgs &P, const UpdateArgs &U, hipStream_t stream) {
     const std::uint32_t rows = (U.r_end - U.r_begin + kBlock - 1) / kBlock,
@@ -1077,11 +1143,10 @@ void factor_panel_leaves(double *A, std::uint32_t n, std::uint32_t k0, std::uint
     }
 }
 
-} // namespace
-
-void lu_factor(double *A, std::uint32_t n, std::int32_t *piv, int *info, double *work, hipStream_t stream,
-               const LuLimits &limits) {
-    const std::uint32_t most = std::clamp(limits.panel_groups, 1u, kMaxPanelGroups) * kPanelRows;
+// The launches of a factorization whose panels may have `groups` workgroups.
+void factor_launches(double *A, std::uint32_t n, std::int32_t *piv, int *info, double *work, std::uint32_t groups,
+                     hipStream_t stream) {
+    const std::uint32_t most = groups * kPanelRows;
     // While more rows are left than the panel's workgroups hold: pairs of 32-column panels
     // P1 = [k0, e1), P2 = [e1, e2), factored on one workgroup leaf by leaf, with one rank-64
     // trailing update. P1 is factored, its interchanges applied and its U rows solved over every
@@ -1134,6 +1199,30 @@ void lu_factor(double *A, std::uint32_t n, std::int32_t *piv, int *info, double 
                            stream, A, n, UpdateArgs{k0, nb, e, n, e, e + next});
         step(A, n, panel(e), UpdateArgs{k0, nb, e, n, e + next, n}, stream);
     }
+}
+
+} // namespace
+
+void lu_factor(const std::function<void()> &fill, double *A, std::uint32_t n, std::int32_t *piv, int *info, double *work,
+               hipStream_t stream, const char *singular, const LuLimits &limits) {
+    int code = 0;
+    auto attempt = [&](std::uint32_t most, int status) {
+        if (fill)
+            fill();
+        const PanelGroups groups(n, most); // until the stream has been waited for
+        hipLaunchKernelGGL(set_status, dim3(1), dim3(1), 0, stream, info, status);
+        hip_check(hipGetLastError(), "LU status");
+        factor_launches(A, n, piv, info, work, groups.count(), stream);
+        hip_check(hipMemcpyAsync(&code, info, sizeof(int), hipMemcpyDeviceToHost, stream), "LU status download");
+        hip_check(hipStreamSynchronize(stream), "LU sync");
+    };
+    attempt(limits.panel_groups, limits.status);
+    if (code == kWaitFailed && fill && !limits.once)
+        attempt(1, 0);
+    if (code == kWaitFailed)
+        throw std::runtime_error("LU factorization: the panel's workgroups did not all become resident");
+    if (code)
+        throw std::runtime_error(singular + std::to_string(code));
 }
 
 void lu_solve(const double *LU, std::uint32_t n, const std::int32_t *piv, double *B, std::uint32_t nrhs,

@@ -56,10 +56,6 @@ unsigned char *device_scratch(int device) {
     return scratch_address[device];
 }
 
-// Clears the status word with a kernel rather than a memset node, so a
-// captured stream records no memset.
-__global__ void clear_status(int *status) { *status = 0; }
-
 } // namespace
 
 std::uint32_t noalloc_lu_max_order() { return kNoAllocMaxOrder; }
@@ -75,13 +71,8 @@ void dense_lu_solve_noalloc(int device, hipStream_t stream, std::uint32_t n, dou
     unsigned char *base = device_scratch(device);
     int *status = reinterpret_cast<int *>(base);
     auto *pivots = reinterpret_cast<std::int32_t *>(base + kStatusBytes);
-    hipLaunchKernelGGL(clear_status, dim3(1), dim3(1), 0, stream, status);
-    hip_check(hipGetLastError(), "status clear");
-    lu_factor(A, n, pivots, status, reinterpret_cast<double *>(base + kExchangeOffset), stream);
-    int code = 0;
-    hip_check(hipMemcpyAsync(&code, status, sizeof(int), hipMemcpyDeviceToHost, stream), "status download");
-    hip_check(hipStreamSynchronize(stream), "LU sync");
-    check_lu_status(code, "LU factorization failed at pivot ");
+    lu_factor(nullptr, A, n, pivots, status, reinterpret_cast<double *>(base + kExchangeOffset), stream,
+              "LU factorization failed at pivot ");
     lu_solve(A, n, pivots, B, nrhs, stream);
     hip_check(hipStreamSynchronize(stream), "LU solve sync");
 }

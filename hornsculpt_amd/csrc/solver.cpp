@@ -1752,15 +1752,13 @@ FrequencyResult MeshSolver::solve_frequency(const PreparedRequest &P, std::size_
     phase(3);
     const auto t_solve = Clock::now();
     if (solver_kind == 0) {
-        hip_check(hipMemcpyAsync(ws.LU.data(), ws.A.data(), ws.A.bytes(), hipMemcpyDeviceToDevice, s), "LU copy");
-        hip_check(hipMemsetAsync(ws.error.data(), 0, sizeof(int), s), "clear info");
+        auto copy = [&] {
+            hip_check(hipMemcpyAsync(ws.LU.data(), ws.A.data(), ws.A.bytes(), hipMemcpyDeviceToDevice, s), "LU copy");
+        };
         const auto t_f = Clock::now();
-        dev::lu_factor(ws.LU.data(), nv, ws.pivots.data(), ws.error.data(), ws.scratch.data(), s);
-        int info = 0;
-        hip_check(hipMemcpyAsync(&info, ws.error.data(), sizeof(int), hipMemcpyDeviceToHost, s), "info");
-        hip_check(hipStreamSynchronize(s), "LU sync");
+        dev::lu_factor(copy, ws.LU.data(), nv, ws.pivots.data(), ws.error.data(), ws.scratch.data(), s,
+                       "LU factorization hit a zero pivot at column ");
         fr.ms[2] = ms_since(t_f);
-        dev::check_lu_status(info, "LU factorization hit a zero pivot at column ");
         const auto t_t = Clock::now();
         hip_check(hipMemcpyAsync(ws.x.data(), ws.rhs.data(), ws.rhs.bytes(), hipMemcpyDeviceToDevice, s), "rhs copy");
         dev::lu_solve(ws.LU.data(), nv, ws.pivots.data(), ws.x.data(), ne, s);

@@ -542,14 +542,19 @@ HSBEM_API int hsbem_assemble(hsbem_mesh *mesh, const hsbem_numerics *numerics, d
 HSBEM_API int hsbem_dense_gmres(hsbem_context *context, uint32_t n, const double *A, const double *b, double *x,
                                 uint32_t restart, uint32_t maximum_iterations, double tolerance,
                                 double *relative_residual, uint32_t *iterations);
-/* Partial-pivot complex LU of a dense n x n matrix and solve of nrhs right-hand sides in place. */
+/* Partial-pivot complex LU of a dense n x n matrix and solve of nrhs right-hand sides in place.
+ * Several workgroups factor a panel together and wait for each other. One process reserves them among
+ * its streams (one per compute unit; a factorization that would need more waits up to two seconds, then
+ * uses fewer). Another process's kernels on the same GPU can keep some of them from starting: after 10 s
+ * the matrix is factored again with one workgroup per panel, here and in every solve. */
 HSBEM_API int hsbem_dense_lu_solve(hsbem_context *context, uint32_t n, const double *A, uint32_t nrhs, double *B);
 /* The same with the factorization's limits set by the caller, for tests and measurements of the paths
  * that only large orders take otherwise (null, or a zero member: the library's own). */
 typedef struct hsbem_lu_limits {
     uint32_t panel_groups; /* workgroups that may factor a panel together, 128 rows each (120) */
     uint32_t permute_rows; /* rows whose interchanges are composed on chip (16384) */
-    int32_t status;        /* status the factorization starts from: negative as if its workgroups had given up waiting */
+    int32_t status;        /* status the factorization starts from: -1 as if its workgroups had given up waiting */
+    uint32_t once;         /* nonzero: no second attempt after that, the call fails instead */
 } hsbem_lu_limits;
 HSBEM_API int hsbem_dense_lu_solve_limited(hsbem_context *context, uint32_t n, const double *A, uint32_t nrhs, double *B,
                                            const hsbem_lu_limits *limits);
@@ -560,7 +565,9 @@ HSBEM_API int hsbem_dense_lu_solve_limited(hsbem_context *context, uint32_t n, c
  * complex n x n, interleaved re/im) is overwritten by its LU factors and B (n x nrhs) by the
  * solutions; n <= 65536 (larger orders are refused with HSBEM_INVALID_ARGUMENT). The work runs on the
  * context's stream, which is synchronised before the call returns; the caller orders its own writes
- * of A and B before the call. Calls that overlap on one GPU share its array and race. */
+ * of A and B before the call. Calls that overlap on one GPU share its array and race. There is no copy of
+ * A to start again from: where the panel's workgroups give up waiting for each other (see
+ * hsbem_dense_lu_solve; only other processes on the GPU can cause it) the call fails. */
 HSBEM_API int hsbem_dense_lu_solve_noalloc(hsbem_context *context, uint32_t n, double *A, uint32_t nrhs, double *B);
 
 #ifdef __cplusplus

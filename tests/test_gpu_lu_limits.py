@@ -3,7 +3,11 @@ orders with that number set by the caller.
 
 A factorization whose workgroups have given up waiting for each other (its status word
 starts negative) does nothing more with what the panel should have left behind: every kernel
-ends, the call reports it and the next one is not affected."""
+ends, and the call factors its matrix again on one workgroup per panel, or reports it where
+that is left out. Factorizations that together want more workgroups than the GPU has wait for
+each other."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -28,5 +32,30 @@ def _check(A, X, B):
 def test_given_up_panel_is_reported(n, groups):
     A, B = _system(n, 2)
     with pytest.raises(RuntimeError, match="resident"):
-        bem.dense_lu_solve(A, B, limits=bem.LuLimits(panel_groups=groups, status=-1))
+        bem.dense_lu_solve(A, B, limits=bem.LuLimits(panel_groups=groups, status=-1, once=1))
     _check(A, bem.dense_lu_solve(A, B), B)
+
+
+@pytest.mark.parametrize("n", [64, 129, 321, 1089])
+def test_given_up_panel_is_factored_again(n):
+    A, B = _system(n, 3)
+    _check(A, bem.dense_lu_solve(A, B, limits=bem.LuLimits(status=-1)), B)
+
+
+def test_concurrent_factorizations():
+    # 10 streams at once, 40 panel workgroups each: more than the GPU has compute units
+    A, B = _system(4099, 1)
+    out = [None] * 10
+
+    def work(i):
+        out[i] = bem.dense_lu_solve(A, B * (i + 1), bem.Context())
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(out))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    _check(A, out[0], B)
+    for i, x in enumerate(out):
+        # the same system up to the order of the sums: a random matrix of this order has a condition below 1e6
+        assert np.linalg.norm(x - out[0] * (i + 1)) <= 1e-9 * np.linalg.norm(x)
