@@ -599,27 +599,50 @@ __device__ __forceinline__ void tile_pair(std::uint32_t p, const TilePairs &t, s
     }
 }
 
+// KIND: the tile list holds far tiles only (A < B, every pair disjoint, not near, at least three
+// edges apart), where a pair takes degree 4 up to k h = 0.5 and degree 6 above: kFar4 tiles have
+// only pairs of degree 4 at this wavenumber, kFar46 tiles both. kGeneral tiles check each pair.
+enum TileKind : int { kGeneral = 0, kFar4 = 1, kFar46 = 2 };
+
 // Far tiles accumulate their node tiles in fixed point with integer LDS atomics
 // (ds_add_u32 / ds_add_u64; the floating-point LDS atomics are several times slower
 // on gfx950 and bound the far tiles otherwise). The scale is a power of two chosen per
 // tile from a bound on every contribution (see far_scale), so no sum can overflow;
-// the resolution is about 2^-30 (FP32 form) or 2^-51 (FP64 form) of that bound.
-template <class R> struct FixedOf;
-template <> struct FixedOf<float> {
-    using type = int;
-    static constexpr double headroom = 1073741824.0; // 2^30
-};
-template <> struct FixedOf<double> {
-    using type = long long;
-    static constexpr double headroom = 2251799813685248.0; // 2^51: rint by the 1.5 * 2^52 shift
+// the resolution is about 2^-30 (FP32 form) or 2^-51 (FP64 form) of that bound on kFar4 tiles.
+// The bound is that of the tile's closest and largest pairs and a typical entry lies about 2^11
+// below it, so kFar46 tiles take 64 bits in both forms, 2^-54 and 2^-62: entries as exact as
+// sums in FP32 and FP64 (at the median FP32 2^-30 gave 3.4e-6 instead of 4.4e-7, FP64 2^-51
+// 1.5e-12 instead of 1e-15). A mixed solve of 20.7k triangles at 8 kHz takes 61.9 ms this way, 64.2 ms
+// with FP32 sums by LDS atomics, and 55.5 ms with the 32 bits that are not enough, in cells that
+// leave room for two workgroups on a compute unit; in the FP64 form the three are the same.
+template <class R, TileKind KIND> struct TileSum {
+    static constexpr bool fixed = KIND != kGeneral, fp32 = sizeof(R) == 4;
+    using Cell = std::conditional_t<!fixed, R, std::conditional_t<fp32 && KIND == kFar4, int, long long>>;
+    static constexpr double headroom = KIND == kFar4 ? (fp32 ? 0x1p30 : 0x1p51) : fp32 ? 0x1p54 : 0x1p62;
+    static constexpr int exponent = fp32 ? 100 : 900; // of the scale, within the range of R
+    // workgroups of 16 wavefronts where the 64-bit cells leave room for one on a compute unit
+    static constexpr int threads = fp32 && KIND == kFar46 ? 2 * kTileThreads : kTileThreads;
 };
 
 // rint(x) as a 64-bit integer for |x| < 2^51: adding 1.5 * 2^52 leaves the rounded
 // integer in the low mantissa bits (round to nearest even), read back as an integer
 // difference of the two bit patterns.
 __device__ __forceinline__ long long rint_to_int64(double x) {
-    constexpr double shift = 6755399441055744.0; // 1.5 * 2^52
+    constexpr double shift = 0x1.8p52;
     return __double_as_longlong(x + shift) - __double_as_longlong(shift);
+}
+
+// The same for |x| <= 2^62 and 2^54: the multiple of 2^11 or 2^24 first, then what is left of x
+// (exact).
+__device__ __forceinline__ long long rint_to_int64_wide(double x) {
+    constexpr double shift = 0x1.8p63;
+    const double up = x + shift;
+    const long long high = __double_as_longlong(up) - __double_as_longlong(shift);
+    return high * 2048 + rint_to_int64(x - (up - shift));
+}
+__device__ __forceinline__ long long rint_to_int64_wide(float x) {
+    const float high = rintf(x * 0x1p-24f);
+    return static_cast<long long>(static_cast<int>(high)) * 16777216 + static_cast<int>(rintf(fmaf(high, -0x1p24f, x)));
 }
 
 // Scale of a far tile (clusters fa, fb: kClusterFar doubles each). Every sample
@@ -630,7 +653,7 @@ __device__ __forceinline__ long long rint_to_int64(double x) {
 // rule weight sum); at most val_a * val_b pairs add to one entry. Returns false
 // when the bound is not usable (the caller raises ERR_RANGE).
 __device__ __forceinline__ bool far_scale(const double *fa, const double *fb, double k, double weight_sum,
-                                          double headroom, double &scale, double &limit) {
+                                          double headroom, int exponent, double &scale, double &limit) {
     const double dx = fa[0] - fb[0], dy = fa[1] - fb[1], dz = fa[2] - fb[2];
     const double r = (sqrt(dx * dx + dy * dy + dz * dz) - fa[3] - fb[3]) * (1 - 1e-9);
     const double wq = 4.0 * fa[4] * fb[4] * 0.07957747154594766788 * weight_sum * weight_sum;
@@ -640,30 +663,29 @@ __device__ __forceinline__ bool far_scale(const double *fa, const double *fb, do
         return false;
     int e = 0;
     frexp(headroom / total, &e);
-    e = min(max(e - 1, -100), 100);
+    e = min(max(e - 1, -exponent), exponent);
     scale = ldexp(1.0, e);
     limit = per * scale;
     return true;
 }
 
-// KIND: the tile list holds far tiles only (A < B, every pair disjoint, not near, at least three
-// edges apart), where a pair takes degree 4 up to k h = 0.5 and degree 6 above: kFar4 tiles have
-// only pairs of degree 4 at this wavenumber, kFar46 tiles both. kGeneral tiles check each pair
-// (20.7k-triangle horn at 8 kHz, all far tiles as kGeneral ones before: 49.2 -> 37.9 ms FP32,
+// Far tiles as kinds of their own (20.7k-triangle horn at 8 kHz, all far tiles as kGeneral ones before: 49.2 -> 37.9 ms FP32,
 // 103 -> 96.6 ms FP64; at 4 kHz 51.2 -> 41.3 and 113 -> 102.7 ms; at 1 kHz 20.2 -> 19.5 and 48.5 ->
 // 41.2 ms). Occupancy: FP32, two 512-thread workgroups per CU
 // (LDS <= 80 KiB, VGPRs <= 128); FP64, one (LDS <= 160 KiB, VGPRs <= 256).
-enum TileKind : int { kGeneral = 0, kFar4 = 1, kFar46 = 2 };
 
 // Pairs that a general tile sorts at a time: what the LDS has left.
 template <class R> constexpr int kSortedPairs = sizeof(R) == 4 ? 2048 : 4096;
 
 template <class R, TileKind KIND>
-__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 2)))
+__global__ __launch_bounds__((TileSum<R, KIND>::threads)) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 2)))
 void regular_tiles_sym(AssemblyArgs args, ClusterView cl, NearView near, const double *rules,
                        const std::uint32_t *tiles, TileRules<R> fixed, std::uint32_t trial_shift) {
-    __shared__ R tab[kTileNodes * kStrideAB];
-    __shared__ R tba[kTileNodes * kStrideBA];
+    using Sum = TileSum<R, KIND>;
+    using Cell = typename Sum::Cell;
+    constexpr int kThreads = Sum::threads;
+    __shared__ Cell tab[kTileNodes * kStrideAB];
+    __shared__ Cell tba[kTileNodes * kStrideBA];
     __shared__ double sv0[2][3][kTilePanels];
     __shared__ R sgf[2][kSymFields][kTilePanels];
     __shared__ std::uint32_t snode[2][3][KIND == kGeneral ? kTilePanels : 1]; // for the touching test
@@ -685,13 +707,13 @@ void regular_tiles_sym(AssemblyArgs args, ClusterView cl, NearView near, const d
     const PanelView &pv = args.panels;
     const int tid = threadIdx.x;
 
-    for (int e = tid; e < kTileNodes * kStrideAB; e += kTileThreads)
-        tab[e] = R(0);
+    for (int e = tid; e < kTileNodes * kStrideAB; e += kThreads)
+        tab[e] = Cell(0);
     if (!diag)
-        for (int e = tid; e < kTileNodes * kStrideBA; e += kTileThreads)
-            tba[e] = R(0);
+        for (int e = tid; e < kTileNodes * kStrideBA; e += kThreads)
+            tba[e] = Cell(0);
     constexpr int kLoaded = G_E1 + kSymFields;
-    for (int e = tid; e < 2 * kLoaded * kTilePanels; e += kTileThreads) {
+    for (int e = tid; e < 2 * kLoaded * kTilePanels; e += kThreads) {
         const int c = e / (kLoaded * kTilePanels), f = (e / kTilePanels) % kLoaded, p = e % kTilePanels;
         if (p < static_cast<int>(c ? nS : nT)) {
             const double v = g_at(pv.geo, f - G_E1 == F_AREA ? G_AREA : f, pv.nt, cl.panels[(c ? s0 : t0) + p]);
@@ -701,7 +723,7 @@ void regular_tiles_sym(AssemblyArgs args, ClusterView cl, NearView near, const d
                 sgf[c][f - G_E1][p] = static_cast<R>(v);
         }
     }
-    for (int e = tid; e < 2 * kTilePanels; e += kTileThreads) {
+    for (int e = tid; e < 2 * kTilePanels; e += kThreads) {
         const int c = e / kTilePanels, p = e % kTilePanels;
         if (p < static_cast<int>(c ? nS : nT)) {
             const std::uint32_t id = cl.panels[(c ? s0 : t0) + p];
@@ -723,36 +745,34 @@ void regular_tiles_sym(AssemblyArgs args, ClusterView cl, NearView near, const d
     const R kf = static_cast<R>(k), inv_k = static_cast<R>(1.0 / k), k_rev = static_cast<R>(k * 0.15915494309189533577);
     const std::uint32_t pairs = nT * nS;
     const TilePairs order = tile_pairs(nT, nS, trial_shift);
-    using Fixed = typename FixedOf<R>::type;
     R fixed_scale = 1, fixed_limit = 0, largest = 0;
     bool out_of_range = false;
-    if constexpr (FAR) {
+    if constexpr (Sum::fixed) {
         double weight_sum = 0, scale = 1, limit = 0;
 #pragma unroll
         for (int q = 0; q < 6; ++q)
             weight_sum += static_cast<double>(fixed.d4[q][R_W]);
-        if (far_scale(cl.far + kClusterFar * ca, cl.far + kClusterFar * cb, k, weight_sum, FixedOf<R>::headroom,
-                      scale, limit)) {
+        if (far_scale(cl.far + kClusterFar * ca, cl.far + kClusterFar * cb, k, weight_sum, Sum::headroom,
+                      Sum::exponent, scale, limit)) {
             fixed_scale = static_cast<R>(scale);
             fixed_limit = static_cast<R>(limit);
         } else {
             out_of_range = true;
         }
     }
-    // One node-tile update: fixed point on far tiles (the sums carry the scale; |v| within the tile bound, else
-    // ERR_RANGE; a non-finite v is reported through `bad`), a floating-point LDS
-    // atomic otherwise.
-    auto tile_add = [&](R *slot, R v) {
-        if constexpr (FAR) {
-            largest = fmax(largest, fabs(v));
-            if constexpr (sizeof(R) == 4)
-                atomicAdd(reinterpret_cast<int *>(slot), static_cast<int>(rintf(v)));
-            else
-                atomicAdd(reinterpret_cast<unsigned long long *>(slot),
-                          static_cast<unsigned long long>(rint_to_int64(v)));
-        } else {
+    // One node-tile update: in fixed point (the sums carry the scale; |v| within the tile bound, else
+    // ERR_RANGE; a non-finite v is reported through `bad`) or a floating-point LDS atomic.
+    auto tile_add = [&](Cell *slot, R v) {
+        if constexpr (!Sum::fixed) {
             unsafeAtomicAdd(slot, v);
+            return;
         }
+        largest = fmax(largest, fabs(v));
+        if constexpr (std::is_same_v<Cell, int>)
+            atomicAdd(slot, static_cast<int>(rintf(v)));
+        else if constexpr (Sum::fixed)
+            atomicAdd(reinterpret_cast<unsigned long long *>(slot),
+                      static_cast<unsigned long long>(KIND == kFar46 ? rint_to_int64_wide(v) : rint_to_int64(v)));
     };
     unsigned long long counted = 0;
     bool bad = false;
@@ -833,11 +853,11 @@ void regular_tiles_sym(AssemblyArgs args, ClusterView cl, NearView near, const d
                 const R cc = curls[i][j];
                 const CplxT<R> tg = T.g[i][j], tp = T.p[i][j], tq = T.q[i][j];
                 // (t, s): row = t's node i (A), column = s's node j (B)
-                R *ts = tab + b * kStrideAB + 2 * a;
+                Cell *ts = tab + b * kStrideAB + 2 * a;
                 tile_add(ts, -tp.re - knn * tg.im + Gk.im * cc);
                 tile_add(ts + 1, -tp.im + knn * tg.re - Gk.re * cc);
                 // (s, t): row = s's node j (B), column = t's node i (A)
-                R *st = diag ? tab + a * kStrideAB + 2 * b : tba + a * kStrideBA + 2 * b;
+                Cell *st = diag ? tab + a * kStrideAB + 2 * b : tba + a * kStrideBA + 2 * b;
                 tile_add(st, -tq.re - knn * tg.im + Gk.im * cc);
                 tile_add(st + 1, -tq.im + knn * tg.re - Gk.re * cc);
             }
@@ -872,7 +892,7 @@ void regular_tiles_sym(AssemblyArgs args, ClusterView cl, NearView near, const d
         }
     };
     if constexpr (FAR) {
-        for (std::uint32_t p = tid + kTileThreads * blockIdx.y; p < pairs; p += kTileThreads * gridDim.y) {
+        for (std::uint32_t p = tid + kThreads * blockIdx.y; p < pairs; p += kThreads * gridDim.y) {
             std::uint32_t lt, ls;
             tile_pair(p, order, lt, ls);
             const SymPair<R> c = make_pair(lt, ls);
@@ -996,20 +1016,20 @@ void regular_tiles_sym(AssemblyArgs args, ClusterView cl, NearView near, const d
             atomicAdd(args.samples, v);
     }
     __syncthreads();
-    if (out_of_range || (FAR && largest > fixed_limit))
+    if (out_of_range || (Sum::fixed && largest > fixed_limit))
         atomicExch(args.error, ERR_RANGE);
     R *A = matrix_of<R>(args);
-    // a far tile's entries back from fixed point (exact power-of-two scaling)
+    // a tile's entries back from fixed point (power-of-two scaling)
     const R unscale = R(1) / fixed_scale;
-    auto entry = [&](const R *slot) {
-        if constexpr (FAR)
-            return static_cast<R>(*reinterpret_cast<const Fixed *>(slot)) * unscale;
+    auto entry = [&](const Cell *slot) {
+        if constexpr (Sum::fixed)
+            return static_cast<R>(*slot) * unscale;
         else
             return *slot;
     };
     // one part (re or im) per lane, so that a wavefront's atomics cover consecutive words
-    auto flush = [&](const R *tile, std::uint32_t r0, std::uint32_t nr, std::uint32_t c0, std::uint32_t nc, int side) {
-        for (std::uint32_t c = tid / 64; c < nc; c += kTileThreads / 64) {
+    auto flush = [&](const Cell *tile, std::uint32_t r0, std::uint32_t nr, std::uint32_t c0, std::uint32_t nc, int side) {
+        for (std::uint32_t c = tid / 64; c < nc; c += kThreads / 64) {
             const std::uint32_t col = cl.nodes[c0 + c];
             for (std::uint32_t q = tid & 63; q < 2 * nr; q += 64) {
                 const R v = entry(tile + c * kStrideAB + q);
@@ -1689,22 +1709,23 @@ void launch_regular(const AssemblyLaunch &L, hipStream_t stream) {
         return block == 4 ? 2u : block == 8 ? 3u : 4u;
     };
     const std::uint32_t shift = shift_of(L.trial_block), far_shift = shift_of(L.far_trial_block);
-    auto launch = [&](auto kernel, std::uint32_t first, std::uint32_t count, const auto &fixed, std::uint32_t block) {
+    auto launch = [&](auto kernel, int threads, std::uint32_t first, std::uint32_t count, const auto &fixed,
+                      std::uint32_t block) {
         if (count)
-            hipLaunchKernelGGL(kernel, dim3(count, parts_of(count)), dim3(kTileThreads), 0, stream, L.args, L.clusters,
+            hipLaunchKernelGGL(kernel, dim3(count, parts_of(count)), dim3(threads), 0, stream, L.args, L.clusters,
                                L.near, L.rules, L.tiles + 2 * static_cast<std::size_t>(first), fixed, block);
     };
     const std::uint32_t far46 = L.separated_tiles - L.far_tiles;
     if (L.args.A32) {
         static const TileRules<float> fixed = make_tile_rules<float>();
-        launch(regular_tiles_sym<float, kFar4>, 0, L.far_tiles, fixed, far_shift);
-        launch(regular_tiles_sym<float, kFar46>, L.far_tiles, far46, fixed, far_shift);
-        launch(regular_tiles_sym<float, kGeneral>, L.separated_tiles, general, fixed, shift);
+        launch(regular_tiles_sym<float, kFar4>, TileSum<float, kFar4>::threads, 0, L.far_tiles, fixed, far_shift);
+        launch(regular_tiles_sym<float, kFar46>, TileSum<float, kFar46>::threads, L.far_tiles, far46, fixed, far_shift);
+        launch(regular_tiles_sym<float, kGeneral>, TileSum<float, kGeneral>::threads, L.separated_tiles, general, fixed, shift);
     } else {
         static const TileRules<double> fixed = make_tile_rules<double>();
-        launch(regular_tiles_sym<double, kFar4>, 0, L.far_tiles, fixed, far_shift);
-        launch(regular_tiles_sym<double, kFar46>, L.far_tiles, far46, fixed, far_shift);
-        launch(regular_tiles_sym<double, kGeneral>, L.separated_tiles, general, fixed, shift);
+        launch(regular_tiles_sym<double, kFar4>, TileSum<double, kFar4>::threads, 0, L.far_tiles, fixed, far_shift);
+        launch(regular_tiles_sym<double, kFar46>, TileSum<double, kFar46>::threads, L.far_tiles, far46, fixed, far_shift);
+        launch(regular_tiles_sym<double, kGeneral>, TileSum<double, kGeneral>::threads, L.separated_tiles, general, fixed, shift);
     }
 }
 
