@@ -1383,15 +1383,16 @@ __global__ __launch_bounds__(256) void near_patches(AssemblyArgs args, const Nea
 // Bound by atomics when each patch adds its 18 entries to the matrix itself: the patches of
 // a pair, and pairs with common nodes, hit the same entries. Here they add to LDS node tiles
 // as the regular pairs do ([B node][A node] for a test panel in A, [A node][B node] for one
-// in B) and each touched entry goes to the matrix once per chunk. A chunk with few patches
+// in B) and each touched entry goes to the matrix once per chunk. Moments and sums of entries are
+// in R; an entry's contribution, with its curl term and its row's scale, is formed in FP64 and
+// rounded once. A chunk with few patches
 // gives a patch to several threads, each a part of its test points. 1.5k-triangle horn
-// (498 thousand patches): 2.20 -> 0.43 ms FP32, 2.16 -> 0.88 ms FP64; 20.7k triangles (1.31
-// million): 3.3 -> 1.09 and 3.2 -> 2.6 ms, now bound by the samples.
+// (498 thousand patches): 2.20 -> 0.40 ms FP32, 2.16 -> 0.88 ms FP64; 20.7k triangles (1.31
+// million): 3.3 -> 1.05 and 3.2 -> 2.7 ms, now bound by the samples.
 template <class R>
 __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 2)))
-void near_tiles(AssemblyArgs args, ClusterView cl, const NearChunk *chunks,
-                                                           const NearPatchItem *items, const PairPatch *patches,
-                                                           const double *rules, TileRules<R> fixed) {
+void near_tiles(AssemblyArgs args, ClusterView cl, const NearChunk *chunks, const NearPatchItem *items,
+                const PairPatch *patches, const double *rules, TileRules<R> fixed) {
     __shared__ R tab[kTileNodes * kStrideAB];
     __shared__ R tba[kTileNodes * kStrideBA];
     __shared__ R srule[4 * (16 + 64)];
@@ -1432,33 +1433,35 @@ void near_tiles(AssemblyArgs args, ClusterView cl, const NearChunk *chunks,
             contract<R, 16>(m, ft, fs, wscale, srule, 16, args.k, bad, fixed.d8, part, parts);
         to_parent(m, Tt, Ts);
         const bool in_b = it.swap & kNearTestInB;
-        const R inv_k = static_cast<R>(1.0 / args.k);
+        const double inv_k = 1.0 / args.k;
         int row[3], col[3];
+        double rs[3];
+        std::uint32_t node[3];
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
             row[i] = cl.local[static_cast<std::size_t>(i) * pv.nt + it.test];
             col[i] = cl.local[static_cast<std::size_t>(i) * pv.nt + it.trial];
+            node[i] = pv.nodes[static_cast<std::size_t>(i) * pv.nt + it.test];
+            rs[i] = args.row_scale[node[i]];
         }
         R *tile = in_b ? tba : tab;
 #pragma unroll
         for (int i = 0; i < 3; ++i)
 #pragma unroll
             for (int j = 0; j < 3; ++j) {
-                const R cc = static_cast<R>(gt[G_C0 + 3 * i] * gs[G_C0 + 3 * j] + gt[G_C0 + 3 * i + 1] * gs[G_C0 + 3 * j + 1] +
-                                            gt[G_C0 + 3 * i + 2] * gs[G_C0 + 3 * j + 2]) * inv_k;
+                const double cc = dot3(gt + G_C0 + 3 * i, gs + G_C0 + 3 * j) * inv_k;
+                const double re = static_cast<double>(m.a[3 * i + j].re) + static_cast<double>(m.g.im) * cc;
+                const double im = static_cast<double>(m.a[3 * i + j].im) - static_cast<double>(m.g.re) * cc;
                 R *slot = tile + col[j] * kStrideAB + 2 * row[i];
-                unsafeAtomicAdd(slot, m.a[3 * i + j].re + m.g.im * cc);
-                unsafeAtomicAdd(slot + 1, m.a[3 * i + j].im - m.g.re * cc);
+                unsafeAtomicAdd(slot, static_cast<R>(re * rs[i]));
+                unsafeAtomicAdd(slot + 1, static_cast<R>(im * rs[i]));
             }
         const std::int32_t fc = args.flux_column[it.trial];
         if (fc >= 0)
 #pragma unroll
-            for (int i = 0; i < 3; ++i) {
-                const std::uint32_t node = pv.nodes[static_cast<std::size_t>(i) * pv.nt + it.test];
-                const double rs = args.row_scale[node];
-                atomic_add_entry(args.BD + 2 * (static_cast<std::size_t>(fc) * pv.nv + node),
-                                 static_cast<double>(m.b[i].re) * rs, static_cast<double>(m.b[i].im) * rs);
-            }
+            for (int i = 0; i < 3; ++i)
+                atomic_add_entry(args.BD + 2 * (static_cast<std::size_t>(fc) * pv.nv + node[i]),
+                                 static_cast<double>(m.b[i].re) * rs[i], static_cast<double>(m.b[i].im) * rs[i]);
     }
     if (bad)
         atomicExch(args.error, ERR_DISTANCE);
@@ -1470,9 +1473,8 @@ void near_tiles(AssemblyArgs args, ClusterView cl, const NearChunk *chunks,
             const R re = tile[c * kStrideAB + 2 * r], im = tile[c * kStrideAB + 2 * r + 1];
             if (re != R(0) || im != R(0)) {
                 const std::uint32_t row = cl.nodes[r0 + r], col = cl.nodes[c0 + c];
-                const R rs = static_cast<R>(args.row_scale[row]);
-                unsafeAtomicAdd(A + 2 * (static_cast<std::size_t>(col) * pv.nv + row), re * rs);
-                unsafeAtomicAdd(A + 2 * (static_cast<std::size_t>(col) * pv.nv + row) + 1, im * rs);
+                unsafeAtomicAdd(A + 2 * (static_cast<std::size_t>(col) * pv.nv + row), re);
+                unsafeAtomicAdd(A + 2 * (static_cast<std::size_t>(col) * pv.nv + row) + 1, im);
             }
         }
     };
