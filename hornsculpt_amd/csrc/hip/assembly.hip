@@ -205,9 +205,9 @@ __device__ __forceinline__ CoreT<double> pair_core(double r2, double wq, double 
 // The regular rules of degree 4, 6 and 8 (6, 12 and 16 points), passed by value as
 // kernel arguments: with the trial loop unrolled over a compile-time count its points
 // are scalar operands, read once per wavefront instead of once per lane and sample. A
-// row holds the barycentrics, the weight, and the weight times y1^2, y1 y2, y2^2 and y0,
-// y1, y2.
-enum : int { R_Y = 0, R_W = 3, R_W11 = 4, R_W12 = 5, R_W22 = 6, R_WY = 7, R_COUNT = 10 };
+// row holds the barycentrics, the weight, and the weight times z1, z2, z1^2, z1 z2 and z2^2 with
+// z = y - 1/3, from the centroid.
+enum : int { R_Y = 0, R_W = 3, R_W1 = 4, R_W2 = 5, R_W11 = 6, R_W12 = 7, R_W22 = 8, R_COUNT = 9 };
 template <class R> struct TileRules {
     R d4[6][R_COUNT], d6[12][R_COUNT], d8[16][R_COUNT];
 };
@@ -397,11 +397,12 @@ enum : int { F_E1 = 0, F_E2 = 3, F_N = 6, F_AREA = 9, F_C0 = 10 };
 
 template <class R> struct SymSums {
     CplxT<R> g[3][3], p[3][3], q[3][3]; // [test basis i][trial basis j]
+    CplxT<R> all;                       // of g without a basis
 };
 
 template <class R> struct SymPair {
     R b[3], te1[3], te2[3], se1[3], se2[3];
-    R Q11, Q12, Q22, A1, A2, C0, T1, T2, Bn, wscale, knn;
+    R Q11, Q12, Q22, A1, A2, C, T1, T2, Bn, wscale, knn; // C: d.n_t from the test vertex 0 to the trial centroid
 };
 
 // A sample without its weight: g = exp(-ikr)/r = re - i im, and F = (1 + ikr) g / r^2, from
@@ -435,10 +436,12 @@ template <class R> __device__ __forceinline__ SymCore<R> sym_core(R r2, R k, R k
 
 // Sums of one pair over rule x rule: N > 0 takes both rules' points from the
 // kernel-argument array frule (N points, trial loop unrolled), N = 0 takes n points
-// from the FP64 table drule. Per sample only the sums of g y_a and of F times y_a, y1^2,
-// y1 y2 and y2^2 are formed, with the weights in the coefficients: d.n_s is constant over the
-// trial points and d.n_t = C0 - y1 A1 - y2 A2 is linear in them, so the sums of P and Q
-// follow once per test point. 34 operations and three transcendentals per sample (46 issue slots,
+// from the FP64 table drule. Per sample only the sums of g and F times 1, z1, z2 and of F times z1^2,
+// z1 z2 and z2^2 are formed, with the weights in the coefficients: d.n_s is constant over the
+// trial points and d.n_t = C - z1 A1 - z2 A2 is linear in them, so the sums of P and Q
+// follow once per test point, and the trial basis y_j from 1, z1, z2 once per pair. (With y in the place
+// of z, d.n_t at a vertex and its differences cancel: FP32 flux columns up to 10 % further off than
+// with d.n_t in each sample, this way 4 to 30 % closer.) 34 operations and three transcendentals per sample (46 issue slots,
 // measured 192 cycles per wavefront and sample at 4.2 per slot); forming P and Q in each sample
 // took 42. The sums on the matrix cores instead (v_mfma_f32_4x4x1, a lane's own four sums per
 // instruction) were 40 % slower: they do not overlap with the VALU here.
@@ -473,19 +476,19 @@ __device__ __forceinline__ void contract_sym(SymSums<R> &T, const SymPair<R> &c,
         const R P1 = R(-2) * (blt[0] * c.se1[0] + blt[1] * c.se1[1] + blt[2] * c.se1[2]);
         const R P2 = R(-2) * (blt[0] * c.se2[0] + blt[1] * c.se2[1] + blt[2] * c.se2[2]);
         const R B = blt[0] * blt[0] + blt[1] * blt[1] + blt[2] * blt[2];
-        // sums of g y_a (re, -im), F y_a, F y1^2, F y1 y2, F y2^2
+        // sums of g (re, -im) and F times 1, z1, z2 and of F times z1^2, z1 z2, z2^2
         R gr[3] = {0, 0, 0}, gi[3] = {0, 0, 0}, fr[3] = {0, 0, 0}, fi[3] = {0, 0, 0}, hr[3] = {0, 0, 0},
           hi[3] = {0, 0, 0};
-        auto sample_at = [&](R y1, R y2, const R *wy, R w11, R w12, R w22) {
+        auto sample_at = [&](R y1, R y2, const R *wz, R w11, R w12, R w22) {
             const R t1 = y1 * c.Q11 + (y2 * c.Q12 + P1), t2 = y2 * c.Q22 + P2;
             const R r2 = y1 * t1 + (y2 * t2 + B);
             const SymCore<R> o = sym_core(r2, k, k_rev);
 #pragma unroll
             for (int j = 0; j < 3; ++j) {
-                gr[j] += wy[j] * o.re;
-                gi[j] += wy[j] * o.im;
-                fr[j] += wy[j] * o.fr;
-                fi[j] += wy[j] * o.fi;
+                gr[j] += wz[j] * o.re;
+                gi[j] += wz[j] * o.im;
+                fr[j] += wz[j] * o.fr;
+                fi[j] += wz[j] * o.fi;
             }
             hr[0] += w11 * o.fr;
             hi[0] += w11 * o.fi;
@@ -498,22 +501,21 @@ __device__ __forceinline__ void contract_sym(SymSums<R> &T, const SymPair<R> &c,
             constexpr int kUnroll = N <= 6 ? N : 4;
 #pragma unroll kUnroll
             for (int yi = 0; yi < N; ++yi)
-                sample_at(frule[yi][R_Y + 1], frule[yi][R_Y + 2], frule[yi] + R_WY, frule[yi][R_W11],
+                sample_at(frule[yi][R_Y + 1], frule[yi][R_Y + 2], frule[yi] + R_W, frule[yi][R_W11],
                           frule[yi][R_W12], frule[yi][R_W22]);
         } else {
             for (int yi = 0; yi < n; ++yi) {
-                const double *y = drule + 4 * yi;
-                const R wy[3] = {static_cast<R>(y[3] * y[0]), static_cast<R>(y[3] * y[1]), static_cast<R>(y[3] * y[2])};
-                sample_at(static_cast<R>(y[1]), static_cast<R>(y[2]), wy, static_cast<R>(y[3] * y[1] * y[1]),
-                          static_cast<R>(y[3] * y[1] * y[2]), static_cast<R>(y[3] * y[2] * y[2]));
+                const double *y = drule + 4 * yi, z1 = y[1] - 1.0 / 3, z2 = y[2] - 1.0 / 3;
+                const R wz[3] = {static_cast<R>(y[3]), static_cast<R>(y[3] * z1), static_cast<R>(y[3] * z2)};
+                sample_at(static_cast<R>(y[1]), static_cast<R>(y[2]), wz, static_cast<R>(y[3] * z1 * z1),
+                          static_cast<R>(y[3] * z1 * z2), static_cast<R>(y[3] * z2 * z2));
             }
         }
         const R fyn = c.Bn + x1 * c.T1 + x2 * c.T2;
-        auto q_of = [&](const R *f, const R *h, R *q) { // sums of -F (C0 - y1 A1 - y2 A2) y_a
-            const R all = f[0] + f[1] + f[2];
-            q[1] = c.A1 * h[0] + (c.A2 * h[1] - c.C0 * f[1]);
-            q[2] = c.A1 * h[1] + (c.A2 * h[2] - c.C0 * f[2]);
-            q[0] = (c.A1 * f[1] + (c.A2 * f[2] - c.C0 * all)) - q[1] - q[2];
+        auto q_of = [&](const R *f, const R *h, R *q) { // sums of -F (C - z1 A1 - z2 A2) times 1, z1, z2
+            q[0] = c.A1 * f[1] + (c.A2 * f[2] - c.C * f[0]);
+            q[1] = c.A1 * h[0] + (c.A2 * h[1] - c.C * f[1]);
+            q[2] = c.A1 * h[1] + (c.A2 * h[2] - c.C * f[2]);
         };
         R qr[3], qi[3];
         q_of(fr, hr, qr);
@@ -532,6 +534,20 @@ __device__ __forceinline__ void contract_sym(SymSums<R> &T, const SymPair<R> &c,
                 T.q[i][j].im += qi[j] * xb[i];
             }
         }
+    }
+    auto to_basis = [](CplxT<R> *v) { // from 1, z1, z2 to y0, y1, y2
+        constexpr R third = R(1.0 / 3);
+        const CplxT<R> all = v[0];
+        v[0] = {all.re * third - v[1].re - v[2].re, all.im * third - v[1].im - v[2].im};
+        v[1] = {v[1].re + all.re * third, v[1].im + all.im * third};
+        v[2] = {v[2].re + all.re * third, v[2].im + all.im * third};
+    };
+    T.all = cadd_t(cadd_t(T.g[0][0], T.g[1][0]), T.g[2][0]);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        to_basis(T.g[i]);
+        to_basis(T.p[i]);
+        to_basis(T.q[i]);
     }
 }
 
@@ -801,7 +817,7 @@ void regular_tiles_sym(AssemblyArgs args, ClusterView cl, NearView near, const d
         c.Q22 = dot(c.se2, c.se2);
         c.A1 = dot(c.se1, tn);
         c.A2 = dot(c.se2, tn);
-        c.C0 = static_cast<R>(bd[0] * tn[0] + bd[1] * tn[1] + bd[2] * tn[2]);
+        c.C = static_cast<R>(bd[0] * tn[0] + bd[1] * tn[1] + bd[2] * tn[2]) - (c.A1 + c.A2) * R(1.0 / 3);
         c.T1 = dot(c.te1, sn);
         c.T2 = dot(c.te2, sn);
         c.Bn = static_cast<R>(bd[0] * sn[0] + bd[1] * sn[1] + bd[2] * sn[2]);
@@ -811,12 +827,7 @@ void regular_tiles_sym(AssemblyArgs args, ClusterView cl, NearView near, const d
     };
     // Both orientations' entries into the node tiles and, for driven panels, B_D.
     auto scatter = [&](const SymSums<R> &T, R knn, std::uint32_t lt, std::uint32_t ls) {
-        CplxT<R> G = {R(0), R(0)};
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-#pragma unroll
-            for (int j = 0; j < 3; ++j)
-                G = cadd_t(G, T.g[i][j]);
+        const CplxT<R> G = T.all;
         bad |= !isfinite(G.re) || !isfinite(G.im);
         const CplxT<R> Gk = {G.re * inv_k, G.im * inv_k};
         // Every LDS read of the scatter first, then one wait, then the node-tile updates
@@ -1675,15 +1686,15 @@ template <class R> TileRules<R> make_tile_rules() {
                                    std::to_string(rule.size()) + " points, the tile kernels expect " +
                                    std::to_string(count));
         for (std::size_t i = 0; i < count; ++i) {
-            const double w = rule[i].weight, y1 = rule[i].bary[1], y2 = rule[i].bary[2];
-            for (int c = 0; c < 3; ++c) {
+            const double w = rule[i].weight, z1 = rule[i].bary[1] - 1.0 / 3, z2 = rule[i].bary[2] - 1.0 / 3;
+            for (int c = 0; c < 3; ++c)
                 dst[i][R_Y + c] = static_cast<R>(rule[i].bary[c]);
-                dst[i][R_WY + c] = static_cast<R>(w * rule[i].bary[c]);
-            }
             dst[i][R_W] = static_cast<R>(w);
-            dst[i][R_W11] = static_cast<R>(w * y1 * y1);
-            dst[i][R_W12] = static_cast<R>(w * y1 * y2);
-            dst[i][R_W22] = static_cast<R>(w * y2 * y2);
+            dst[i][R_W1] = static_cast<R>(w * z1);
+            dst[i][R_W2] = static_cast<R>(w * z2);
+            dst[i][R_W11] = static_cast<R>(w * z1 * z1);
+            dst[i][R_W12] = static_cast<R>(w * z1 * z2);
+            dst[i][R_W22] = static_cast<R>(w * z2 * z2);
         }
     };
     fill(t.d4, 4, 6);
