@@ -482,10 +482,12 @@ std::shared_ptr<DevicePlan> MeshSolver::device_plan(const Numerics &n, double k_
     const auto t0 = Clock::now();
     auto dp = std::make_shared<DevicePlan>();
     dp->plan = plan(n, k_max, s, device);
-    { // longest rules first, so that the 4 jobs of a wavefront have the same length
+    { // one kind after the other, so that the 4 jobs of a wavefront have the same length, and the kinds with the
+      // largest entries last: coincident panels first cost an icosphere's FP32 matrix half a digit (2.8e-7
+      // against 1.1e-7 of the FP64 one at 1280 triangles, 500 Hz), since every later addition rounds there
         std::vector<TouchingJob> jobs = dp->plan.touching;
         std::stable_sort(jobs.begin(), jobs.end(), [](const TouchingJob &x, const TouchingJob &y) {
-            return x.permutation.topology > y.permutation.topology;
+            return x.permutation.topology < y.permutation.topology;
         });
         dp->touching.upload(jobs, s);
     }

@@ -7,7 +7,11 @@ sums. They are sums of some thousand terms of alternating sign: at the median th
 differ by 16 units in the last place, in FP64 and in FP32, on a mesh of any size.
 
 Flux columns of the mixed form against the FP64 ones: no further off than with the normal
-projections formed in every sample, 2.46e-8 on this sphere."""
+projections formed in every sample, 2.46e-8 on this sphere.
+
+The matrix of the mixed form against the FP64 one: its largest entries are sums of some forty
+touching pairs, the smaller terms first, so that few roundings are those of the whole sum: one
+and a quarter units of FP32 in the Frobenius norm."""
 import math
 
 import numpy as np
@@ -43,3 +47,13 @@ def test_mixed_flux_columns():
     error = np.linalg.norm(B32 - B) / np.linalg.norm(B)
     print(f"flux columns {error:.2e}")
     assert error <= 2.5e-8
+
+
+def test_mixed_matrix():
+    solver = bem.HipBemSolver(meshes.icosphere(3))
+    k = 2 * math.pi * 500.0 / 343.0
+    A, _ = solver.assemble(bem.BemNumerics(), k, k)
+    A32, _ = solver.assemble(bem.BemNumerics(precision=bem.PRECISION_MIXED), k, k)
+    error = np.linalg.norm(A32 - A) / np.linalg.norm(A)
+    print(f"matrix {error:.2e}")
+    assert error <= 1.25 * 2.0**-23
