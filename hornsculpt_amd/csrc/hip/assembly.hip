@@ -710,6 +710,7 @@ void regular_tiles_sym(AssemblyArgs args, ClusterView cl, NearView near, const d
     __shared__ std::uint8_t slocal[2][3][kTilePanels];
     __shared__ std::int32_t sfc[2][kTilePanels];
     __shared__ R srs[2][kTileNodes];
+    __shared__ std::uint32_t sid[2][kTileNodes];
 
     constexpr bool FAR = KIND != kGeneral;
     __shared__ std::uint16_t slist[FAR ? 1 : kSortedPairs<R>];
@@ -755,8 +756,10 @@ void regular_tiles_sym(AssemblyArgs args, ClusterView cl, NearView near, const d
                 slocal[c][l][p] = cl.local[static_cast<std::size_t>(l) * pv.nt + id];
             }
         }
-        if (p < static_cast<int>(c ? nB : nA))
-            srs[c][p] = static_cast<R>(args.row_scale[cl.nodes[(c ? b0 : a0) + p]]);
+        if (p < static_cast<int>(c ? nB : nA)) {
+            sid[c][p] = cl.nodes[(c ? b0 : a0) + p];
+            srs[c][p] = static_cast<R>(args.row_scale[sid[c][p]]);
+        }
     }
     __syncthreads();
 
@@ -1037,21 +1040,21 @@ void regular_tiles_sym(AssemblyArgs args, ClusterView cl, NearView near, const d
             return *slot;
     };
     // one part (re or im) per lane, so that a wavefront's atomics cover consecutive words
-    auto flush = [&](const Cell *tile, std::uint32_t r0, std::uint32_t nr, std::uint32_t c0, std::uint32_t nc, int side) {
+    auto flush = [&](const Cell *tile, std::uint32_t nr, std::uint32_t nc, int side) {
         for (std::uint32_t c = tid / 64; c < nc; c += kThreads / 64) {
-            const std::uint32_t col = cl.nodes[c0 + c];
+            const std::uint32_t col = sid[1 - side][c];
             for (std::uint32_t q = tid & 63; q < 2 * nr; q += 64) {
                 const R v = entry(tile + c * kStrideAB + q);
                 if (v != R(0)) {
-                    const std::uint32_t row = cl.nodes[r0 + q / 2];
+                    const std::uint32_t row = sid[side][q / 2];
                     unsafeAtomicAdd(A + 2 * (static_cast<std::size_t>(col) * pv.nv + row) + (q & 1), v * srs[side][q / 2]);
                 }
             }
         }
     };
-    flush(tab, a0, nA, b0, nB, 0);
+    flush(tab, nA, nB, 0);
     if (!diag)
-        flush(tba, b0, nB, a0, nA, 1);
+        flush(tba, nB, nA, 1);
 }
 
 template <class M, class R>
