@@ -1708,37 +1708,40 @@ template <class R> TileRules<R> make_tile_rules() {
 
 } // namespace
 
+// Small meshes have fewer tiles than the chip holds workgroups: the pairs of a tile are split
+// over up to 8 of them, each with its own node tiles (512-triangle sphere, 36 tiles: 0.83 ->
+// 0.25 ms FP64; 1.5k triangles, 300 tiles: 0.79 -> 0.48 ms FP32; at 4096 workgroups 0.53 ms, since
+// every part adds its entries to the matrix).
+std::uint32_t regular_tile_parts(std::uint32_t tiles) { return std::clamp(2048u / std::max(tiles, 1u), 1u, 8u); }
+
 // The tile list holds unordered cluster pairs (a <= b), far tiles first: those of degree 4 only
 // at this wavenumber, the other far ones, then the general ones.
 void launch_regular(const AssemblyLaunch &L, hipStream_t stream) {
     const std::uint32_t general = L.tile_count - L.separated_tiles;
-    // Small meshes have fewer tiles than the chip holds workgroups: the pairs of a tile are split
-    // over up to 8 of them, each with its own node tiles (512-triangle sphere, 36 tiles: 0.83 ->
-    // 0.25 ms FP64; 1.5k triangles, 300 tiles: 0.79 -> 0.49 ms FP32; at 4096 workgroups 0.53 ms, since
-    // every part adds its entries to the matrix).
-    auto parts_of = [](std::uint32_t tiles) { return std::clamp(2048u / std::max(tiles, 1u), 1u, 8u); };
     auto shift_of = [](std::uint32_t block) {
         if (block != 4 && block != 8 && block != 16)
             throw std::invalid_argument("regular tiles: the trial block must be 4, 8 or 16 panels");
         return block == 4 ? 2u : block == 8 ? 3u : 4u;
     };
-    const std::uint32_t shift = shift_of(L.trial_block), far_shift = shift_of(L.far_trial_block);
+    const std::uint32_t shift = shift_of(L.trial_block), far_shift = shift_of(L.far_trial_block),
+                        far46_shift = shift_of(L.far46_trial_block);
     auto launch = [&](auto kernel, int threads, std::uint32_t first, std::uint32_t count, const auto &fixed,
                       std::uint32_t block) {
         if (count)
-            hipLaunchKernelGGL(kernel, dim3(count, parts_of(count)), dim3(threads), 0, stream, L.args, L.clusters,
-                               L.near, L.rules, L.tiles + 2 * static_cast<std::size_t>(first), fixed, block);
+            hipLaunchKernelGGL(kernel, dim3(count, L.parts ? L.parts : regular_tile_parts(count)), dim3(threads), 0, stream,
+                               L.args, L.clusters, L.near, L.rules, L.tiles + 2 * static_cast<std::size_t>(first), fixed,
+                               block);
     };
     const std::uint32_t far46 = L.separated_tiles - L.far_tiles;
     if (L.args.A32) {
         static const TileRules<float> fixed = make_tile_rules<float>();
         launch(regular_tiles_sym<float, kFar4>, TileSum<float, kFar4>::threads, 0, L.far_tiles, fixed, far_shift);
-        launch(regular_tiles_sym<float, kFar46>, TileSum<float, kFar46>::threads, L.far_tiles, far46, fixed, far_shift);
+        launch(regular_tiles_sym<float, kFar46>, TileSum<float, kFar46>::threads, L.far_tiles, far46, fixed, far46_shift);
         launch(regular_tiles_sym<float, kGeneral>, TileSum<float, kGeneral>::threads, L.separated_tiles, general, fixed, shift);
     } else {
         static const TileRules<double> fixed = make_tile_rules<double>();
         launch(regular_tiles_sym<double, kFar4>, TileSum<double, kFar4>::threads, 0, L.far_tiles, fixed, far_shift);
-        launch(regular_tiles_sym<double, kFar46>, TileSum<double, kFar46>::threads, L.far_tiles, far46, fixed, far_shift);
+        launch(regular_tiles_sym<double, kFar46>, TileSum<double, kFar46>::threads, L.far_tiles, far46, fixed, far46_shift);
         launch(regular_tiles_sym<double, kGeneral>, TileSum<double, kGeneral>::threads, L.separated_tiles, general, fixed, shift);
     }
 }

@@ -129,10 +129,12 @@ struct AssemblyLaunch {
     const NearChunk *near_chunks;          // runs of one cluster pair and one rule
     std::uint32_t near_chunk_count;
     const PairPatch *patches;
-    // regular tiles: trial panels per wavefront block (4, 8 or 16) of the general and
-    // of the far tiles
-    std::uint32_t trial_block = 8, far_trial_block = 8;
+    // regular tiles: trial panels per wavefront block (4, 8 or 16) of the general tiles, of the
+    // far tiles of degree 4 only and of the other far ones; workgroups per tile (0: by the
+    // length of each list, regular_tile_parts)
+    std::uint32_t trial_block = 8, far_trial_block = 8, far46_trial_block = 8, parts = 0;
 };
+std::uint32_t regular_tile_parts(std::uint32_t tiles);
 
 // ---- adaptive near-pair patch estimates (estimator.hip) ----
 

@@ -707,42 +707,37 @@ dev::AssemblyLaunch MeshSolver::assembly_launch(const DevicePlan &p, const Numer
 }
 
 // Trial block of the regular tiles (4, 8 or 16 trial panels per wavefront block),
-// chosen per (mesh, precision, far or general tiles) by the autotuner on a prefix of
-// that tile list (max(512, count / 32) tiles, all when fewer): one warm and one timed
-// launch per candidate. The launches add into A, B, the error flag and the sample
-// counter, which the caller clears afterwards. HSBEM_TILE_BLOCK = 4 / 8 / 16 pins it.
+// chosen per (mesh, precision, kind of tile) by the autotuner on a prefix of that kind's
+// tiles (max(512, count / 32), all when fewer), launched with as many workgroups per tile as
+// the whole list has: one warm and one timed launch per candidate. The launches add into A, B,
+// the error flag and the sample counter, which the caller clears afterwards.
+// HSBEM_TILE_BLOCK = 4 / 8 / 16 pins it.
 void MeshSolver::tune_regular_tiles(dev::AssemblyLaunch &L, bool mixed, hipStream_t s) const {
     const auto pinned = autotune::pinned_from_env("HSBEM_TILE_BLOCK", {4, 8, 16});
     std::ostringstream key;
     key << "mesh " << std::hex << hash_ << std::dec << " (" << nt() << " panels) " << (mixed ? "fp32" : "fp64");
-    auto tune = [&](bool far) {
-        const std::uint32_t count = far ? L.separated_tiles : L.tile_count - L.separated_tiles;
-        if (!count)
+    // tiles [first, end) of the list; degree4, separated: what a launch of these tiles takes them for
+    auto tune = [&](const char *kind, std::uint32_t first, std::uint32_t end, bool degree4, bool separated) {
+        if (first == end)
             return 8u;
+        const std::uint32_t prefix = std::min(end - first, std::max(512u, (end - first) / 32));
         dev::AssemblyLaunch T = L;
-        const std::uint32_t prefix = std::min(count, std::max(512u, count / 32));
-        if (far) {
-            // the kind that most of the far tiles have
-            const bool low = 2 * L.far_tiles >= count;
-            const std::uint32_t first = low ? 0 : L.far_tiles, kind = low ? L.far_tiles : count - L.far_tiles;
-            T.tiles = L.tiles + 2 * static_cast<std::size_t>(first);
-            T.tile_count = T.separated_tiles = std::min(kind, prefix);
-            T.far_tiles = low ? T.tile_count : 0;
-        } else {
-            T.tiles = L.tiles + 2 * static_cast<std::size_t>(L.separated_tiles);
-            T.tile_count = prefix;
-            T.far_tiles = T.separated_tiles = 0;
-        }
+        T.tiles = L.tiles + 2 * static_cast<std::size_t>(first);
+        T.tile_count = prefix;
+        T.separated_tiles = separated ? prefix : 0;
+        T.far_tiles = degree4 ? prefix : 0;
+        T.parts = dev::regular_tile_parts(end - first);
         return autotune::choose(
-            "tile_trial_block", key.str() + (far ? " far" : " general"), {4, 8, 16}, 8, s,
+            "tile_trial_block", key.str() + kind, {4, 8, 16}, 8, s,
             [&](std::uint32_t w) {
-                T.trial_block = T.far_trial_block = w;
+                T.trial_block = T.far_trial_block = T.far46_trial_block = w;
                 dev::launch_regular(T, s);
             },
             1, pinned);
     };
-    L.far_trial_block = tune(true);
-    L.trial_block = tune(false);
+    L.far_trial_block = tune(" degree 4 far", 0, L.far_tiles, true, true);
+    L.far46_trial_block = tune(" degree 4 or 6 far", L.far_tiles, L.separated_tiles, false, true);
+    L.trial_block = tune(" general", L.separated_tiles, L.tile_count, false, false);
 }
 
 void MeshSolver::assemble_dense(const Numerics &n, double k_max, double k, double *A_out, double *B_out) {

@@ -96,3 +96,18 @@ def test_autotuner_reports_fastest_candidates(unpinned):
         assert r["chosen"] == min(timings, key=timings.get)
     nv = len(mesh.vertices)
     assert any(r["tunable"] == "gemv_shape" and r["key"] == f"n={nv} fp32" for r in report)
+
+
+def test_far_tile_kinds_are_tuned_by_themselves(unpinned):
+    # 400 Hz: pairs of degree 4 only; 3 kHz: most are above k h = .5
+    mesh = meshes.exponential_horn(0.0128)
+    solver = bem.HipBemSolver(mesh)
+    panels = f"({len(mesh.triangles)} panels)"
+    k_max = 2 * math.pi * 3000.0 / 343.0
+    seen = []
+    for f in (400.0, 3000.0):
+        solver.assemble(bem.BemNumerics(), k_max, 2 * math.pi * f / 343.0)
+        seen.append({r["key"].split("fp64 ")[1] for r in bem.tuning_report()
+                     if r["tunable"] == "tile_trial_block" and panels in r["key"]})
+    assert "degree 4 far" in seen[0] and "degree 4 or 6 far" not in seen[0]
+    assert "degree 4 or 6 far" in seen[1]
