@@ -297,6 +297,7 @@ def run_sweep(variant_count, frequency_count, slots, tolerance):
 
 STREAM_SEED = 20261203   # arrivals and request draws (mt19937_64)
 POOL_SEED = 20261204     # horn shapes of the resident mesh pool
+TIMED_SECONDS = 90.0  # of the served stream's timed windows together, per form
 DIRECTIVITY_DEG = (0.0, 15.0, 30.0, 45.0, 60.0, 90.0)
 
 
@@ -640,6 +641,8 @@ def main_stream(args):
     """The headline: the served stream, plain FP64 then mixed, on the same arrivals."""
     steps = 3 if args.steps is None else args.steps
     warmup = 1 if args.warmup is None else args.warmup
+    if args.window is None:
+        args.window = min(30.0, TIMED_SECONDS / steps)
     t0 = time.perf_counter()
     pool = StreamPool(args.pool, args.pool_min, args.pool_max)
     sizes = [e["triangles"] for e in pool.entries]
@@ -786,7 +789,9 @@ def main():
     ap.add_argument("--horn", action="store_true",
                     help="only the dense horn sweep (20.7k triangles, 16 frequencies; one JSON line)")
     ap.add_argument("--rate", type=float, default=20.0, help="served stream: Poisson arrivals per second")
-    ap.add_argument("--window", type=float, default=30.0, help="served stream: seconds per step (window)")
+    ap.add_argument("--window", type=float, default=None,
+                    help="served stream: seconds per step (window; default 30, less where the steps would take more "
+                         f"than {TIMED_SECONDS:.0f} s together)")
     ap.add_argument("--pool", type=int, default=8, help="served stream: resident horn meshes")
     ap.add_argument("--pool-min", type=float, default=2000.0)
     ap.add_argument("--pool-max", type=float, default=120000.0)
