@@ -59,3 +59,33 @@ def test_concurrent_factorizations():
     for i, x in enumerate(out):
         # the same system up to the order of the sums: a random matrix of this order has a condition below 1e6
         assert np.linalg.norm(x - out[0] * (i + 1)) <= 1e-9 * np.linalg.norm(x)
+
+
+# one workgroup takes panels of more than 128 rows a limit's workgroup: 4 columns at a time, pairs of 32
+# columns, until few enough rows are left (the hand-over to 64-column panels at k0 > 0), and the
+# interchanges of the right-hand sides go through memory
+@pytest.mark.parametrize("n,nrhs,groups", [(129, 1, 1), (193, 2, 1), (257, 3, 1), (257, 1, 2), (321, 9, 1), (449, 2, 2),
+                                           (513, 1, 1), (513, 4, 2), (1091, 5, 3), (2113, 1, 7)])
+@pytest.mark.parametrize("pivoted", [True, False])
+def test_panels_beyond_the_limit(n, nrhs, groups, pivoted):
+    A, B = _system(n, nrhs)
+    if not pivoted:
+        A += 4 * n * np.eye(n)
+    X = bem.dense_lu_solve(A, B, limits=bem.LuLimits(panel_groups=groups, permute_rows=1))
+    _check(A, X, B)
+    _check(A, bem.dense_lu_solve(A, B, limits=bem.LuLimits(panel_groups=groups)), B)
+
+
+@pytest.mark.parametrize("groups", [0, 1, 2])
+@pytest.mark.parametrize("column", [0, 3, 130, 300])
+def test_zero_pivot_beyond_the_limit(groups, column):
+    A, B = _system(301, 1)
+    A[:, column] = 0
+    with pytest.raises(RuntimeError, match=f"pivot {column + 1}$"):
+        bem.dense_lu_solve(A, B, limits=bem.LuLimits(panel_groups=groups))
+
+
+def test_many_panel_workgroups():
+    # 73 workgroups of one panel, an odd tail
+    A, B = _system(9217, 1)
+    _check(A, bem.dense_lu_solve(A, B), B)
