@@ -21,7 +21,8 @@
 //                   patch points over lanes.
 //   mass            1/2 M_pp into A, -alpha 1/2 M_pq into the flux columns.
 // Precision: the sample type R is double (plain form) or float (mixed form:
-// FP32 samples and accumulation, FP64 geometry differences, FP32 matrix).
+// FP32 samples and accumulation, FP64 geometry differences, FP32 matrix; entries of near
+// patches formed in FP64, node tiles in FP32 or in fixed point, see TileSum).
 #include "../host/plan.hpp"
 #include "../host/qualification.hpp"
 #include "../host/rules.hpp"
@@ -377,9 +378,9 @@ template <> __device__ __forceinline__ float *matrix_of<float>(const AssemblyArg
 // (t in A, s in B) is integrated once on its rule x rule samples and both ordered
 // pairs (t, s) and (s, t) are formed from them: distance, phase, g and the radial
 // factor are shared, only the normal projections differ. With d = x - y (x on t, y
-// on s), P = radial (d.n_s)/r^2 and Q = -radial (d.n_t)/(k r^2):
-//   (t, s):  a = -P + i knn g,     b = -g + i Q
-//   (s, t):  a = -k Q + i knn g,   b = -g + i P / k
+// on s), F = (1 + i k r) g / r^2, P = F (d.n_s) and Q = -F (d.n_t):
+//   (t, s):  a = -P + i knn g,   b = -g + i Q / k
+//   (s, t):  a = -Q + i knn g,   b = -g + i P / k
 // (for (s, t) the displacement is -d, its trial normal n_t and its test normal n_s).
 // The sums TG, TP, TQ of g, P, Q weighted by the test basis x_i and the trial basis
 // y_j (3 x 3 complex each) give all 2 x 9 A moments and 2 x 3 B moments. The (t, s)
@@ -629,9 +630,10 @@ enum TileKind : int { kGeneral = 0, kFar4 = 1, kFar46 = 2 };
 // The bound is that of the tile's closest and largest pairs and a typical entry lies about 2^11
 // below it, so kFar46 tiles take 64 bits in both forms, 2^-54 and 2^-62: entries as exact as
 // sums in FP32 and FP64 (at the median FP32 2^-30 gave 3.4e-6 instead of 4.4e-7, FP64 2^-51
-// 1.5e-12 instead of 1e-15). A mixed solve of 20.7k triangles at 8 kHz takes 61.9 ms this way, 64.2 ms
-// with FP32 sums by LDS atomics, and 55.5 ms with the 32 bits that are not enough, in cells that
-// leave room for two workgroups on a compute unit; in the FP64 form the three are the same.
+// 1.5e-12 instead of 1e-15). In the FP64 form that costs nothing. In the FP32 form the cells leave
+// room for one workgroup on a compute unit: tiles of a 20.7k-triangle horn at 8 kHz take 36.3 ms, where
+// the 32 bits that are not enough take 29.4 ms (35.1 ms with one workgroup as well); FP32 sums by
+// LDS atomics are slower still (a whole solve 64.2 against 61.9 ms).
 template <class R, TileKind KIND> struct TileSum {
     static constexpr bool fixed = KIND != kGeneral, fp32 = sizeof(R) == 4;
     using Cell = std::conditional_t<!fixed, R, std::conditional_t<fp32 && KIND == kFar4, int, long long>>;
@@ -686,10 +688,10 @@ __device__ __forceinline__ bool far_scale(const double *fa, const double *fb, do
     return true;
 }
 
-// Far tiles as kinds of their own (20.7k-triangle horn at 8 kHz, all far tiles as kGeneral ones before: 49.2 -> 37.9 ms FP32,
-// 103 -> 96.6 ms FP64; at 4 kHz 51.2 -> 41.3 and 113 -> 102.7 ms; at 1 kHz 20.2 -> 19.5 and 48.5 ->
-// 41.2 ms). Occupancy: FP32, two 512-thread workgroups per CU
-// (LDS <= 80 KiB, VGPRs <= 128); FP64, one (LDS <= 160 KiB, VGPRs <= 256).
+// All tiles of a 20.7k-triangle horn, against far tiles of degree 4 only and general ones unsorted:
+// at 8 kHz 49.4 -> 43.5 ms FP32 and 104 -> 95.9 ms FP64, at 4 kHz 51.5 -> 47.6 and 107 -> 101 ms, at
+// 1 kHz 21.0 -> 19.7 and 42.8 -> 36.5 ms. Occupancy: FP32, two 512-thread workgroups per CU
+// (LDS <= 80 KiB, VGPRs <= 128) or one of 1024 (kFar46); FP64, one of 512 (LDS <= 160 KiB, VGPRs <= 256).
 
 // Pairs that a general tile sorts at a time: what the LDS has left.
 template <class R> constexpr int kSortedPairs = sizeof(R) == 4 ? 2048 : 4096;

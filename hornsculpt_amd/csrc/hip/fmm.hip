@@ -10,9 +10,9 @@
 //                    (-R_lm - alpha n . grad R_lm) phi_i / m_i of the leaf's P1 DOFs;
 //   * emission       multipole of a leaf = E_leaf p (one block per leaf);
 //   * translation    every M2M / M2L / L2L link is rotate-to-axis, coaxial m-block
-//                    translation, rotate-back (O(p^3)): the rotations run per chunk
-//                    of links sharing a direction with the Wigner blocks staged in
-//                    LDS, the coaxial products per link, and one block per
+//                    translation, rotate-back (O(p^3)): three passes per chunk of up to
+//                    16 links that share a direction and a coaxial plan, as products on
+//                    the matrix cores with operands straight from memory, and one block per
 //                    destination sums its links (no atomics);
 //   * testing        y_i += T_leaf L_leaf (one wavefront per DOF).
 #include "fmm_kernels.hpp"

@@ -192,7 +192,8 @@ __device__ __forceinline__ double2 minus_product(double2 b, double2 l, double2 q
 // Bound by latency, not by work: about 3 us per column with an exchange (two dependent reads
 // through the memory that every XCD sees) and 1.3 us without; leaves of 4 columns on one
 // workgroup took 9 us (n = 4099 in all: 20.1 against 52.6 ms, n = 10373: 110 against 252 ms,
-// where the trailing updates run at 72 TFLOP/s and cover all but the last panels).
+// where the launches that factor a panel beside the update of the one before take 92.6 ms for
+// 2.98 TFLOP, 32 TFLOP/s).
 // Ring slots are emptied by their owner one column after use: by then every group has
 // published its next candidate, which it does after reading this one, and a slot is
 // written again three columns later.

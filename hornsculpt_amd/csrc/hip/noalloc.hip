@@ -2,8 +2,8 @@
 //
 // The factorization needs device memory beyond the caller's matrix and
 // right-hand sides: the pivot rows (n int32), the singular-pivot status
-// word and the exchange words of the panel's workgroups. Here they live in one file-scope device array (`scratch`) instead of
-// hipMalloc'd buffers, so the entry point can serve callers that may not
+// word and the exchange words of the panel's workgroups. Here they live in one file-scope device
+// array (`scratch`) instead of hipMalloc'd buffers, so the entry point can serve callers that may not
 // allocate (code under stream capture, tight serving loops, harnesses that
 // forbid hipMalloc). Every GPU the library runs on holds its own copy of the
 // array until the process ends; its device address is resolved once per

@@ -842,8 +842,9 @@ namespace {
 // into a HIP graph and replayed once per iteration; the host reads the cycle state
 // every kPoll steps, one poll behind the queue, so it never waits for a step to
 // finish before queuing the next, and solves the small triangular system once per
-// cycle. Same arithmetic as gmres(): the same reductions in the same order and the
-// same rotation formulas (evaluated on the device).
+// cycle. Equal to gmres() up to rounding: the same steps and rotation formulas (evaluated on
+// the device), but the product's column chunks are summed by the first orthogonalization pass,
+// in another order than by the product's own reduction when there are more than eight.
 constexpr std::uint32_t kPoll = 4;
 
 void dense_gmres_graph(hipStream_t s, const void *A, bool fp32, std::uint32_t n, const double *b, double *x,
